@@ -58,14 +58,15 @@ struct Counters {
   unsigned long long children, child_nodes, child_consts, parent_nodes, parent_consts, child_code_words, child_pool_words;
 };
 
+// Totals of one work item of the looping kernel (a program on one tile
+// group), combined per program by k_loop_finish.
+struct alignas(16) LoopPart {
+  long long sum;            // of the integral scores
+  unsigned long long fuel;  // charged fuel
+  unsigned wrong, errors, timeouts, fractional;
+};
 // Device state of one search. Every pointer is device memory owned by the
 // host Search object.
-// Totals of one program's tiles in the looping kernel (device atomics).
-struct LoopAcc {
-  unsigned long long sum;   // two's-complement int64 sum of the integral scores
-  unsigned long long fuel;  // charged fuel
-  unsigned wrong, errors, timeouts, fractional, tiles, pad;
-};
 
 struct DSearch {
   int active;
@@ -103,7 +104,7 @@ struct DSearch {
   GAS int *code_len, *pool_len, *code_jumps;
   GAS std::uint64_t* child_hash;
   // pending[2B]: children to score, general ones from the front of [0, B),
-  // vm_fast ones from its back, vm_loop ones in [B, 2B); n_pending[3] counts each.
+  // vm_fast ones from its back, vm_steps ones in [B, 2B); n_pending[3] counts each.
   GAS int *pending, *n_pending;
   GAS std::uint64_t* table_key;  // genotype hash | 1, 0 = empty
   GAS int* table;                // a member with that hash
@@ -137,7 +138,10 @@ struct DSearch {
   GAS const double* select;
   int general_scores;  // the general evaluation kernel has an LDS score buffer for this search
   GAS double* loop_scores;  // the looping kernel's case scores: C per program slot
-  GAS LoopAcc* loop_acc;    // the looping kernel's per-program tile totals (zero between evaluations)
+  GAS LoopPart* loop_part;  // the looping kernel's totals: one per 64-case tile and program slot
+  GAS Step* steps;          // decoded steps of the programs of the looping path, step_cap per slot
+  GAS int* step_n;
+  int step_cap;
   int stage_cases;     // the typed evaluation kernel stages the case set in LDS
   int typed_tiles;     // typed programs go to k_eval_tiles (more than one 64-case tile, C <= kScoreCases)
 };
@@ -199,17 +203,23 @@ __global__ __launch_bounds__(64 * kVaryWaves) void k_init_pop(DSearch* all, cons
 // kWalks: the lowering instantiation with traversals (grammars that have them).
 // Returns the code flags it stores (code_jumps).
 template <bool kWalks>
-__device__ inline int lower_into_w(const PhaseView& g, const DSearch& d, const CRow& row, int slot, WalkStore<kWalks>& ws) {
+__device__ __attribute__((always_inline)) inline int lower_into_w(const PhaseView& g, const DSearch& d, const CRow& row, int slot, WalkStore<kWalks>& ws) {
   Ins* code = d.code + std::size_t(slot) * d.code_cap;
   Val* pool = d.pool + std::size_t(slot) * d.pool_cap;
   const LowerResult r =
       lower_phase_w<kWalks>(g, row, d.local_types, d.n_locals, d.expected_type, code, d.code_cap, pool, d.pool_cap, ws);
   const bool ok = r.status == ST_OK && r.stack_bound >= 1 && r.stack_bound <= d.stack_slots &&
                   r.locals - d.n_locals <= d.temp_slots - d.input_shadow;
-  // bit 0: jumps; bit 1: typed straight-line (vm_fast); bit 2: Bool result; bit 3: typed looping (vm_loop)
+  // bit 0: jumps; bit 1: typed straight-line (vm_fast); bit 2: Bool result; bit 3: typed looping (vm_steps)
   const int flags = r.jumps | (r.fast ? 2 : 0) | (r.result_type == TAG_BOOL ? 4 : 0) | (r.loop ? 8 : 0);
+  int steps = 0;
+  if (ok && r.loop && d.steps) {
+    wave_fence();  // the code and pool stored above are read across the lanes
+    steps = decode_steps_w(code, r.code, pool, d.n_locals, d.steps + std::size_t(slot) * d.step_cap);
+  }
   if (wlane() == 0) {
     if (!ok) raise(d, 200 + r.status);
+    if (d.steps) d.step_n[slot] = steps;
     d.code_len[slot] = ok ? r.code : 0;
     d.pool_len[slot] = ok ? r.constants : 0;
     d.code_jumps[slot] = flags;
@@ -617,50 +627,53 @@ __device__ inline double canonical_from_scores(const EvalParams& e, int C, const
 }
 
 // Items of the looping kernel: (program, group of `group` consecutive
-// 64-case tiles) pairs, one wavefront each; blocks for n programs (at most
-// 8192, which loop over the rest).
+// 64-case tiles) pairs, one wavefront each; blocks of one wavefront for n
+// programs (at most kLoopBlocks, which loop over the rest).
+constexpr int kLoopBlocks = 16384;
 __host__ __device__ inline int loop_blocks(int C, int n, int group = 1) {
   const int tiles = (C + 63) / 64, groups = (tiles + group - 1) / group;
-  const long long waves = (long long)n * groups;
-  return int(std::min<long long>(8192, (waves + kWavesPerBlock - 1) / kWavesPerBlock));
+  return int(std::min<long long>(kLoopBlocks, (long long)n * groups));
 }
 
-// The looping path as a tile queue: every wavefront takes (program, tile
-// group) items of its own, program-major, so no wavefront waits for another.
+// The looping path as a tile queue: every block is one wavefront and takes
+// (program, tile group) items of its own, so no wavefront waits for another.
 // A group is `group` consecutive 64-case tiles of one program, run one after
-// another by the wavefront (the program's decoded code stays in registers).
+// another by the wavefront. Items go tile group first: the cases are visited
+// by descending list length, so the longest items of all programs start
+// first and the launch ends with the shortest.
 // Scores go to the program's row of loop_scores (HBM). A program with one
-// group is finished by its wavefront; otherwise each group adds its counts
-// and its exact integer score sum to the program's LoopAcc with device
-// atomics, and the wavefront that completes the last group forms the
-// fitness: the sum, or the canonical replay from the scores when some tile
-// had a non-integral score. It then clears the record for the program's next
-// evaluation. LDS: per wavefront kLoopSlots slots of 64 lanes, independent of
-// the case count.
+// group is finished by its wavefront; otherwise every group writes its totals
+// to its own LoopPart and k_loop_finish, the next launch, combines them: no
+// fence or atomic orders the items of one program. LDS: step_slots(n_inputs)
+// slots of 64 lanes, independent of the case count.
 // kGrouped false is the one-tile instantiation (group 1): its loop-carried
-// totals fold away, which keeps five wavefronts per SIMD.
+// totals fold away.
+// Bound by instruction issue of the step loop (scalar decode and branches).
+// Four-wavefront blocks of one program held their slots until the longest of
+// its tiles ended, and every item paid two device-wide fences and thirteen
+// atomics. Measured together with the decoded steps, per launch: population
+// 8192 x 200 list cases 3.18 -> 0.65 ms, 64 mixed searches 5.59 -> 1.52 ms,
+// population 1500 x 130 cases of statement programs 0.85 -> 0.32 ms.
 template <bool kGrouped>
-__global__ __launch_bounds__(kEvalThreads) void k_eval_loop(DSearch* all, const BlockMap* map, int mode, int group_arg) {
+__global__ __launch_bounds__(64) void k_eval_loop(DSearch* all, const BlockMap* map, int mode, int group_arg) {
   const int group = kGrouped ? group_arg : 1;
   const BlockMap bm = map[blockIdx.x];
   const DSearch& d = all[bm.search];
   if (mode == 1 ? !search_live(d) : (!d.active || *d.error)) return;
-  extern __shared__ unsigned char smem[];
-  const int wave = wave_index(), lane = threadIdx.x % 64;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int lane = threadIdx.x;
   const int C = d.cd.C, tiles = (C + 63) / 64, groups = (tiles + group - 1) / group;
-  LAS std::int64_t* const slots = (LAS std::int64_t*)smem + std::size_t(wave) * kLoopSlots * 64;
+  LAS std::int64_t* const slots = (LAS std::int64_t*)smem;
   const EvalParams e{d.cd, d.fuel, d.lanes, d.penalty, d.policy};
   const int count = mode == 1 ? d.n_pending[2] : d.P;
   const long long items = (long long)count * groups;
-  for (long long k = (long long)bm.block * kWavesPerBlock + wave; k < items; k += (long long)bm.blocks * kWavesPerBlock) {
-    const int i = int(k / groups), first = int(k % groups) * group, last = min(tiles, first + group);
+  for (long long k = bm.block; k < items; k += bm.blocks) {
+    const int q0 = int(k / count), i = int(k % count), first = q0 * group, last = min(tiles, first + group);
     const int slot = mode == 1 ? d.pending[pending_at(d.B, 2, i)] : i;
     const int pmode = d.code_jumps[slot];
     if (mode == 0 && eval_class(pmode, C) != 2) continue;  // another kernel scores it (uniform per wavefront)
-    const ProgView pv{d.code + std::size_t(slot) * d.code_cap, d.pool + std::size_t(slot) * d.pool_cap, d.code_len[slot],
-                      d.n_locals, pmode & 1, (pmode >> 1) & 1, d.pool_len[slot], (pmode & 4) ? TAG_BOOL : TAG_INT};
-    const LoopProgram lp = loop_load(pv, lane);
-    const int n_in = staged_inputs_of(pv.n_locals, e.cd.n_inputs);
+    const int n_in = staged_inputs_of(d.n_locals, e.cd.n_inputs), result_tag = (pmode & 4) ? TAG_BOOL : TAG_INT;
+    const StepProgram sp = steps_load(d.steps + std::size_t(slot) * d.step_cap, d.step_n[slot], lane);
     GAS double* const scores = d.loop_scores + std::size_t(slot) * C;
     long long total = 0;  // exact while no score is fractional
     bool frac = false;
@@ -673,8 +686,9 @@ __global__ __launch_bounds__(kEvalThreads) void k_eval_loop(DSearch* all, const 
       const int at = (first + q) * 64 + lane;
       const bool active = at < C;
       const int c = active ? e.cd.order[at] : 0;
-      const LaneResult r = vm_loop(lp, fast_inputs(e.cd, pv.n_locals, c, active), n_in, e.cd.arena, slots, lane, active, e.fuel,
-                                   pv.result_tag);
+      const FastInputs in = fast_inputs(e.cd, d.n_locals, c, active);
+      const LaneResult r = sp.n <= 64 ? vm_steps<1>(sp, in, n_in, e.cd.arena, slots, lane, active, e.fuel, result_tag)
+                                      : vm_steps<4>(sp, in, n_in, e.cd.arena, slots, lane, active, e.fuel, result_tag);
       double sc = 0;
       bool exact = true;
       if (active) {
@@ -687,48 +701,17 @@ __global__ __launch_bounds__(kEvalThreads) void k_eval_loop(DSearch* all, const 
       const double ws = wave_sum_d(sc);
       frac = frac || fractional;
       if (!frac) total += (long long)ws;
-      tw += wave_sum_u(active && !exact);
-      te += wave_sum_u(active && r.err != ERR_NONE);
-      tt += wave_sum_u(active && r.err == ERR_TIMEOUT);
-      unsigned long long f = active ? unsigned(r.fuel_used) : 0u;
-      for (int off = 32; off > 0; off >>= 1) f += __shfl_xor(f, off, 64);
-      tf += f;
+      tw += unsigned(__popcll(__ballot(active && !exact)));
+      te += unsigned(__popcll(__ballot(active && r.err != ERR_NONE)));
+      tt += unsigned(__popcll(__ballot(active && r.err == ERR_TIMEOUT)));
+      tf += wave_sum_u64(active ? unsigned(r.fuel_used) : 0u);
     }
-    if (frac) total = 0;
     if (groups > 1) {
-      GAS LoopAcc* const acc = d.loop_acc + slot;
-      __threadfence();  // this group's scores before its arrival
-      unsigned prev = 0;
-      if (lane == 0) {
-        atomicAdd(&acc->sum, (unsigned long long)total);
-        atomicAdd(&acc->fuel, tf);
-        atomicAdd(&acc->wrong, tw);
-        atomicAdd(&acc->errors, te);
-        atomicAdd(&acc->timeouts, tt);
-        if (frac) atomicOr(&acc->fractional, 1u);
-        __threadfence();
-        prev = atomicAdd(&acc->tiles, 1u);
-      }
-      if (__shfl(prev, 0, 64) != unsigned(groups - 1)) continue;  // another group finishes the program
-      __threadfence();  // every group's scores and counts after the last arrival
-      unsigned long long v[2] = {0, 0};
-      unsigned u[4] = {0, 0, 0, 0};
-      if (lane == 0) {
-        v[0] = atomicAdd(&acc->sum, 0ull); v[1] = atomicAdd(&acc->fuel, 0ull);
-        u[0] = atomicAdd(&acc->wrong, 0u); u[1] = atomicAdd(&acc->errors, 0u);
-        u[2] = atomicAdd(&acc->timeouts, 0u); u[3] = atomicAdd(&acc->fractional, 0u);
-        // cleared for the program's next evaluation
-        atomicExch(&acc->sum, 0ull); atomicExch(&acc->fuel, 0ull); atomicExch(&acc->wrong, 0u);
-        atomicExch(&acc->errors, 0u); atomicExch(&acc->timeouts, 0u); atomicExch(&acc->fractional, 0u);
-        atomicExch(&acc->tiles, 0u);
-      }
-      total = (long long)__shfl(v[0], 0, 64);
-      tf = __shfl(v[1], 0, 64);
-      tw = __shfl(u[0], 0, 64); te = __shfl(u[1], 0, 64); tt = __shfl(u[2], 0, 64);
-      frac = __shfl(u[3], 0, 64) != 0;
-    } else {
-      wave_fence();  // the canonical replay reads the other lanes' scores
+      if (lane == 0)
+        d.loop_part[std::size_t(slot) * tiles + q0] = LoopPart{frac ? 0 : total, tf, tw, te, tt, unsigned(frac)};
+      continue;
     }
+    wave_fence();  // the canonical replay reads the other lanes' scores
     const double fitness = frac ? canonical_from_scores(e, C, scores, lane) : double(total);
     if (lane == 0) {
       // Ranking rounds every published fitness to a 40-bit mantissa.
@@ -737,6 +720,51 @@ __global__ __launch_bounds__(kEvalThreads) void k_eval_loop(DSearch* all, const 
       d.e_errors[slot] = te;
       d.e_timeouts[slot] = tt;
       d.e_fuel[slot] = tf;
+    }
+  }
+}
+
+// Combines the LoopParts of every program of more than one tile group: 16
+// lanes per program and four programs per wavefront, the canonical replay
+// over the program's scores by the whole wavefront where some tile had a
+// non-integral one.
+constexpr int kFinishPrograms = 4 * kWavesPerBlock;  // programs per block
+__global__ __launch_bounds__(kEvalThreads) void k_loop_finish(DSearch* all, const BlockMap* map, int mode, int group) {
+  const BlockMap bm = map[blockIdx.x];
+  const DSearch& d = all[bm.search];
+  if (mode == 1 ? !search_live(d) : (!d.active || *d.error)) return;
+  const int C = d.cd.C, tiles = (C + 63) / 64, groups = (tiles + group - 1) / group;
+  if (groups <= 1 || C > kScoreCases) return;
+  const int lane = threadIdx.x % 64, part = lane % 16;
+  const EvalParams e{d.cd, d.fuel, d.lanes, d.penalty, d.policy};
+  const int count = mode == 1 ? d.n_pending[2] : d.P;
+  for (int base = bm.block * kFinishPrograms + 4 * wave_index(); base < count; base += bm.blocks * kFinishPrograms) {
+    const int i = base + lane / 16;
+    const int slot = i >= count ? -1 : mode == 1 ? d.pending[pending_at(d.B, 2, i)] : i;
+    const bool mine = slot >= 0 && (mode == 1 || eval_class(d.code_jumps[slot], C) == 2);
+    LoopPart t{0, 0, 0, 0, 0, 0};
+    for (int q = part; mine && q < groups; q += 16) {
+      const LoopPart x = d.loop_part[std::size_t(slot) * tiles + q];
+      t.sum += x.sum; t.fuel += x.fuel;
+      t.wrong += x.wrong; t.errors += x.errors; t.timeouts += x.timeouts; t.fractional |= x.fractional;
+    }
+    for (int off = 8; off > 0; off >>= 1) {
+      t.sum += __shfl_xor(t.sum, off, 64); t.fuel += __shfl_xor(t.fuel, off, 64);
+      t.wrong += __shfl_xor(t.wrong, off, 64); t.errors += __shfl_xor(t.errors, off, 64);
+      t.timeouts += __shfl_xor(t.timeouts, off, 64); t.fractional |= __shfl_xor(t.fractional, off, 64);
+    }
+    double fitness = double(t.sum);
+    for (unsigned long long m = __ballot(mine && part == 0 && t.fractional); m; m &= m - 1) {
+      const int from = wave_first(m);
+      const double total = canonical_from_scores(e, C, d.loop_scores + std::size_t(rdlane(slot, from)) * C, lane);
+      if (lane == from) fitness = total;
+    }
+    if (mine && part == 0) {
+      if (mode == 1) { d.c_fit[slot] = canon40(fitness); d.c_wrong[slot] = t.wrong; }
+      else { d.fitness[slot] = canon40(fitness); d.wrong[slot] = t.wrong; }
+      d.e_errors[slot] = t.errors;
+      d.e_timeouts[slot] = t.timeouts;
+      d.e_fuel[slot] = t.fuel;
     }
   }
 }
@@ -1781,9 +1809,13 @@ struct SearchState {
     DeviceCases dc;
     dc.upload(a, train);
     x.cd = dc.cd;
-    if (x.cd.C <= kScoreCases) {
-      x.loop_scores = a.alloc<double>(std::size_t(std::max(P, B)) * std::size_t(x.cd.C));
-      x.loop_acc = a.upload(std::vector<LoopAcc>(std::size_t(std::max(P, B))));
+    const std::size_t slots = std::size_t(std::max(P, B));
+    if (x.cd.C <= kScoreCases) x.loop_scores = a.alloc<double>(slots * std::size_t(x.cd.C));
+    if (x.cd.C <= kScoreCases && may_jump) {
+      x.loop_part = a.alloc<LoopPart>(slots * std::size_t((x.cd.C + 63) / 64));
+      x.step_cap = std::min(x.code_cap, kStepMax);
+      x.steps = a.alloc<Step>(slots * std::size_t(x.step_cap));
+      x.step_n = a.alloc<int>(slots);
     }
     const std::size_t rows = std::size_t(P) * R, crows = std::size_t(B) * R;
     x.cur_origin = a.alloc<int>(rows); x.cur_site = a.alloc<int>(rows); x.cur_cval = a.alloc<Val>(rows);
@@ -1939,8 +1971,7 @@ struct Batch::Impl {
     }
   }
   std::size_t eval_fast_lds = 0, eval_general_lds = 0, eval_tiles_lds = 0;  // dynamic LDS of the evaluation kernels
-  static constexpr std::size_t kLoopLds = std::size_t(kWavesPerBlock) * kLoopSlots * 64 * 8;  // the looping slots
-  std::size_t eval_loop_lds = 0;
+  std::size_t eval_loop_lds = 0;  // the looping path's slots
   std::size_t vary_lds_bytes = 0;  // phase-table copy of the staged reproduction kernel
   bool vary_global = false;        // some search reproduces from global tables
   bool any_generational = false;
@@ -1949,7 +1980,7 @@ struct Batch::Impl {
   struct Grid { GAS BlockMap* map = nullptr; int blocks = 0; };
   DeviceArena map_arena;
   Grid g_init, g_lower, g_eval_init, g_vary_staged, g_vary_global, g_vary_staged_w, g_vary_global_w, g_table, g_member,
-      g_eval, g_eval_tiles, g_eval_general, g_eval_loop, g_member_w;
+      g_eval, g_eval_tiles, g_eval_general, g_eval_loop, g_finish, g_member_w;
   // Evaluation launch shapes of the round (the autotuner's choice, or the
   // fixed default: one program per wavefront, one 64-case tile per item).
   TuneChoice tune;
@@ -2002,6 +2033,7 @@ struct Batch::Impl {
     g_eval_tiles = tiles_grid(map_arena, live, false);
     g_eval_general = eval_grid(map_arena, 1);
     g_eval_loop = loop_grid(map_arena, tune.loop_group);
+    g_finish = finish_grid(map_arena, live, false);
   }
   // Evaluation grids of the live searches: `per_wave` pending programs per
   // wavefront of the typed and general kernels; `group` tiles per work item
@@ -2019,8 +2051,13 @@ struct Batch::Impl {
   Grid tiles_grid(DeviceArena& arena, const std::vector<int>& table, bool members) {
     return build_grid(arena, table, [&](const SearchState& s) { return s.d.typed_tiles ? std::min(4096, members ? s.P : s.B) : 0; });
   }
+  Grid finish_grid(DeviceArena& arena, const std::vector<int>& table, bool members) {
+    return build_grid(arena, table, [&](const SearchState& s) {
+      return s.may_jump && s.d.cd.C > 64 && s.d.cd.C <= kScoreCases ? up(members ? s.P : s.B, kFinishPrograms) : 0;
+    });
+  }
   Grid loop_grid(DeviceArena& arena, int group) {
-    return build_grid(arena, live, [&](const SearchState& s) { return s.may_jump ? loop_blocks(s.d.cd.C, s.B, group) : 0; });
+    return build_grid(arena, live, [&](const SearchState& s) { return s.may_jump && s.d.steps ? loop_blocks(s.d.cd.C, s.B, group) : 0; });
   }
 
   // Allocates one search and fixes its kernel variants and LDS needs.
@@ -2040,7 +2077,7 @@ struct Batch::Impl {
   // LDS sizes and kernel attributes for a table of searches.
   void size_kernels(const std::vector<int>& table) {
     eval_fast_lds = eval_general_lds = eval_tiles_lds = vary_lds_bytes = place_lds_bytes = place_hbm_bytes = 0;
-    eval_loop_lds = kLoopLds;
+    eval_loop_lds = 0;
     vary_global = any_generational = false;
     max_P = max_B = max_slots = max_table = 0;
     for (int id : table) {
@@ -2051,7 +2088,7 @@ struct Batch::Impl {
       const std::size_t cases = x.d.stage_cases ? staged_case_bytes(x.d.cd.C, staged_inputs_of(x.d.n_locals, x.d.cd.n_inputs)) : 0;
       if (x.d.cd.C <= kScoreCases) {
         eval_fast_lds = std::max(eval_fast_lds, score_buf + cases);
-        eval_loop_lds = kLoopLds;
+        eval_loop_lds = std::max(eval_loop_lds, std::size_t(step_slots(staged_inputs_of(x.d.n_locals, x.d.cd.n_inputs))) * 64 * 8);
       }
       if (x.d.typed_tiles) eval_tiles_lds = std::max(eval_tiles_lds, std::size_t(8) * x.d.cd.C);
       if (x.d.stage_tables) vary_lds_bytes = std::max(vary_lds_bytes, phase_tables_bytes(x.d.g));
@@ -2140,8 +2177,10 @@ struct Batch::Impl {
       });
     if (any_jumps(ids))
       timer.time("k_eval_init_loop", stream, [&] {
-        const Grid gp = build_grid(tmp, ids, [&](const SearchState& x) { return loop_blocks(x.d.cd.C, x.P); });
-        hipLaunchKernelGGL(k_eval_loop<false>, dim3(gp.blocks), dim3(kEvalThreads), eval_loop_lds, stream, t, gp.map, 0, 1);
+        const Grid gp = build_grid(tmp, ids, [&](const SearchState& x) { return x.may_jump && x.d.steps ? loop_blocks(x.d.cd.C, x.P) : 0; });
+        if (gp.blocks) hipLaunchKernelGGL(k_eval_loop<false>, dim3(gp.blocks), dim3(64), eval_loop_lds, stream, t, gp.map, 0, 1);
+        const Grid gf = finish_grid(tmp, ids, true);
+        if (gf.blocks) hipLaunchKernelGGL(k_loop_finish, dim3(gf.blocks), dim3(kEvalThreads), 0, stream, t, gf.map, 0, 1);
       });
     timer.time("k_eval_init_general", stream, [&] {
       hipLaunchKernelGGL(k_eval<0>, dim3(ge.blocks), dim3(kEvalThreads), eval_general_lds, stream, t, ge.map, 0);
@@ -2289,9 +2328,9 @@ struct Batch::Impl {
         const Grid g = loop_grid(tmp, group);
         return g.blocks ? measure([&] {
           if (group == 1)
-            hipLaunchKernelGGL(k_eval_loop<false>, dim3(g.blocks), dim3(kEvalThreads), eval_loop_lds, stream, d_all, g.map, 1, 1);
+            hipLaunchKernelGGL(k_eval_loop<false>, dim3(g.blocks), dim3(64), eval_loop_lds, stream, d_all, g.map, 1, 1);
           else
-            hipLaunchKernelGGL(k_eval_loop<true>, dim3(g.blocks), dim3(kEvalThreads), eval_loop_lds, stream, d_all, g.map, 1, group);
+            hipLaunchKernelGGL(k_eval_loop<true>, dim3(g.blocks), dim3(64), eval_loop_lds, stream, d_all, g.map, 1, group);
         }) : 0.f;
       });
     }
@@ -2385,9 +2424,10 @@ struct Batch::Impl {
     // The three evaluation kernels score disjoint pending programs.
     branches({[&](hipStream_t s) {
                 if (loop_kernel && tune.loop_group == 1)
-                  launch_on(s, "k_eval_loop", g_eval_loop, k_eval_loop<false>, kEvalThreads, eval_loop_lds, 1, 1);
+                  launch_on(s, "k_eval_loop", g_eval_loop, k_eval_loop<false>, 64, eval_loop_lds, 1, 1);
                 else if (loop_kernel)
-                  launch_on(s, "k_eval_loop", g_eval_loop, k_eval_loop<true>, kEvalThreads, eval_loop_lds, 1, tune.loop_group);
+                  launch_on(s, "k_eval_loop", g_eval_loop, k_eval_loop<true>, 64, eval_loop_lds, 1, tune.loop_group);
+                if (loop_kernel) launch_on(s, "k_loop_finish", g_finish, k_loop_finish, kEvalThreads, 0, 1, tune.loop_group);
               },
               [&](hipStream_t s) {
                 launch_on(s, "k_eval", g_eval, k_eval<1>, kEvalThreads, eval_fast_lds, 1);

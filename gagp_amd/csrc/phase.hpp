@@ -404,11 +404,10 @@ constexpr int kMaxStack = 64;
 
 // Limits of the typed straight-line VM path (vm_fast in vm.hpp).
 constexpr int kFastStack = 16, kFastCode = 128, kFastPool = 128, kFastInputs = 4;
-// Limits of the typed looping VM path (vm_loop): hidden locals (one
+// Limits of the typed looping VM path (vm_steps): hidden locals (one
 // traversal's temporaries; sequential traversals reuse them), code and
 // constants held in registers.
 constexpr int kLoopStack = 6, kLoopLocals = 9, kLoopCode = 256, kLoopPool = 256;
-constexpr int kLoopSlots = kLoopStack + kLoopLocals;  // LDS slots per lane of the looping path
 // Tags of a traversal's fixed instruction sequences, held in the argc byte
 // of their first instruction (a LOAD or STORE, whose argc is otherwise 0);
 // the low bits give the direction (1 forward, 2 reverse).

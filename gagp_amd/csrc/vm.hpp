@@ -13,6 +13,7 @@
 #pragma once
 #include "core.hpp"
 #include "phase.hpp"
+#include "steps.hpp"
 
 namespace gagp_amd {
 
@@ -528,410 +529,371 @@ __device__ inline LaneResult vm_fast(const FastProgram& f, const FastInputs& in,
 // ---- typed looping path ----
 // A program certified like the straight-line path but with jumps, hidden
 // locals or IntList views (phase.hpp loop_operation): values are untagged
-// int64 (Bool as 0/1, an IntList as its view payload), the operand stack and
-// the hidden locals are 8-byte LDS slots per lane (conflict-free, addressed
-// by the instruction's static height and operand), and code and constants
-// sit in four register groups read with readlane. Lanes follow their own branches under the
-// reference's per-case semantics: fuel is charged per lane, and the wave
-// executes the smallest pending instruction index for the lanes that are at
-// it. That index is the previous one plus one except after a jump or when a
-// lane finished, where a wave minimum recomputes it.
-struct LoopProgram {
-  int w0[4], w1[4];  // instruction: op | argc << 8 | sp << 16 | fuel << 24, operand
-  int c0[4], c1[4];  // constant payload, low and high words
-  int len;
+// int64 (Bool as 0/1, an IntList as its view payload). It runs as decoded
+// steps (steps.hpp): the top of the operand stack is a register, and inputs,
+// hidden locals and the elements below the top are 8-byte LDS slots per lane
+// (slot-major, conflict-free). Step j sits in lane j % 64 of register group
+// j / 64 and is read with readlane, so a fetch costs no memory round trip.
+//
+// Lanes follow their own branches. The lanes at the smallest step index run
+// together as a group under the execution mask: inside a run the step index,
+// the decoded fields and the fuel charged are scalar, no operation is
+// predicated, and fuel is checked against the group's smallest balance by one
+// scalar compare. A run ends where the group's lanes part, a lane finishes,
+// or the group reaches the step at which other lanes wait; only there are the
+// per-lane indexes and balances written and the next group chosen.
+// Interpreting the bytecode itself, predicated and one instruction (or fixed
+// sequence) at a time, issued about 31 vector and 40 scalar instructions per
+// step and three times the steps; k_eval_loop has the measured times.
+struct StepProgram {
+  unsigned w0[4], w1[4], c0[4], c1[4];
+  int n;
 };
-__device__ inline LoopProgram loop_load(const ProgView& p, int lane) {
-  LoopProgram f;
-  f.len = p.len;
+__device__ inline StepProgram steps_load(GAS const Step* steps, int n, int lane) {
+  StepProgram f;
+  f.n = n;
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
     const int j = g * 64 + lane;
-    int w0 = 0, w1 = 0;
-    if (j < p.len) {
-      const Ins ins = p.code[j];
-      w0 = int(ins.op) | int(ins.argc) << 8 | int(ins.sp) << 16 | int(unsigned(ins.fuel) << 24);
-      w1 = ins.a;
+    Step s{0, 0, 0};
+    if (j < n) {
+      s.w0 = steps[j].w0;
+      s.w1 = steps[j].w1;
+      s.c = steps[j].c;
     }
-    std::int64_t v = 0;
-    if (j < p.n_pool) {
-      const Val x = p.pool[j];
-      v = x.tag == TAG_BOOL ? std::int64_t(x.b != 0) : x.i;
-    }
-    f.w0[g] = w0;
-    f.w1[g] = w1;
-    f.c0[g] = int(std::uint32_t(std::uint64_t(v)));
-    f.c1[g] = int(std::uint32_t(std::uint64_t(v) >> 32));
+    f.w0[g] = s.w0;
+    f.w1[g] = s.w1;
+    f.c0[g] = unsigned(std::uint64_t(s.c));
+    f.c1[g] = unsigned(std::uint64_t(s.c) >> 32);
   }
   return f;
 }
-// The binary operations of the looping path on untagged operands; `zero`:
-// MOD by zero (ZeroDivisionError). MOD is Python's, by the shared truncating
-// division of vm_fast.
-__device__ inline std::int64_t loop_binary(int op, std::int64_t x, std::int64_t y, bool& zero) {
-  switch (op) {
-    case OP_ADD: return wrap_add(x, y);
-    case OP_SUB: return wrap_sub(x, y);
-    case OP_MUL: return wrap_mul(x, y);
-    case OP_LT: return x < y;
-    case OP_LE: return x <= y;
-    case OP_GT: return x > y;
-    case OP_GE: return x >= y;
-    case OP_EQ: return x == y;
-    case OP_NE: return x != y;
-    default: {  // OP_MOD
-      const std::int64_t safe = (y == 0 || y == -1) ? 1 : y;
-      const std::int64_t rem = y == -1 ? 0 : x - (x / safe) * safe;
-      zero = y == 0;
-      return y == 0 ? 0 : ((rem != 0 && ((rem < 0) != (y < 0))) ? rem + y : rem);
-    }
+// Word `v` of step k (uniform, below 64 * kGroups).
+template <int kGroups>
+__device__ inline unsigned step_word(const unsigned (&v)[4], int k) {
+  if constexpr (kGroups == 1) return unsigned(__builtin_amdgcn_readlane(int(v[0]), k));
+  const int g = k & 63;
+  unsigned w = unsigned(__builtin_amdgcn_readlane(int(v[0]), g));
+  if (k >= 64) {
+    const unsigned w1 = unsigned(__builtin_amdgcn_readlane(int(v[1]), g));
+    const unsigned w2 = unsigned(__builtin_amdgcn_readlane(int(v[2]), g)), w3 = unsigned(__builtin_amdgcn_readlane(int(v[3]), g));
+    w = k < 128 ? w1 : k < 192 ? w2 : w3;
   }
+  return w;
 }
-__device__ inline int loop_pick(const int (&v)[4], int k) {
-  const int x0 = __builtin_amdgcn_readlane(v[0], k & 63), x1 = __builtin_amdgcn_readlane(v[1], k & 63);
-  const int x2 = __builtin_amdgcn_readlane(v[2], k & 63), x3 = __builtin_amdgcn_readlane(v[3], k & 63);
-  return k < 128 ? (k < 64 ? x0 : x1) : (k < 192 ? x2 : x3);
+// Smallest value over the wave (all lanes active), in the data-parallel
+// shifts: row of 16, then across rows; the last lane holds the result.
+__device__ inline int wave_min_all(int x) {
+  const auto shifted = [&](auto control, auto rows) {
+    const int y = __builtin_amdgcn_update_dpp(0x7fffffff, x, decltype(control)::value, decltype(rows)::value, 0xf, false);
+    x = y < x ? y : x;
+  };
+  shifted(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{});
+  shifted(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{});
+  shifted(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{});
+  shifted(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{});
+  shifted(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});
+  shifted(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});
+  return __builtin_amdgcn_readlane(x, 63);
 }
-// `slots`: this wave's LDS area of kLoopSlots untagged slots, slot-major
-// (slot k of lane j at k * 64 + j): the operand stack, then the hidden locals.
-__device__ inline LaneResult vm_loop(const LoopProgram& f, FastInputs in, int n_inputs, GAS const std::int64_t* arena,
-                                     LAS std::int64_t* slots, int lane, bool active, int fuel0, int result_tag) {
-  // `in` is this lane's copy: statement targets may store into inputs.
+// Truncating quotient and remainder of x by y (y neither 0 nor -1) for the
+// active lanes. Where every operand fits 32 bits the quotient comes from one
+// refined double reciprocal: |x| / |y| is below 2^32 and the reciprocal is
+// good to 2^-44, so the floor is the quotient or one off, the fused remainder
+// is exact and one correction either way settles it.
+__device__ inline void divide_trunc(std::int64_t x, std::int64_t y, std::int64_t& q, std::int64_t& rem) {
+  const bool wide = x != std::int64_t(int(x)) || y != std::int64_t(int(y));
+  if (__ballot(wide) == 0) {
+    const double a = __builtin_fabs(double(int(x))), b = __builtin_fabs(double(int(y)));
+    double r = __builtin_amdgcn_rcp(b);
+    r = __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);
+    double f = __builtin_floor(a * r), m = __builtin_fma(-f, b, a);
+    const bool under = m < 0;
+    f = under ? f - 1 : f;
+    m = under ? m + b : m;
+    const bool over = m >= b;
+    f = over ? f + 1 : f;
+    m = over ? m - b : m;
+    const std::int64_t uq = std::int64_t(unsigned(f)), ur = std::int64_t(unsigned(m));
+    q = (x < 0) != (y < 0) ? -uq : uq;
+    rem = x < 0 ? -ur : ur;
+    return;
+  }
+  q = x / y;
+  rem = x - q * y;
+}
+// MOD and the protected divisions on untagged operands (MOD by zero: 0).
+__device__ inline std::int64_t step_divide(int op, std::int64_t x, std::int64_t y) {
+  const std::int64_t safe = (y == 0 || y == -1) ? 1 : y;
+  std::int64_t q, rem;
+  divide_trunc(x, safe, q, rem);
+  if (y == -1) { q = wrap_neg(x); rem = 0; }
+  const std::int64_t floor_mod = (rem != 0 && ((rem < 0) != (y < 0))) ? rem + y : rem;  // Python %
+  if (op == SO_MOD || op == SO_IMOD0) return y == 0 ? 0 : floor_mod;                              // py_mod
+  if (op == SO_IDIV0) return y == 0 ? 0 : q;                                                       // wrap_div
+  const bool none = y == 0 || (x == INT64_MIN && y == -1);
+  return none ? 0 : op == SO_TDIV0 ? q : rem;                                                      // trunc_div0, trunc_mod0
+}
+// `slots`: this wave's LDS area of step_slots(n_inputs) slots (slot k of lane
+// j at k * 64 + j). kGroups: register groups that hold the program's steps.
+// The run loop is one nest of two-way uniform branches with a single exit (no
+// switch, break or continue) and no divergent branch: what a lane records when
+// it ends is written after the loop, from the event that ended it. In this
+// form the compiler keeps the step index, the fields, the balances and the
+// event in scalar registers and only the stack's top in vector ones; any
+// per-lane record merged inside the loop would be copied on every path of
+// every step.
+template <int kGroups>
+__device__ inline LaneResult vm_steps(const StepProgram& f, const FastInputs& in, int n_inputs, GAS const std::int64_t* arena,
+                                      LAS std::int64_t* slots, int lane, bool active, int fuel0, int result_tag) {
+  constexpr int kNone = 0x7fffffff, kMost = 12;  // the largest charge of a step
+  constexpr unsigned kStepNoSlot = ~0u;
+  enum Event : int { EV_NONE, EV_BRANCH, EV_TEST, EV_ZERO_DIV, EV_VALUE, EV_RETURN, EV_FAIL_TYPE, EV_FAIL_VALUE };
   LaneResult r{0, TAG_INVALID, 0, active ? ERR_NONE : ERR_VALUE, 0};
-  bool done = !active;
   LAS std::int64_t* const sl = slots + lane;
-  // Heights are certified below kLoopStack; the clamp keeps every slot in range.
-  const auto S = [&](int k) -> LAS std::int64_t& { return sl[(k < 0 ? 0 : k < kLoopStack ? k : kLoopStack - 1) * 64]; };
-  const auto L = [&](int k) -> LAS std::int64_t& { return sl[(kLoopStack + (k < 0 ? 0 : k < kLoopLocals ? k : 0)) * 64]; };
-  unsigned assigned = 0;  // hidden locals stored so far
-  int fuel = fuel0, ip = 0, at = 0;
-  // The top of this lane's operand stack lives in a register; the LDS
-  // slots hold the elements below it (slot k: element k, for k < height - 1).
-  // Only the lanes that execute a step change either.
-  std::int64_t tos = 0;
-  // Every step that finishes a lane, jumps or runs a fixed sequence sets
-  // `resched`; any other step leaves the live lanes as they were, at + 1.
-  bool resched = true;
-  // Every step runs one instruction of at least one live lane, which charges
-  // fuel, so this bound is never reached by a certified program. A wave that
-  // never stops must jump, so the bound is checked when rescheduling.
-  const long long limit = 64LL * ((long long)fuel0 + 2LL * f.len + 2) + 64;
-  for (long long step = 0;; ++step) {
-    if (resched) {
-      // Converged live lanes (the common case) share their ip; otherwise
-      // take the smallest one.
-      const unsigned long long live = __ballot(!done);
-      if (live == 0) break;
-      if (step > limit) {
-        if (!done) { r.err = ERR_VALUE; r.fuel_used = fuel0 - fuel; done = true; }
-        break;
-      }
-      const int lead = __builtin_amdgcn_readlane(ip, __ffsll((long long)live) - 1);
-      if (__ballot(!done && ip != lead) == 0) at = lead;
-      else at = __builtin_amdgcn_readfirstlane(wave_min_bits<9>(done ? 511 : (ip < 511 ? ip : 510)));  // ip <= len <= 256
-      resched = false;
-    }
-    // `at` is wave-uniform on every path; restating that keeps it (and the
-    // decode below) in scalar registers across the loop's merges.
-    at = __builtin_amdgcn_readfirstlane(at);
-    const bool mine = !done && ip == at;
-    if (at >= f.len) {  // ran off the end without RETURN
-      if (mine) { r.err = ERR_VALUE; r.fuel_used = fuel0 - fuel; done = true; }
-      resched = true;
-      continue;
-    }
-    // The decoded fields are scalar values; readfirstlane states that for
-    // the compiler, which then indexes the register arrays with them.
-    const int w = __builtin_amdgcn_readfirstlane(loop_pick(f.w0, at)), a = __builtin_amdgcn_readfirstlane(loop_pick(f.w1, at));
-    const int op = w & 0xff, argc = (w >> 8) & 0xff, sp = (w >> 16) & 0xff, cost = int(unsigned(w) >> 24);
-    if ((argc & 0x80) && (argc & 0xf0) != kFuse) {
-      // A traversal's or for_range loop's fixed sequence as one step
-      // (phase.hpp kWalkTest, kWalkNext, kRangeTest, kRangeNext). Every
-      // instruction of it costs one unit of fuel and none
-      // can fail otherwise, so a lane with fewer units than the sequence
-      // charges times out inside it, with no fuel left.
-      const bool reverse = (argc & 3) == 2;
-      const int k_counter = a - n_inputs;
-      const int tag = argc & 0xf0;
-      if (tag == kRangeTest || tag == kRangeNext) {
-        // A for_range step (phase.hpp kRangeTest, kRangeNext): unit costs
-        // and no failure but fuel, as for the traversal sequences.
-        const bool test = tag == kRangeTest;
-        const int k_bound = __builtin_amdgcn_readfirstlane(loop_pick(f.w1, at + 1)) - n_inputs;
-        const int exit_at = __builtin_amdgcn_readfirstlane(loop_pick(f.w1, at + 3));
-        const int k_var = __builtin_amdgcn_readfirstlane(loop_pick(f.w1, at + 5)) - n_inputs;
-        const int head = __builtin_amdgcn_readfirstlane(loop_pick(f.w1, at + 4));
-        const std::int64_t counter = L(k_counter);
-        const bool more = test && counter < L(k_bound);
-        const int need = test ? (more ? 6 : 4) : 5;
-        const bool starve = mine && fuel < need;
-        const bool run = mine && !starve;
-        if (run) {
-          if (more && k_var < 0) {
-            in.set(k_var + n_inputs, counter);  // an input target (uniform)
-          } else if (more) {
-            L(k_var) = counter;
-            assigned |= 1u << k_var;
-          } else if (!test) {
-            L(k_counter) = wrap_add(counter, 1);
-          }
-          fuel -= need;
-          ip = test ? (more ? at + 6 : exit_at) : head;
-        }
-        if (starve) {
-          fuel = 0;
-          r.err = ERR_TIMEOUT;
-          r.fuel_used = fuel0;
-          done = true;
-        }
-      } else if (tag == kWalkTest) {
-        // LOAD counter, LOAD bound, LT/GE, JIF done, LOAD xs, LOAD counter,
-        // index, STORE element, LOAD start, LOAD counter, ADD, STORE index.
-        const int k_bound = __builtin_amdgcn_readfirstlane(loop_pick(f.w1, at + 1)) - n_inputs;
-        const int done_at = __builtin_amdgcn_readfirstlane(loop_pick(f.w1, at + 3));
-        const int k_xs = __builtin_amdgcn_readfirstlane(loop_pick(f.w1, at + 4)) - n_inputs;
-        const int k_element = __builtin_amdgcn_readfirstlane(loop_pick(f.w1, at + 7)) - n_inputs;
-        const int k_start = __builtin_amdgcn_readfirstlane(loop_pick(f.w1, at + 8)) - n_inputs;
-        const int k_index = __builtin_amdgcn_readfirstlane(loop_pick(f.w1, at + 11)) - n_inputs;
-        const std::int64_t counter = L(k_counter), bound = L(k_bound);
-        const bool more = reverse ? counter >= bound : counter < bound;
-        const int need = more ? 12 : 4;
-        const bool starve = mine && fuel < need;
-        const bool run = mine && !starve;
-        // The counter lies in [0, len): the element read is in bounds.
-        const std::int64_t xs = L(k_xs);
-        const bool read = run && more;
-        const std::int64_t element = arena[read ? (std::uint64_t(xs) >> 16) + std::uint64_t(counter) : 0];
-        if (read) {
-          L(k_element) = element;
-          L(k_index) = wrap_add(L(k_start), counter);
-          assigned |= (1u << k_element) | (1u << k_index);
-        }
-        if (run) {
-          fuel -= need;
-          ip = more ? at + 12 : done_at;
-        }
-        if (starve) {
-          fuel = 0;
-          r.err = ERR_TIMEOUT;
-          r.fuel_used = fuel0;
-          done = true;
-        }
+  for (int k = 0; k < n_inputs; ++k) sl[k * 64] = in.pick(k);
+  bool done = !active;
+  std::int64_t top = 0;
+  int ip = 0, fuel = fuel0;
+  // No live lane has less fuel than `low`. Lanes with an unbound input run
+  // step by step, checked before each.
+  unsigned bound = in.bound;
+  const bool unbound = __ballot(active && (~bound & ((1u << n_inputs) - 1u)) != 0) != 0;
+  int low = unbound ? 0 : fuel0;
+  for (;;) {
+    const unsigned long long live = __ballot(!done);
+    if (live == 0) break;
+    // The group: the lanes at the smallest index; `stop`: the next one at
+    // which lanes wait. Mostly one index, or two.
+    int at = __builtin_amdgcn_readlane(ip, __ffsll((long long)live) - 1), stop = f.n;
+    const unsigned long long same = __ballot(!done && ip == at);
+    if (same != live) {
+      const int other = __builtin_amdgcn_readlane(ip, __ffsll((long long)(live & ~same)) - 1);
+      if ((same | __ballot(!done && ip == other)) == live) {
+        stop = at < other ? other : at;
+        at = at < other ? at : other;
       } else {
-        // STORE state, LOAD counter, PUSH 1, ADD/SUB, STORE counter, JMP head.
-        const int k_state = k_counter;
-        const int k_step = __builtin_amdgcn_readfirstlane(loop_pick(f.w1, at + 1)) - n_inputs;
-        const int head = __builtin_amdgcn_readfirstlane(loop_pick(f.w1, at + 5));
-        const bool starve = mine && fuel < 6;
-        const bool run = mine && !starve;
-        const std::int64_t deeper = S(sp - 2);  // the top once the state is stored
-        if (run) {
-          L(k_state) = tos;
-          assigned |= 1u << k_state;
-          const std::int64_t c = L(k_step);
-          L(k_step) = reverse ? wrap_sub(c, 1) : wrap_add(c, 1);
-          fuel -= 6;
-          ip = head;
-          tos = deeper;
-        }
-        if (starve) {
-          fuel = 0;
-          r.err = ERR_TIMEOUT;
-          r.fuel_used = fuel0;
-          done = true;
-        }
+        at = wave_min_all(done ? kNone : ip);
+        stop = wave_min_all(done || ip == at ? kNone : ip);
       }
-      resched = true;
+    }
+    // Restated as uniform: values merged where the branches above part are
+    // not known to be.
+    at = __builtin_amdgcn_readfirstlane(at);
+    stop = __builtin_amdgcn_readfirstlane(stop);
+    low = __builtin_amdgcn_readfirstlane(low);
+    if (at >= f.n) {  // ran off the end without RETURN
+      if (!done && ip == at) { r.err = ERR_VALUE; r.fuel_used = fuel0 - fuel; done = true; }
       continue;
     }
-    if ((argc & 0xf0) == kFuse) {
-      // A LOAD or PUSH_CONST and the binary operation after it (phase.hpp
-      // kFuse) as one step, when every lane at `at` has the fuel of both;
-      // otherwise the first runs alone below.
-      const int w2 = __builtin_amdgcn_readfirstlane(loop_pick(f.w0, at + 1));
-      const int op2 = w2 & 0xff, cost2 = int(unsigned(w2) >> 24);
-      if (__ballot(mine && fuel < cost + cost2) == 0) {
-        std::int64_t y;
-        bool bound = true;
-        if (op == OP_PUSH_CONST) {
-          const std::uint32_t lo = std::uint32_t(loop_pick(f.c0, a)), hi = std::uint32_t(loop_pick(f.c1, a));
-          y = std::int64_t(std::uint64_t(hi) << 32 | lo);
-        } else if (a < n_inputs) {  // uniform branch
-          y = in.pick(a);
-          bound = (in.bound >> (a & 31)) & 1u;
-        } else {
-          const int k = a - n_inputs < kLoopLocals ? a - n_inputs : 0;
-          y = L(k);
-          bound = (assigned >> k) & 1u;
+    const bool mine = !done && ip == at;
+    int budget = low;
+    if (low < kMost) {
+      // Near exhaustion the group takes one step at a time. Lanes that cannot
+      // pay for it end here, their last unit charged inside it (every
+      // instruction charges one).
+      const unsigned w0 = step_word<kGroups>(f.w0, at), w1 = step_word<kGroups>(f.w1, at);
+      const int op = int(w0 & 63u);
+      int need = int(w0 >> 24), err = ERR_TIMEOUT, used = fuel0;
+      if (op == SO_WALK_TEST || op == SO_RANGE_TEST) {
+        const std::int64_t counter = sl[(w1 & 31u) * 64], limit = sl[((w1 >> 5) & 31u) * 64];
+        const bool reverse = op == SO_WALK_TEST && (step_word<kGroups>(f.c0, at) >> 24) != 0;
+        if (!(reverse ? counter >= limit : counter < limit)) need = 4;
+      }
+      bool fails = mine && fuel < need;
+      if (unbound && op < kStepControl) {
+        // Loads of unbound inputs, in order: an exchanged pair's first operand
+        // is its second load.
+        const unsigned a = w1 & 31u, b = (w1 >> 5) & 31u, loads = w0 >> 14 & 3u;
+        const bool x_out = (w0 & kStepX) && a < unsigned(n_inputs) && !(bound >> a & 1u);
+        const bool y_out = ((w0 >> 8) & 3u) == 1 && b < unsigned(n_inputs) && !(bound >> b & 1u);
+        const int charge = x_out ? (loads == 3 ? 2 : 1) : (loads >= 2 ? 2 : 1);
+        if (mine && (x_out || y_out) && fuel >= charge) {
+          fails = true;
+          err = ERR_NAME;
+          used = fuel0 - fuel + charge;
         }
-        bool zero = false;
-        const std::int64_t v = loop_binary(op2, tos, y, zero);
-        int err2 = ERR_NONE;
-        if (mine) {
-          if (!bound) {
-            err2 = ERR_NAME;
-            fuel -= cost;
-          } else {
-            fuel -= cost + cost2;
-            if (zero) err2 = ERR_ZERO_DIV;
-            tos = v;
-            ip = at + 2;
-          }
-        }
-        if (mine && err2 != ERR_NONE) {
-          r.err = err2;
-          r.fuel_used = fuel0 - fuel;
-          done = true;
-        }
-        resched = true;
-        continue;
+      }
+      if (fails) { r.err = err; r.fuel_used = used; done = true; }
+      if (__ballot(fails) != 0) continue;
+      if (!unbound) {
+        // Other lanes may be the ones near exhaustion.
+        low = wave_min_all(done ? kNone : fuel);
+        budget = wave_min_all(mine ? fuel : kNone);
       }
     }
-    // Every lane computes the instruction; the lanes at `at` with fuel
-    // commit it (predication instead of divergent branches).
-    const bool starve = mine && fuel < cost;
-    const bool run = mine && !starve;
-    int err = starve ? ERR_TIMEOUT : ERR_NONE;
-    bool ret = false;
-    int next = ip + 1;
-    const int below = sp - 2, push = sp;
-    // Binary operations read both operands before any store.
-    switch (op) {
-      case OP_PUSH_CONST: {
-        const std::uint32_t lo = std::uint32_t(loop_pick(f.c0, a)), hi = std::uint32_t(loop_pick(f.c1, a));
-        if (run) {
-          if (push > 0) S(push - 1) = tos;
-          tos = std::int64_t(std::uint64_t(hi) << 32 | lo);
-        }
-        break;
-      }
-      case OP_LOAD: {
-        std::int64_t v;
-        bool bound;
-        if (a < n_inputs) {  // uniform branch
-          v = in.pick(a);
-          bound = (in.bound >> (a & 31)) & 1u;
-        } else {
-          const int k = a - n_inputs < kLoopLocals ? a - n_inputs : 0;
-          v = L(k);
-          bound = (assigned >> k) & 1u;
-        }
-        if (run && !bound) err = ERR_NAME;
-        if (run) {
-          if (push > 0) S(push - 1) = tos;
-          tos = v;
-        }
-        break;
-      }
-      case OP_STORE: {
-        const std::int64_t deeper = S(below);  // the top after the pop
-        if (a < n_inputs) {  // an input target (uniform branch)
-          if (run) { in.set(a, tos); tos = deeper; }
-          break;
-        }
-        const int k = a - n_inputs < kLoopLocals ? a - n_inputs : 0;
-        if (run) { L(k) = tos; assigned |= 1u << k; tos = deeper; }
-        break;
-      }
-      case OP_JMP: next = a; break;
-      case OP_JMP_IF_FALSE: case OP_JMP_IF_TRUE: {
-        const std::int64_t deeper = S(below);  // the condition is popped
-        next = (tos != 0) == (op == OP_JMP_IF_TRUE) ? a : ip + 1;
-        if (run) tos = deeper;
-        break;
-      }
-      case OP_CHECK_INT: break;
-      // argc 1 marks a NEG of a Bool (the for_range bound check): TypeError.
-      case OP_NEG:
-        if (run && argc == 1) err = ERR_TYPE;
-        else if (run) tos = wrap_neg(tos);
-        break;
-      case OP_NOT: if (run) tos = std::int64_t(tos == 0); break;
-      case OP_ADD: case OP_SUB: case OP_MUL: case OP_MOD: case OP_LT: case OP_LE: case OP_GT: case OP_GE: case OP_EQ:
-      case OP_NE: {
-        bool zero = false;
-        const std::int64_t v = loop_binary(op, S(below), tos, zero);
-        if (run && zero) err = ERR_ZERO_DIV;
-        if (run) tos = v;
-        break;
-      }
-      case OP_CALL_BUILTIN: {
-        // The last argument is the register top; the others are below it.
-        const int base = sp - argc;
-        const std::int64_t x = argc == 1 ? tos : S(base), y = argc == 2 ? tos : S(base + 1);
-        std::int64_t out = 0;
-        switch (a) {
-          case B_ABS: out = x < 0 ? wrap_neg(x) : x; break;
-          case B_MIN: out = x < y ? x : y; break;
-          case B_MAX: out = x > y ? x : y; break;
-          case B_CLIP: {
-            const std::int64_t hi = argc == 3 ? tos : S(base + 2), m = x > y ? x : y;
-            out = m < hi ? m : hi;
-            break;
-          }
-          case B_IDIV0: case B_IMOD0: case B_TRUNC_DIV0: case B_TRUNC_MOD0: {
-            const std::int64_t safe = (y == 0 || y == -1) ? 1 : y;
-            std::int64_t q = x / safe, rem = x - q * safe;
-            if (y == -1) { q = wrap_neg(x); rem = 0; }
-            const std::int64_t floor_mod = (rem != 0 && ((rem < 0) != (y < 0))) ? rem + y : rem;
-            if (a == B_IDIV0) out = y == 0 ? 0 : q;
-            else if (a == B_IMOD0) out = y == 0 ? 0 : floor_mod;
-            else if (a == B_TRUNC_DIV0) out = (y == 0 || (x == INT64_MIN && y == -1)) ? 0 : q;
-            else out = (y == 0 || (x == INT64_MIN && y == -1)) ? 0 : rem;
-            break;
-          }
-          case B_LEN: out = std::int64_t(std::uint64_t(x) & 0xffff); break;
-          case B_IS_INT: out = 1; break;  // certified on an Int operand
-          case B_INDEX: case B_INDEX_NONNEG: case B_INDEX_CLAMPED: {  // as in vm_run
-            const std::int64_t n = std::int64_t(std::uint64_t(x) & 0xffff);
-            const std::uint64_t off = std::uint64_t(x) >> 16;
-            std::int64_t j = y;
-            bool ok = true, zero = false;
-            if (a == B_INDEX_CLAMPED) {
-              zero = n == 0;
-              j = j < 0 ? 0 : (j >= n ? n - 1 : j);
+    int charged = 0;
+    budget = __builtin_amdgcn_readfirstlane(budget);
+    if (mine) {
+      // Here ip == at, and the compiler may take the lane's value for both.
+      at = __builtin_amdgcn_readfirstlane(at);
+      int spent = 0, event = EV_NONE, last = at;
+      unsigned long long mask = 0;  // the lanes an event names
+      unsigned sink_slot = kStepNoSlot;
+      do {
+        const unsigned w0 = step_word<kGroups>(f.w0, at), w1 = step_word<kGroups>(f.w1, at);
+        const int op = int(w0 & 63u), cost = int(w0 >> 24);
+        budget -= cost;
+        spent += cost;
+        const int a = int(w1 & 31u), b = int((w1 >> 5) & 31u), p = int((w1 >> 10) & 31u), target = int(w1 >> 16);
+        int next = at + 1;
+        if (op < kStepControl) {
+          std::int64_t x = top, y = top;
+          if (w0 & kStepPush) sl[p * 64] = top;
+          if (w0 & kStepX) x = sl[a * 64];
+          const unsigned yk = (w0 >> 8) & 3u, sink = (w0 >> 10) & 7u;
+          if (yk == 2) y = std::int64_t(std::uint64_t(step_word<kGroups>(f.c1, at)) << 32 | step_word<kGroups>(f.c0, at));
+          else if (yk == 1) y = sl[b * 64];
+          unsigned long long holds = 0;
+          std::int64_t out = y;
+          if (op >= kStepBool) {
+            if (op < SO_GT) {
+              if (op < SO_LT) holds = op == SO_TEST ? __ballot(x != 0) : __ballot(x == 0);
+              else if (op == SO_LT) holds = __ballot(x < y);
+              else holds = __ballot(x <= y);
             } else {
-              if (a == B_INDEX_NONNEG && j < 0) ok = false;
-              if (j < 0) j += n;
-              if (j < 0 || j >= n) ok = false;
+              if (op < SO_EQ) {
+                if (op == SO_GT) holds = __ballot(x > y);
+                else holds = __ballot(x >= y);
+              } else {
+                if (op == SO_EQ) holds = __ballot(x == y);
+                else holds = __ballot(x != y);
+              }
             }
-            if (run && !ok) err = ERR_VALUE;
-            // Only running lanes with a valid index read the arena; the rest
-            // read its first element (the arena is never empty).
-            const bool read = run && ok && !zero;
-            const std::int64_t v = arena[read ? off + std::uint64_t(j) : 0];
-            out = read ? v : 0;
-            break;
+            out = std::int64_t((holds >> lane) & 1u);
+          } else if (op < SO_MIN) {
+            if (op < SO_SUB) {
+              if (op == SO_ADD) out = wrap_add(x, y);
+            } else {
+              if (op == SO_SUB) out = wrap_sub(x, y);
+              else out = wrap_mul(x, y);
+            }
+          } else if (op < SO_INDEX) {
+            if (op < SO_MOD) {
+              if (op == SO_MIN) out = x < y ? x : y;
+              else out = x > y ? x : y;
+            } else {
+              out = step_divide(op, x, y);
+              mask = op == SO_MOD ? __ballot(y == 0) : 0;
+              event = mask != 0 ? EV_ZERO_DIV : EV_NONE;
+            }
+          } else if (op < SO_NEG) {
+            // List indexing, as in vm_run. Only a valid index is read; the
+            // rest read the arena's first element (it is never empty).
+            const std::int64_t n = std::int64_t(std::uint64_t(x) & 0xffff);
+            const bool clamped = op == SO_INDEX_CLAMPED;  // an empty list reads as 0
+            const bool negative = op == SO_INDEX_NONNEG && y < 0;
+            const std::int64_t inside = y < 0 ? 0 : y >= n ? n - 1 : y, wrapped = y < 0 ? y + n : y;
+            const std::int64_t k = clamped ? inside : wrapped;
+            const bool ok = !negative && k >= 0 && k < n;
+            const std::int64_t v = arena[ok ? (std::uint64_t(x) >> 16) + std::uint64_t(k) : 0];
+            out = ok ? v : 0;
+            mask = clamped ? 0 : __ballot(!ok);
+            event = mask != 0 ? EV_VALUE : EV_NONE;
+          } else if (op < SO_LEN) {
+            out = op == SO_NEG || x < 0 ? wrap_neg(x) : x;  // NEG, ABS
+          } else if (op < SO_CLIP) {
+            out = op == SO_LEN ? std::int64_t(std::uint64_t(x) & 0xffff) : 1;
+          } else {
+            const std::int64_t m = x > y ? x : y;
+            out = m < top ? m : top;
           }
-          default: if (run) err = ERR_NAME; break;
+          if (sink < SK_IF_FALSE) {
+            top = out;
+            next = sink == SK_TOP_JUMP ? target : next;
+          } else {
+            if (sink == SK_STORE) {
+              sl[target * 64] = out;
+              sink_slot = unsigned(target);
+            } else {
+              const unsigned long long group = __ballot(true), jumps = sink == SK_IF_TRUE ? holds : group & ~holds;
+              mask = jumps;
+              event = jumps != 0 && jumps != group ? EV_BRANCH : EV_NONE;
+              next = jumps == group ? target : next;
+            }
+            if (w0 & kStepPop) top = sl[p * 64];
+          }
+        } else if (op < SO_WALK_TEST) {
+          event = op == SO_JUMP ? EV_NONE : EV_RETURN;
+          next = target;
+        } else if (op < SO_RANGE_TEST) {
+          if (op == SO_WALK_NEXT) {
+            sl[a * 64] = top;
+            if (w0 & kStepPop) top = sl[p * 64];
+            const std::int64_t counter = sl[b * 64];
+            sl[b * 64] = wrap_add(counter, step_word<kGroups>(f.c0, at) ? -1 : 1);
+            next = target;
+          } else {
+            // A loop's test: leaving it charges four units. Leaving lanes
+            // bind the arena's first element, which nothing reads.
+            const unsigned c0 = step_word<kGroups>(f.c0, at);
+            const std::int64_t counter = sl[a * 64], limit = sl[b * 64], xs = sl[p * 64], start = sl[((c0 >> 8) & 31u) * 64];
+            const bool more = (c0 >> 24) != 0 ? counter >= limit : counter < limit;
+            const unsigned long long stay = __ballot(more), group = __ballot(true);
+            // The counter of a staying lane lies in [0, length).
+            sl[(c0 & 31u) * 64] = arena[more ? (std::uint64_t(xs) >> 16) + std::uint64_t(counter) : 0];
+            sl[((c0 >> 16) & 31u) * 64] = wrap_add(start, counter);
+            mask = stay;
+            event = stay != 0 && stay != group ? EV_TEST : EV_NONE;
+            next = stay == 0 ? target : next;
+            const int refund = stay == 0 ? cost - 4 : 0;
+            budget += refund;
+            spent -= refund;
+          }
+        } else if (op < SO_FAIL_TYPE) {
+          const std::int64_t counter = sl[a * 64];
+          if (op == SO_RANGE_NEXT) {
+            sl[a * 64] = wrap_add(counter, 1);
+            next = target;
+          } else {
+            // Leaving lanes keep the variable.
+            const std::int64_t limit = sl[b * 64], old = sl[p * 64];
+            const bool more = counter < limit;
+            const unsigned long long stay = __ballot(more), group = __ballot(true);
+            sl[p * 64] = more ? counter : old;
+            sink_slot = unsigned(p);
+            mask = stay;
+            event = stay != 0 && stay != group ? EV_TEST : EV_NONE;
+            next = stay == 0 ? target : next;
+            const int refund = stay == 0 ? cost - 4 : 0;
+            budget += refund;
+            spent -= refund;
+          }
+        } else {
+          event = op == SO_FAIL_TYPE ? EV_FAIL_TYPE : EV_FAIL_VALUE;
         }
-        if (run) tos = out;
-        break;
+        last = at;
+        at = next;
+      } while (event == EV_NONE && at < stop && budget >= kMost);
+      // What ended the run.
+      const bool named = (mask >> lane) & 1u;
+      ip = at;
+      if (event == EV_BRANCH) {
+        ip = named ? int(step_word<kGroups>(f.w1, last) >> 16) : at;
+      } else if (event == EV_TEST) {
+        const unsigned w0 = step_word<kGroups>(f.w0, last);
+        ip = named ? at : int(step_word<kGroups>(f.w1, last) >> 16);
+        fuel += named ? 0 : int(w0 >> 24) - 4;
+      } else if (event != EV_NONE) {
+        const bool all = event >= EV_RETURN;
+        if (all || named) {
+          r.fuel_used = fuel0 - (fuel - spent);
+          done = true;
+          if (event == EV_RETURN) {
+            r.t = std::uint8_t(result_tag);
+            if (result_tag == TAG_BOOL) r.b = top != 0;
+            else r.v = top;
+          } else {
+            r.err = event == EV_ZERO_DIV ? ERR_ZERO_DIV : event == EV_FAIL_TYPE ? ERR_TYPE : ERR_VALUE;
+          }
+        }
       }
-      case OP_RETURN: ret = true; break;
-      default: if (run) err = ERR_VALUE; break;
+      if (unbound && sink_slot < unsigned(n_inputs)) bound |= named || event != EV_TEST ? 1u << sink_slot : 0u;
+      fuel -= spent;
+      charged = spent;
     }
-    if (run) {
-      ip = next;
-      fuel -= cost;
-    }
-    const bool finished = mine && (err != ERR_NONE || ret);
-    if (finished) {
-      r.err = err;
-      if (err == ERR_NONE) {
-        const std::int64_t v = tos;
-        if (result_tag == TAG_BOOL) { r.t = TAG_BOOL; r.b = v != 0; r.v = 0; }
-        else { r.t = TAG_INT; r.v = v; }
-      }
-      r.fuel_used = fuel0 - fuel;
-      done = true;
-    }
-    // The next instruction index: after a jump, or when a lane at this index
-    // finished, recompute the minimum; otherwise every lane that ran is at
-    // at + 1 and every other live lane was already past `at`.
-    const bool jump = op == OP_JMP || op == OP_JMP_IF_FALSE || op == OP_JMP_IF_TRUE;
-    if (jump || __ballot(finished) != 0) resched = true;
-    else ++at;
+    // No lane was charged more than the group.
+    low -= unbound ? 0 : __builtin_amdgcn_readlane(charged, __ffsll((long long)__ballot(mine)) - 1);
   }
   return r;
 }
