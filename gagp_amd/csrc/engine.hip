@@ -1488,7 +1488,7 @@ __global__ __launch_bounds__(kEvalThreads) void k_eval_programs(const DProg* pro
   double* scores = kFast ? reinterpret_cast<double*>(smem) + std::size_t(wave) * e.cd.C : nullptr;
   for (int i = blockIdx.x * kWavesPerBlock + wave; i < n; i += gridDim.x * kWavesPerBlock) {
     const DProg p = progs[i];
-    if ((p.fast != 0) != kFast) continue;
+    if (p.fast != int(kFast)) continue;  // 2: k_eval_steps scores it
     const EvalOut r = eval_program<kFast ? 1 : 0>(e, view_of(p), st, scores, lane);
     if (lane == 0) {
       fitness[i] = r.fitness;
@@ -1497,6 +1497,80 @@ __global__ __launch_bounds__(kEvalThreads) void k_eval_programs(const DProg* pro
       counts[3 * i + 1] = r.errors;
       counts[3 * i + 2] = r.timeouts;
     }
+  }
+}
+// A caller's looping programs on the decoded steps (certify_loop): one block
+// per program, whose wavefronts take its 64-case tiles in turn in the visiting
+// order (longest lists first). Totals are combined in LDS as in k_eval_tiles.
+// LDS: step_slots(n_inputs) slots per wavefront, then C scores. Bound by the
+// step loop's issue, as k_eval_loop; 512 programs x 200 list cases took
+// 6.17 ms on the general VM (tagged values, a few cases' branches predicated
+// per instruction) and take 0.45 ms here.
+struct StepProg { GAS const Step* steps; int n_steps, index, result_tag; };
+__global__ __launch_bounds__(kEvalThreads) void k_eval_steps(const StepProg* progs, int n, EvalParams e, double* fitness,
+                                                              unsigned* wrong, unsigned* counts) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  __shared__ double part_sum[kWavesPerBlock];
+  __shared__ unsigned part_count[kWavesPerBlock][4];  // wrong, errors, timeouts, integral
+  const int waves = int(blockDim.x) / 64, wave = wave_index(), lane = threadIdx.x % 64;
+  const int C = e.cd.C, n_in = e.cd.n_inputs, slots = step_slots(n_in);
+  LAS std::int64_t* const sl = (LAS std::int64_t*)smem + std::size_t(wave) * slots * 64;
+  double* const scores = reinterpret_cast<double*>(smem + std::size_t(waves) * slots * 64 * 8);
+  for (int i = blockIdx.x; i < n; i += gridDim.x) {  // one program per block, uniform
+    const StepProg p = progs[i];
+    const StepProgram sp = steps_load(p.steps, p.n_steps, lane);
+    double isum = 0;
+    unsigned w = 0, errs = 0, touts = 0;
+    bool integral = true;  // C <= kScoreCases <= 4096
+    for (int tile = wave * 64; tile < C; tile += waves * 64) {
+      const bool active = tile + lane < C;
+      const int c = active ? e.cd.order[tile + lane] : 0;
+      const FastInputs in = fast_inputs(e.cd, n_in, c, active);
+      const LaneResult r = sp.n <= 64 ? vm_steps<1>(sp, in, n_in, e.cd.arena, sl, lane, active, e.fuel, p.result_tag)
+                                      : vm_steps<4>(sp, in, n_in, e.cd.arena, sl, lane, active, e.fuel, p.result_tag);
+      if (active) {
+        bool exact = false;
+        const double sc = lane_score(e, r, expected_of(e.cd, c), exact);
+        w += !exact;
+        errs += r.err != ERR_NONE;
+        touts += r.err == ERR_TIMEOUT;
+        integral = integral && sc == double(std::int64_t(sc)) && sc >= -68719476736.0 && sc <= 68719476736.0;
+        isum += sc;
+        scores[c] = sc;
+      }
+    }
+    const double ws = wave_sum_d(isum);
+    const unsigned ww = wave_sum_u(w), we = wave_sum_u(errs), wt = wave_sum_u(touts);
+    const bool wint = __ballot(!integral) == 0;
+    if (lane == 0) {
+      part_sum[wave] = ws;
+      part_count[wave][0] = ww;
+      part_count[wave][1] = we;
+      part_count[wave][2] = wt;
+      part_count[wave][3] = wint;
+    }
+    __syncthreads();  // every wavefront's scores and totals
+    if (wave == 0) {
+      double total = 0;
+      unsigned tw = 0, te = 0, tt = 0;
+      bool all_integral = true;
+      for (int k = 0; k < waves; ++k) {
+        total += part_sum[k];
+        tw += part_count[k][0];
+        te += part_count[k][1];
+        tt += part_count[k][2];
+        all_integral = all_integral && part_count[k][3] != 0;
+      }
+      const double f = all_integral ? total : canonical_from_scores(e, C, scores, lane);
+      if (lane == 0) {
+        fitness[p.index] = f;
+        wrong[p.index] = e.policy.metric == METRIC_LEGACY ? 0 : tw;
+        counts[3 * p.index + 0] = unsigned(C);
+        counts[3 * p.index + 1] = te;
+        counts[3 * p.index + 2] = tt;
+      }
+    }
+    __syncthreads();  // before the next program reuses the scores
   }
 }
 template <bool kFast>
@@ -3265,14 +3339,119 @@ FastCert certify_fast(const std::vector<Ins>& code, const std::vector<Val>& cons
   return cert;  // falls off the end: the general VM reports it
 }
 
+// The looping certificate of external bytecode: the program runs on the
+// decoded steps when, by the types every path brings, each operand is an Int,
+// a Bool or an IntList view that an operation of the looping path takes
+// (loop_operation), every hidden local is stored before it is read, all
+// returns share one type, every instruction charges one unit and the limits
+// of the path hold. A forward data-flow pass over the verified code (whose
+// stack heights agree at joins); a local two paths leave with different types
+// has none.
+struct LoopCert { bool loop = false; int result_tag = TAG_INT; };
+LoopCert certify_loop(const std::vector<Ins>& code, const std::vector<Val>& consts, const std::vector<std::uint8_t>& input_tags,
+                      int n_locals, int max_stack, bool unit_fuel, int C) {
+  LoopCert cert;
+  const int n = int(code.size()), K = int(input_tags.size());
+  if (!unit_fuel || n > kLoopCode || int(consts.size()) > kLoopPool || max_stack > kLoopStack || K > kFastInputs ||
+      n_locals < K || n_locals - K > kLoopLocals || C > kScoreCases)
+    return cert;
+  struct State { std::uint8_t stack[kLoopStack], local[kFastInputs + kLoopLocals]; };
+  std::vector<State> at(std::size_t(n) + 1);
+  std::vector<char> seen(std::size_t(n) + 1, 0);
+  State first;
+  std::fill(std::begin(first.stack), std::end(first.stack), TAG_INVALID);
+  std::fill(std::begin(first.local), std::end(first.local), TAG_INVALID);
+  for (int k = 0; k < K; ++k) first.local[k] = input_tags[std::size_t(k)];
+  std::vector<int> work;
+  int returned = TAG_INVALID;
+  // Brings `s` (stack height h) to instruction `to`; false when two paths
+  // disagree on a stack element's type.
+  const auto flow = [&](int to, const State& s, int h) {
+    State& d = at[std::size_t(to)];
+    if (!seen[std::size_t(to)]) {
+      d = s;
+      seen[std::size_t(to)] = 1;
+      work.push_back(to);
+      return true;
+    }
+    for (int k = 0; k < h; ++k)
+      if (d.stack[k] != s.stack[k]) return false;
+    bool changed = false;
+    for (int k = 0; k < n_locals; ++k)
+      if (d.local[k] != s.local[k] && d.local[k] != TAG_INVALID) { d.local[k] = TAG_INVALID; changed = true; }
+    if (changed) work.push_back(to);
+    return true;
+  };
+  flow(0, first, 0);
+  while (!work.empty()) {
+    const int ip = work.back();
+    work.pop_back();
+    if (ip == n) continue;  // off the end: ValueError on the steps too
+    State s = at[std::size_t(ip)];
+    const Ins& x = code[std::size_t(ip)];
+    const int h = x.sp;
+    int after = h;
+    bool falls = true;
+    switch (x.op) {
+      case OP_PUSH_CONST: case OP_LOAD: {
+        if (x.op == OP_LOAD && x.a >= n_locals) return cert;
+        const std::uint8_t t = x.op == OP_LOAD ? s.local[x.a] : consts[std::size_t(x.a)].tag;
+        if (!loop_type(t)) return cert;
+        s.stack[h] = t;
+        after = h + 1;
+        break;
+      }
+      case OP_STORE:
+        if (x.a >= n_locals) return cert;
+        s.local[x.a] = s.stack[h - 1];
+        after = h - 1;
+        break;
+      case OP_JMP: if (!flow(x.a, s, h)) return cert; falls = false; break;
+      case OP_JMP_IF_FALSE: case OP_JMP_IF_TRUE:
+        if (s.stack[h - 1] != TAG_BOOL || !flow(x.a, s, h - 1)) return cert;
+        after = h - 1;
+        break;
+      case OP_RETURN:
+        if (!fast_type(s.stack[h - 1]) || (returned != TAG_INVALID && returned != s.stack[h - 1])) return cert;
+        returned = s.stack[h - 1];
+        falls = false;
+        break;
+      default: {
+        const bool call = x.op == OP_CALL_BUILTIN;
+        const int arity = call ? x.argc : x.op == OP_NEG || x.op == OP_NOT || x.op == OP_CHECK_INT ? 1 : 2;
+        if (arity < 1 || arity > 3) return cert;
+        const std::uint8_t* a = s.stack + (h - arity);
+        const bool is_int = call && x.a == B_IS_INT;
+        if (is_int ? (arity != 1 || a[0] != TAG_INT)
+                   : !loop_operation(x.op, call ? x.a : 0, arity, a[0], arity > 1 ? a[1] : 0, arity > 2 ? a[2] : 0))
+          return cert;
+        const bool boolean = is_int || x.op == OP_NOT || (x.op >= OP_LT && x.op <= OP_NE);
+        s.stack[h - arity] = boolean ? TAG_BOOL : TAG_INT;
+        after = h - arity + 1;
+        break;
+      }
+    }
+    if (falls && !flow(ip + 1, s, after)) return cert;
+  }
+  // Unreachable code is unverified: the general VM skips it.
+  if (returned == TAG_INVALID || std::count(seen.begin(), seen.end() - 1, 0) != 0) return cert;
+  cert.loop = true;
+  cert.result_tag = returned;
+  return cert;
+}
+
 namespace {
 // Host packing of one evaluation launch: verified code and pools laid out
-// back to back, with each program's offsets and certificate.
+// back to back, with each program's offsets and certificate (`fast`: 1 the
+// typed straight-line path, 2 the decoded steps, 0 the general VM).
 struct PackedPrograms {
   std::vector<Ins> code;
   std::vector<Val> pool;
   std::vector<std::size_t> code_off, pool_off;
   std::vector<int> lens, jumps, locals, fast, pool_n, result;
+  std::vector<Step> steps;  // of the looping programs
+  std::vector<std::size_t> step_off;
+  std::vector<int> step_n, step_index;
   int slots = 1, temps = 0, shadow = 0;
   bool any_fast = false, any_general = false;
 };
@@ -3288,9 +3467,12 @@ struct Session::Impl {
   double penalty;
   Policy policy;
   float last_ms = 0;
-  PackedPrograms pack(const std::vector<ProgramIn>& programs) const;
+  // `decode`: certify and decode looping programs for the steps.
+  PackedPrograms pack(const std::vector<ProgramIn>& programs, bool decode) const;
   std::vector<DProg> program_table(const PackedPrograms& k, GAS const Ins* code, GAS const Val* pool) const;
-  void launch(const PackedPrograms& k, const DProg* progs, int n, double* fit, unsigned* wrong, unsigned* counts) const;
+  std::vector<StepProg> step_table(const PackedPrograms& k, GAS const Step* steps) const;
+  void launch(const PackedPrograms& k, const DProg* progs, const StepProg* step_progs, int n, double* fit, unsigned* wrong,
+              unsigned* counts) const;
 };
 
 namespace {
@@ -3334,7 +3516,7 @@ Session::Session(const Cases& c, int fuel, int lanes, double penalty, Policy pol
 Session::~Session() = default;
 float Session::last_kernel_ms() const { return impl_->last_ms; }
 
-PackedPrograms Session::Impl::pack(const std::vector<ProgramIn>& programs) const {
+PackedPrograms Session::Impl::pack(const std::vector<ProgramIn>& programs, bool decode) const {
   const auto& I = *this;
   PackedPrograms k;
   bool stores = false;  // some program stores into an input
@@ -3345,10 +3527,25 @@ PackedPrograms Session::Impl::pack(const std::vector<ProgramIn>& programs) const
     const auto ins = verify_program(p, I.cases.cd.n_inputs, ms, j, &stores);
     for (const auto& v : p.consts) check_view(v, I.arena_len);
     const FastCert cert = certify_fast(ins, p.consts, I.input_tags, p.n_locals, ms, j, I.cases.cd.C);
-    k.fast.push_back(cert.fast);
-    k.result.push_back(cert.result_tag);
-    k.pool_n.push_back(int(p.consts.size()));
+    int kind = cert.fast ? 1 : 0, result = cert.result_tag;
+    if (!kind && decode) {
+      const bool unit = std::all_of(ins.begin(), ins.end(), [](const Ins& x) { return x.fuel == 1; });
+      const LoopCert loop = certify_loop(ins, p.consts, I.input_tags, p.n_locals, ms, unit, I.cases.cd.C);
+      if (loop.loop) {
+        kind = 2;
+        result = loop.result_tag;
+        Step steps[kStepMax];
+        const int n = decode_steps(ins.data(), int(ins.size()), p.consts.data(), I.cases.cd.n_inputs, false, steps);
+        k.step_off.push_back(k.steps.size());
+        k.step_n.push_back(n);
+        k.step_index.push_back(int(k.fast.size()));
+        k.steps.insert(k.steps.end(), steps, steps + n);
+      }
+    }
     k.slots = std::max(k.slots, ms + 1);
+    k.fast.push_back(kind);
+    k.result.push_back(result);
+    k.pool_n.push_back(int(p.consts.size()));
     k.code_off.push_back(k.code.size());
     k.pool_off.push_back(k.pool.size());
     k.code.insert(k.code.end(), ins.begin(), ins.end());
@@ -3372,8 +3569,16 @@ std::vector<DProg> Session::Impl::program_table(const PackedPrograms& k, GAS con
   return progs;
 }
 
-// Both evaluation kernels over a packed launch on the null stream.
-void Session::Impl::launch(const PackedPrograms& k, const DProg* progs, int n, double* fit, unsigned* wrong, unsigned* counts) const {
+std::vector<StepProg> Session::Impl::step_table(const PackedPrograms& k, GAS const Step* steps) const {
+  std::vector<StepProg> progs(k.step_n.size());
+  for (std::size_t i = 0; i < progs.size(); ++i)
+    progs[i] = StepProg{steps + k.step_off[i], k.step_n[i], k.step_index[i], k.result[std::size_t(k.step_index[i])]};
+  return progs;
+}
+
+// The evaluation kernels over a packed launch on the null stream.
+void Session::Impl::launch(const PackedPrograms& k, const DProg* progs, const StepProg* step_progs, int n, double* fit,
+                           unsigned* wrong, unsigned* counts) const {
   const auto& I = *this;
   const EvalParams e{I.cases.cd, I.fuel, I.lanes, I.penalty, I.policy};
   const std::size_t lds = std::size_t(kWavesPerBlock) * (k.slots + k.temps) * 64 * 10;
@@ -3385,6 +3590,16 @@ void Session::Impl::launch(const PackedPrograms& k, const DProg* progs, int n, d
     HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_eval_programs<true>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                int(fast_lds)));
   const int blocks = std::min(4096, (n + kWavesPerBlock - 1) / kWavesPerBlock);
+  if (const int loops = int(k.step_n.size())) {
+    const int waves = std::min(kWavesPerBlock, (I.cases.cd.C + 63) / 64);
+    const std::size_t step_lds =
+        std::size_t(waves) * step_slots(I.cases.cd.n_inputs) * 64 * 8 + 8 * std::size_t(I.cases.cd.C);
+    if (step_lds > 65536)
+      HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_eval_steps), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                 int(step_lds)));
+    hipLaunchKernelGGL(k_eval_steps, dim3(std::min(16384, loops)), dim3(64 * waves), step_lds, nullptr, step_progs, loops, e, fit,
+                       wrong, counts);
+  }
   if (k.any_fast)
     hipLaunchKernelGGL(k_eval_programs<true>, dim3(blocks), dim3(kEvalThreads), fast_lds, nullptr, progs, n, e, k.slots, k.temps,
                        k.shadow, fit, wrong, counts);
@@ -3398,11 +3613,13 @@ void Session::eval(const std::vector<ProgramIn>& programs, double* fitness, std:
   auto& I = *impl_;
   const int n = int(programs.size());
   if (!n) return;
-  const PackedPrograms k = I.pack(programs);
+  const PackedPrograms k = I.pack(programs, true);
   DeviceArena tmp;
   auto dcode = tmp.upload(k.code);
   auto dpool = tmp.upload(k.pool);
   auto dprogs = tmp.upload(I.program_table(k, dcode, dpool));
+  auto dsteps = tmp.upload(k.steps);
+  auto dloops = tmp.upload(I.step_table(k, dsteps));
   auto dfit = tmp.alloc<double>(std::size_t(n));
   auto dwrong = tmp.alloc<unsigned>(std::size_t(n));
   auto dcounts = tmp.alloc<unsigned>(std::size_t(n) * 3);
@@ -3410,7 +3627,7 @@ void Session::eval(const std::vector<ProgramIn>& programs, double* fitness, std:
   HIP_OK(hipEventCreate(&a));
   HIP_OK(hipEventCreate(&b));
   HIP_OK(hipEventRecord(a, nullptr));
-  I.launch(k, (const DProg*)dprogs, n, (double*)dfit, (unsigned*)dwrong, (unsigned*)dcounts);
+  I.launch(k, (const DProg*)dprogs, (const StepProg*)dloops, n, (double*)dfit, (unsigned*)dwrong, (unsigned*)dcounts);
   HIP_OK(hipEventRecord(b, nullptr));
   HIP_OK(hipEventSynchronize(b));
   HIP_OK(hipEventElapsedTime(&I.last_ms, a, b));
@@ -3462,8 +3679,14 @@ void Session::eval_static(const std::vector<ProgramIn>& programs, double* fitnes
   const auto& I = *impl_;
   const int n = int(programs.size());
   if (!n) return;
-  const PackedPrograms k = I.pack(programs);
+  // Steps are staged only where they fit beside the documented parts; a
+  // launch that fits without them then runs its looping programs on the
+  // general VM.
+  PackedPrograms k = I.pack(programs, true);
   const std::size_t need = static_bytes(std::size_t(n), k.code.size(), k.pool.size());
+  if (!k.steps.empty() && need <= kStaticScratchBytes &&
+      need + align256(k.steps.size() * sizeof(Step)) + align256(k.step_n.size() * sizeof(StepProg)) > kStaticScratchBytes)
+    k = I.pack(programs, false);
   if (need > kStaticScratchBytes)
     throw std::invalid_argument("programs need " + std::to_string(need) + " bytes of evaluation workspace; the allocation-free "
                                 "entry point holds at most " + std::to_string(kStaticScratchBytes));
@@ -3477,10 +3700,18 @@ void Session::eval_static(const std::vector<ProgramIn>& programs, double* fitnes
   auto* dwrong = reinterpret_cast<unsigned*>(carve(std::size_t(n) * sizeof(unsigned)));
   auto* dcounts = reinterpret_cast<unsigned*>(carve(std::size_t(3) * n * sizeof(unsigned)));
   const auto progs = I.program_table(k, gbl(static_cast<const Ins*>(dcode)), gbl(static_cast<const Val*>(dpool)));
+  StepProg* dloops = nullptr;
+  if (!k.steps.empty()) {
+    auto* dsteps = reinterpret_cast<Step*>(carve(k.steps.size() * sizeof(Step)));
+    dloops = reinterpret_cast<StepProg*>(carve(k.step_n.size() * sizeof(StepProg)));
+    const auto loops = I.step_table(k, gbl(static_cast<const Step*>(dsteps)));
+    HIP_OK(hipMemcpy(dsteps, k.steps.data(), k.steps.size() * sizeof(Step), hipMemcpyHostToDevice));
+    HIP_OK(hipMemcpy(dloops, loops.data(), loops.size() * sizeof(StepProg), hipMemcpyHostToDevice));
+  }
   HIP_OK(hipMemcpy(dcode, k.code.data(), k.code.size() * sizeof(Ins), hipMemcpyHostToDevice));
   HIP_OK(hipMemcpy(dpool, k.pool.data(), k.pool.size() * sizeof(Val), hipMemcpyHostToDevice));
   HIP_OK(hipMemcpy(dprogs, progs.data(), progs.size() * sizeof(DProg), hipMemcpyHostToDevice));
-  I.launch(k, dprogs, n, dfit, dwrong, dcounts);
+  I.launch(k, dprogs, dloops, n, dfit, dwrong, dcounts);
   HIP_OK(hipMemcpy(fitness, dfit, sizeof(double) * n, hipMemcpyDeviceToHost));
   if (wrong) HIP_OK(hipMemcpy(wrong, dwrong, sizeof(unsigned) * n, hipMemcpyDeviceToHost));
   if (counts) HIP_OK(hipMemcpy(counts, dcounts, sizeof(unsigned) * 3 * n, hipMemcpyDeviceToHost));
