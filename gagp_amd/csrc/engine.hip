@@ -163,28 +163,34 @@ __device__ inline void raise(const DSearch& d, int code) { atomicCAS(d.error, 0,
 // largest search).
 struct BlockMap { int search, block, blocks; };
 
-constexpr int kVaryWaves = 4;  // wavefronts (rows) per block of the row kernels
+// Wavefronts (rows) per block of the row kernels. Eight share one LDS copy of
+// the phase tables: with four, the list grammar's tables (21 KB a block) left
+// room for 28 wavefronts per CU where a population of 8192 brings 32, and the
+// last eighth of the children started 100 us late.
+constexpr int kVaryWaves = 8;
 
 // ---- initial population (phase_population_cpu.cpp:54-113) ----
 // One wavefront per member runs the derivation uniformly (as mutation does),
 // so members with different retry counts do not diverge within a wavefront.
+// kStaged as k_vary.
+template <bool kStaged>
 __global__ __launch_bounds__(64 * kVaryWaves) void k_init_pop(DSearch* all, const BlockMap* map) {
   const BlockMap bm = map[blockIdx.x];
   const DSearch& d = all[bm.search];
+  if (!d.active || d.imported || (d.stage_tables != 0) != kStaged) return;  // uniform per block
+  extern __shared__ __attribute__((aligned(16))) unsigned char vary_lds[];
+  const PhaseView g = kStaged ? stage_phase_tables<64 * kVaryWaves>(d.g, vary_lds) : view_of(d.g);
   const int m = bm.block * kVaryWaves + wave_index();
-  if (!d.active || d.imported || m >= d.P) return;
+  if (m >= d.P) return;
   const int sd = d.site_depth;
   const int ramp = sd < 2 ? sd : 2 + m % (sd - 1);
   const std::size_t o = std::size_t(m) * d.R;
   GenResult gen{ST_INVALID, 0, 0, 0};
   const int room = d.slot.max_variable_nodes < kPhaseCapacity ? d.slot.max_variable_nodes : kPhaseCapacity;
-  const PhaseView g = view_of(d.g);
   for (int logical = ramp, attempt = 0; gen.status != ST_OK; ++attempt) {
     if (room <= 0 || room > d.R) { raise(d, 101); return; }
     const std::uint64_t s = splitmix_mix(d.seed ^ splitmix_mix((std::uint64_t(m) * 8 + 0) * 64 + std::uint64_t(attempt)));
-    WaveTasks pending;
-    gen = generate_phase_with(g, g.root, 0, d.slot.max_depth, room, s, d.cur_origin + o, d.cur_cval + o, d.cur_site + o, logical,
-                              pending);
+    gen = derive_phase_w(g, g.root, 0, d.slot.max_depth, room, s, d.cur_origin + o, d.cur_cval + o, d.cur_site + o, logical);
     // A statement program may read an unassigned local: the next seed is tried.
     if (gen.status == ST_OK && d.slot.statement &&
         !locals_defined_w(g, CRow{d.cur_origin + o, d.cur_site + o, d.cur_cval + o, gen.nodes, gen.constants}))
@@ -305,8 +311,10 @@ __device__ inline int pending_at(int B, int kind, int i) { return kind == 0 ? i 
 // ---- reproduction: one wavefront per child (phase_operators.cuh:156-265) ----
 // kStaged: the block first copies the phase tables into LDS (searches whose
 // tables fit); otherwise the operators read them from global memory.
+// At most 64 vector registers, so eight wavefronts per SIMD: a population of
+// 8192 is resident at once.
 template <bool kStaged, bool kWalks>
-__global__ __launch_bounds__(64 * kVaryWaves) void k_vary(DSearch* all, const BlockMap* map) {
+__global__ __launch_bounds__(64 * kVaryWaves) __attribute__((amdgpu_num_vgpr(64))) void k_vary(DSearch* all, const BlockMap* map) {
   const BlockMap bm = map[blockIdx.x];
   const DSearch& d = all[bm.search];
   if (!search_live(d) || (d.stage_tables != 0) != kStaged || (d.walks != 0) != kWalks) return;  // uniform per block
@@ -1875,10 +1883,23 @@ struct SearchState {
     x.n_locals = int(train.input_names.size());
     x.site_depth = cfg.site_depth;
     x.seed = cfg.seed;
-    x.g = PhaseTables{a.upload(phase.exprs), int(phase.exprs.size()), a.upload(phase.prods), int(phase.prods.size()),
-                    a.upload(phase.nts), int(phase.nts.size()), a.upload(phase.domains), int(phase.domains.size()),
-                    a.upload(phase.values), int(phase.values.size()), a.upload(phase.minimum), phase.depth_count,
-                    phase.logical_count, phase.site_depth ? 1 : 0, phase.root};
+    // The phase tables back to back in one block (stage_phase_tables).
+    std::vector<unsigned char> tables;
+    const auto append = [&](const auto& v) {
+      using T = typename std::decay_t<decltype(v)>::value_type;
+      const std::size_t at = tables.size();
+      tables.resize(at + table_bytes(v.size() * sizeof(T)));
+      if (!v.empty()) std::memcpy(tables.data() + at, v.data(), v.size() * sizeof(T));
+      return at;
+    };
+    const std::size_t o_expr = append(phase.exprs), o_prod = append(phase.prods), o_nt = append(phase.nts),
+                      o_dom = append(phase.domains), o_val = append(phase.values), o_min = append(phase.minimum);
+    GAS unsigned char* const base = a.upload(tables);
+    x.g = PhaseTables{(GAS const PExpr*)(base + o_expr), int(phase.exprs.size()), (GAS const PProd*)(base + o_prod),
+                      int(phase.prods.size()), (GAS const PNt*)(base + o_nt), int(phase.nts.size()),
+                      (GAS const PDomain*)(base + o_dom), int(phase.domains.size()), (GAS const Val*)(base + o_val),
+                      int(phase.values.size()), (GAS const unsigned*)(base + o_min), phase.depth_count, phase.logical_count,
+                      phase.site_depth ? 1 : 0, phase.root};
     x.local_types = a.upload(train.input_types);
     DeviceCases dc;
     dc.upload(a, train);
@@ -2178,6 +2199,7 @@ struct Batch::Impl {
     const auto attr = [](const void* k, std::size_t bytes) {
       if (bytes > 65536) HIP_OK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)));
     };
+    attr(reinterpret_cast<const void*>(&k_init_pop<true>), vary_lds_bytes);
     attr(reinterpret_cast<const void*>(&k_vary<true, false>), vary_lds_bytes);
     attr(reinterpret_cast<const void*>(&k_vary<true, true>), vary_lds_bytes);
     attr(reinterpret_cast<const void*>(&k_eval<0>), eval_general_lds);
@@ -2236,7 +2258,11 @@ struct Batch::Impl {
       up_v.push_back(std::move(cval));
     }
     timer.time("k_init_pop", stream,
-               [&] { hipLaunchKernelGGL(k_init_pop, dim3(gi.blocks), dim3(64 * kVaryWaves), 0, stream, t, gi.map); });
+               [&] {
+                 if (vary_lds_bytes)
+                   hipLaunchKernelGGL(k_init_pop<true>, dim3(gi.blocks), dim3(64 * kVaryWaves), vary_lds_bytes, stream, t, gi.map);
+                 if (vary_global) hipLaunchKernelGGL(k_init_pop<false>, dim3(gi.blocks), dim3(64 * kVaryWaves), 0, stream, t, gi.map);
+               });
     timer.time("k_lower_members", stream,
                [&] { hipLaunchKernelGGL(k_lower_members<false>, dim3(gl.blocks), dim3(64 * kVaryWaves), 0, stream, t, gl.map); });
     if (any_walks(ids))

@@ -59,24 +59,31 @@ __device__ inline std::uint64_t wave_sum_u64(std::uint64_t x) {
 // a view of the copy. The operators then read expression, production,
 // domain and minimum-cost entries at LDS latency instead of one dependent
 // global round trip per lookup.
+// The tables lie back to back in one global block (t.expr is its start), so
+// the copy is one loop of 16-byte loads, all in flight at once.
 template <int kThreads>
 __device__ inline PhaseView stage_phase_tables(const PhaseTables& t, unsigned char* lds) {
+  const std::size_t bytes = phase_tables_bytes(t);
+  GAS const uint4* const from = (GAS const uint4*)t.expr;
+  uint4* const to = reinterpret_cast<uint4*>(lds);
+  for (std::size_t k = threadIdx.x; k < bytes / 16; k += kThreads) {
+    const unsigned x = from[k].x, y = from[k].y, z = from[k].z, w = from[k].w;
+    to[k] = make_uint4(x, y, z, w);
+  }
   std::size_t off = 0;
-  const auto copy = [&](GAS const void* src, std::size_t bytes) {
-    unsigned* dst = reinterpret_cast<unsigned*>(lds + off);
-    GAS const unsigned* from = (GAS const unsigned*)src;
-    for (std::size_t k = threadIdx.x; k < bytes / 4; k += kThreads) dst[k] = from[k];
-    off += table_bytes(bytes);
-    return static_cast<const void*>(dst);
+  const auto at = [&](std::size_t n) {
+    const void* p = lds + off;
+    off += table_bytes(n);
+    return p;
   };
   PhaseView v;
-  v.expr = static_cast<const PExpr*>(copy(t.expr, sizeof(PExpr) * std::size_t(t.n_expr)));
-  v.prod = static_cast<const PProd*>(copy(t.prod, sizeof(PProd) * std::size_t(t.n_prod)));
-  v.nt = static_cast<const PNt*>(copy(t.nt, sizeof(PNt) * std::size_t(t.n_nt)));
-  v.dom = static_cast<const PDomain*>(copy(t.dom, sizeof(PDomain) * std::size_t(t.n_dom)));
-  v.values = static_cast<const Val*>(copy(t.values, sizeof(Val) * std::size_t(t.n_values)));
+  v.expr = static_cast<const PExpr*>(at(sizeof(PExpr) * std::size_t(t.n_expr)));
+  v.prod = static_cast<const PProd*>(at(sizeof(PProd) * std::size_t(t.n_prod)));
+  v.nt = static_cast<const PNt*>(at(sizeof(PNt) * std::size_t(t.n_nt)));
+  v.dom = static_cast<const PDomain*>(at(sizeof(PDomain) * std::size_t(t.n_dom)));
+  v.values = static_cast<const Val*>(at(sizeof(Val) * std::size_t(t.n_values)));
   v.minimum = static_cast<const unsigned*>(
-      copy(t.minimum, sizeof(unsigned) * std::size_t(t.n_expr) * std::size_t(t.depth_count) * std::size_t(t.logical_count)));
+      at(sizeof(unsigned) * std::size_t(t.n_expr) * std::size_t(t.depth_count) * std::size_t(t.logical_count)));
   v.n_expr = t.n_expr;
   v.n_prod = t.n_prod;
   v.n_nt = t.n_nt;
@@ -160,6 +167,300 @@ __device__ inline int choose_production(const WaveTasks&, const PhaseView& g, co
     if (choice < 0) break;
   }
   return chosen;
+}
+
+// ---- derivation in lane registers ----
+// A grammar of at most 64 expressions, nonterminals and productions held one
+// entry per lane: lane e has expression e, lane k nonterminal k, lane i
+// production i. A field of a uniform entry is then a readlane (a few cycles)
+// where the tables cost a dependent LDS or global round trip.
+struct WaveGrammar {
+  unsigned expr;                  // kind [2:0], arity [6:3], scope count [10:7], BOUND well formed [11], target [31:16]
+  unsigned c01, c23, c45, c67;    // children, two per register
+  unsigned scopes;                // 4 bits per child: its scope count + 1, 0 to inherit
+  unsigned nt;                    // production offset [7:0], count [15:8], scope count [23:16], normalized [24]
+  int prod;                       // the production's expression
+  double weight;
+};
+// Fills `w`; false when the grammar does not fit.
+__device__ inline bool wave_grammar(const PhaseView& g, WaveGrammar& w) {
+  w = WaveGrammar{0, 0, 0, 0, 0, 0, 0, -1, 0.0};
+  if (g.n_expr > 64 || g.n_nt > 64 || g.n_prod > 64 || g.n_dom > 64 || g.depth_count > 256 || g.logical_count > 256) return false;
+  const int lane = wlane();
+  bool bad = false;
+  if (lane < g.n_expr) {
+    const PExpr& x = g.expr[lane];
+    const bool bound = x.node.arity == 0 && x.node.operand >= 0 && x.node.operand < 16;
+    w.expr = unsigned(x.kind) | unsigned(x.node.arity & 15) << 3 | unsigned(x.scope_count & 15) << 7 | unsigned(bound) << 11 |
+             unsigned(x.target) << 16;
+    w.c01 = unsigned(x.children[0] & 0xffff) | unsigned(x.children[1]) << 16;
+    w.c23 = unsigned(x.children[2] & 0xffff) | unsigned(x.children[3]) << 16;
+    w.c45 = unsigned(x.children[4] & 0xffff) | unsigned(x.children[5]) << 16;
+    w.c67 = unsigned(x.children[6] & 0xffff) | unsigned(x.children[7]) << 16;
+#pragma unroll
+    for (int k = 0; k < kMaxArity; ++k) {
+      w.scopes |= unsigned((x.child_scope[k] + 1) & 15) << (4 * k);
+      bad = bad || x.child_scope[k] > 14;
+    }
+    bad = bad || x.kind < 0 || x.kind > 7 || x.node.arity < 0 || x.node.arity > kMaxArity || x.scope_count < 0 || x.scope_count > 15 ||
+          x.target < -1 || x.target > 64;
+  }
+  if (lane < g.n_nt) {
+    const PNt n = g.nt[lane];
+    w.nt = unsigned(n.production_offset) | unsigned(n.production_count) << 8 | unsigned(n.scope_count & 255) << 16 |
+           unsigned(n.normalized != 0) << 24;
+  }
+  if (lane < g.n_prod) {
+    const PProd p = g.prod[lane];
+    w.prod = p.expression;
+    w.weight = p.weight;
+  }
+  return __ballot(bad) == 0;
+}
+// v mod n for 0 < n < 2^20: two exact double steps of 48 and 36 bits.
+__device__ inline unsigned mod_small(std::uint64_t v, unsigned n) {
+  const double d = double(n);
+  double r = __builtin_amdgcn_rcp(d);
+  r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
+  r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
+  const auto step = [&](double x) {  // x mod n for an integer x < 2^48: the quotient is right or one off
+    const double m = __builtin_fma(-__builtin_floor(x * r), d, x);
+    const double up = m < 0 ? m + d : m;
+    return up >= d ? up - d : up;
+  };
+  const double high = step(double(v >> 16));
+  return unsigned(step(high * 65536.0 + double(unsigned(v & 0xffff))));
+}
+// The draws of a SplitMix64 stream, 64 at a time: the stream is
+// counter-based, so lane k computes draw k.
+struct WaveDraws {
+  std::uint64_t base;  // state before draw 0
+  unsigned lo, hi;
+  int next = 0;
+  __device__ explicit WaveDraws(std::uint64_t state) : base(state) { fill(); }
+  __device__ void fill() {
+    const std::uint64_t v = splitmix_mix(base + std::uint64_t(wlane()) * 0x9e3779b97f4a7c15ULL);
+    lo = unsigned(v);
+    hi = unsigned(v >> 32);
+    next = 0;
+  }
+  __device__ std::uint64_t take() {
+    if (next == 64) {
+      base += 64 * 0x9e3779b97f4a7c15ULL;
+      fill();
+    }
+    const unsigned l = unsigned(rdlane(int(lo), next)), h = unsigned(rdlane(int(hi), next));
+    ++next;
+    return std::uint64_t(h) << 32 | l;
+  }
+  __device__ double unit() { return double(take() >> 11) * 0x1.0p-53; }
+};
+
+// generate_phase_with by one wavefront over a WaveGrammar: the same draws,
+// results and failures. Returns false, having done nothing that matters, when
+// the pending stack would pass 64 tasks, a constant's domain has 2^20 values
+// or more, or a draw might be rejected (the caller then runs the general
+// derivation). Pending tasks, one per lane, carry the minimum cost they
+// reserved; a reference goes straight on to the production it chose; a node's
+// children are costed and pushed by the lanes that hold them; and nodes
+// collect one per lane and are stored 64 at a time.
+// Bound by its chain of dependent steps, each one LDS round trip and a few
+// dozen scalar instructions: a subtree of 31 nodes takes about 45 us where the
+// general form took 80, and the initial population of 1500 statement programs
+// (up to 256 attempts a member) 5.9 ms instead of 10.0.
+__device__ inline bool derive_w(const PhaseView& g, const WaveGrammar& w, int root_expression, int scope_count, int depth, int capacity,
+                                std::uint64_t seed, int* origins, Val* constants, int* sites, int logical_depth, GenResult& r) {
+  r = GenResult{ST_INVALID, 0, 0, 0};
+  if (root_expression < 0 || root_expression >= g.n_expr || scope_count < 0 || scope_count > 15 || depth <= 0 ||
+      depth >= g.depth_count || depth > 64 || logical_depth < 0 || logical_depth >= g.logical_count || capacity <= 0 ||
+      capacity > kPhaseCapacity)
+    return true;
+  const int lane = wlane();
+  constexpr int kRunning = -1, kOther = -2;
+  int status = kRunning, count = 0, nodes = 0, n_constants = 0, steps = 0;
+  unsigned reserved = g_minimum(g, root_expression, depth, logical_depth);
+  if (reserved > unsigned(capacity)) { r.status = ST_CAPACITY; return true; }
+  // The current task, and the pending ones: e | scope count << 8 | logical
+  // depth << 16, and depth | reserved cost << 16.
+  int e = root_expression, d = depth, sc = scope_count, l = logical_depth;
+  unsigned required = reserved;
+  unsigned ta = 0, tb = 0;
+  int next_site = -1, node_origin = 0, node_site = -1;
+  WaveDraws draws(seed);
+  const int spend = g.site_depth ? 1 : 0;
+  while (status == kRunning) {
+    if (++steps > 8192) {
+      status = ST_CAPACITY;
+    } else {
+      // `required` is part of `reserved` (it was added when the task was pushed).
+      reserved -= required;
+      const unsigned x = unsigned(rdlane(int(w.expr), e));
+      const int kind = int(x & 7u), arity = int((x >> 3) & 15u), target = int(std::int16_t(x >> 16));
+      if (kind == PK_REFERENCE) {
+        const int scopes = int((x >> 7) & 15u);
+        const unsigned nt = target >= 0 && target < g.n_nt ? unsigned(rdlane(int(w.nt), target)) : 0u;
+        const int offset = int(nt & 255u), productions = int((nt >> 8) & 255u);
+        if (productions == 0 || int((nt >> 16) & 255u) != scopes || scopes > 8 || offset + productions > g.n_prod ||
+            (sites && next_site >= 0)) {
+          status = ST_INVALID;
+        } else if ((spend && l == 0) || reserved > unsigned(capacity - nodes)) {
+          status = ST_CAPACITY;
+        } else {
+          next_site = site_pack(e, sc);
+          const int nl = l - spend;
+          const unsigned available = unsigned(capacity - nodes) - reserved;
+          // Lane offset + i holds production i. Weights of productions that do
+          // not fit count as zero, which leaves every in-order sum as it is.
+          const bool in = lane >= offset && lane < offset + productions;
+          const unsigned cost = in ? g_minimum(g, w.prod, d, nl) : 0xffffffffu;
+          const bool eligible = in && cost <= available;
+          double weight = eligible ? w.weight : 0.0;
+          bool positive = true;
+          if (!(nt >> 24 & 1u)) {
+            double most = 0;
+            for (int k = 0; k < productions; ++k) {
+              const double o = rdlane_d(weight, offset + k);
+              most = o > most ? o : most;
+            }
+            positive = most > 0;
+            weight = positive ? weight / most : 0.0;
+          }
+          double total = 0;
+          for (int k = 0; k < productions; ++k) total += rdlane_d(weight, offset + k);
+          const std::uint64_t mask = __ballot(eligible);
+          if (!positive) {
+            status = ST_CAPACITY;
+          } else {
+            double left = draws.unit() * total;
+            // Lane offset + j holds the choice less productions 0..j.
+            for (int k = 0; k < productions; ++k) {
+              const double o = rdlane_d(weight, offset + k);
+              left -= lane >= offset + k ? o : 0.0;
+            }
+            const std::uint64_t under = __ballot(eligible && left < 0);
+            if (mask == 0) {
+              status = ST_INVALID;
+            } else {
+              const int chosen = under ? wave_first(under) : 63 - __clzll((long long)mask);
+              e = rdlane(w.prod, chosen);
+              required = unsigned(rdlane(int(cost), chosen));
+              reserved += required;
+              sc = scopes;
+              l = nl;
+            }
+          }
+        }
+      } else {
+        bool well = kind == PK_OPERATION || kind == PK_INPUT || (kind == PK_BOUND && (x >> 11 & 1u)) ||
+                    (kind == PK_CONSTANT && target >= 0 && target < g.n_dom && arity == 0);
+        well = well && arity <= kMaxArity;
+        if (d <= 0 || nodes >= capacity) {
+          status = kind == PK_ALIAS ? ST_INVALID : ST_CAPACITY;
+        } else if (!well) {
+          status = ST_INVALID;
+        } else {
+          if (kind == PK_CONSTANT) {
+            const PDomain dom = g.dom[target];
+            Val v{};
+            const std::uint64_t width = std::uint64_t(dom.maximum) - std::uint64_t(dom.minimum) + 1;
+            const bool range = dom.integer_range != 0;
+            if (range ? dom.minimum > dom.maximum
+                      : dom.value_offset < 0 || dom.value_count <= 0 || dom.value_offset > g.n_values ||
+                            dom.value_count > g.n_values - dom.value_offset) {
+              status = ST_INVALID;
+            } else {
+              // bounded(n) takes a draw of at least 2^64 mod n, and any draw
+              // of at least n is. The general derivation has the rest.
+              const std::uint64_t n = range ? width : std::uint64_t(dom.value_count), draw = draws.take();
+              if (n == 0 || n >= (1u << 20) || draw < n) {
+                status = kOther;
+              } else {
+                const int k = int(__builtin_amdgcn_readfirstlane(int(mod_small(draw, unsigned(n)))));
+                if (range) v = val_int(wrap_add(dom.minimum, k));
+                else v = g.values[dom.value_offset + k];
+              }
+            }
+            if (status == kRunning && (v.tag == TAG_INVALID || v.tag == TAG_FALLBACK)) status = ST_INVALID;
+            if (status == kRunning) constants[n_constants++] = v;
+          }
+          if (status == kRunning) {
+            const int at = nodes & 63;
+            node_origin = lane == at ? e : node_origin;
+            node_site = lane == at ? next_site : node_site;
+            next_site = -1;
+            ++nodes;
+            if (at == 63) {
+              origins[nodes - 64 + lane] = node_origin;
+              if (sites) sites[nodes - 64 + lane] = node_site;
+            }
+            if (count + arity > 64) {
+              status = kOther;
+            } else if (arity > 0) {
+              // Child arity - 1 goes deepest: lane count + j takes child arity - 1 - j.
+              const int k = count + arity - 1 - lane;
+              const bool mine = k >= 0 && k < arity;
+              const unsigned w01 = unsigned(rdlane(int(w.c01), e)), w23 = unsigned(rdlane(int(w.c23), e));
+              const unsigned w45 = unsigned(rdlane(int(w.c45), e)), w67 = unsigned(rdlane(int(w.c67), e));
+              const unsigned scopes = unsigned(rdlane(int(w.scopes), e));
+              const unsigned pair = k < 4 ? (k < 2 ? w01 : w23) : (k < 6 ? w45 : w67);
+              const int child = int((pair >> (16 * (k & 1))) & 0xffffu);
+              const unsigned own = (scopes >> ((4 * k) & 31)) & 15u;
+              const unsigned need = mine ? g_minimum(g, child, d - 1, l) : 0u;
+              const unsigned room = unsigned(capacity - nodes);
+              unsigned sum = reserved;
+              for (int j = 0; j < arity; ++j) {
+                const unsigned n = unsigned(rdlane(int(need), count + j));
+                sum += n < 4096u ? n : 4096u;
+              }
+              if (sum > room) {
+                status = ST_CAPACITY;
+              } else {
+                ta = mine ? unsigned(child) | (own ? own - 1 : unsigned(sc)) << 8 | unsigned(l) << 16 : ta;
+                tb = mine ? unsigned(d - 1) | need << 16 : tb;
+                reserved = sum;
+                count += arity;
+              }
+            }
+            if (status == kRunning) {
+              if (count == 0) {
+                status = reserved ? ST_INVALID : ST_OK;
+              } else {
+                --count;
+                const unsigned a = unsigned(rdlane(int(ta), count)), b = unsigned(rdlane(int(tb), count));
+                e = int(a & 255u);
+                sc = int((a >> 8) & 255u);
+                l = int(a >> 16);
+                d = int(b & 0xffffu);
+                required = b >> 16;
+              }
+            }
+          }
+        }
+      }
+    }
+  }
+  if (status == kOther) return false;
+  if (nodes & 63) {
+    const int base = nodes & ~63, k = nodes & 63;
+    if (lane < k) {
+      origins[base + lane] = node_origin;
+      if (sites) sites[base + lane] = node_site;
+    }
+  }
+  r = GenResult{status, nodes, n_constants, steps};
+  return true;
+}
+// The derivation of a wavefront: in lane registers where the grammar and its
+// pending stack fit, else the general one. The row is stored across the
+// lanes: readers of other lanes' nodes fence first.
+__device__ inline GenResult derive_phase_w(const PhaseView& g, int root_expression, int scope_count, int depth, int capacity,
+                                           std::uint64_t seed, int* origins, Val* constants, int* sites, int logical_depth) {
+  GenResult r{ST_INVALID, 0, 0, 0};
+  WaveGrammar w;
+  if (wave_grammar(g, w) && derive_w(g, w, root_expression, scope_count, depth, capacity, seed, origins, constants, sites, logical_depth, r))
+    return r;
+  WaveTasks pending;
+  return generate_phase_with(g, root_expression, scope_count, depth, capacity, seed, origins, constants, sites, logical_depth, pending);
 }
 
 // Open nodes of the definite-assignment check: frame k in lane k.
@@ -578,11 +879,9 @@ __device__ inline void mutate_w(const PhaseView& g, const SlotInfo& s, int child
   const bool capped = pol.mutation_max_nodes > 0 && pol.mutation_max_nodes < uncapped;
   const int bounded = capped ? pol.mutation_max_nodes : uncapped;
   if (bounded > s.row_capacity) { st.error = 10; return; }  // node budget exceeds the physical row
-  WaveTasks pending;
-  // Every lane runs the derivation and stores the same values, so each lane
-  // reads back its own stores below.
-  const GenResult gen = generate_phase_with(g, site_entry(site), site_parent_scope(site), s.max_depth - depth + 1, bounded,
-                                            random.next(), tmp.origin, tmp.cval, tmp.site, logical, pending);
+  const GenResult gen = derive_phase_w(g, site_entry(site), site_parent_scope(site), s.max_depth - depth + 1, bounded, random.next(),
+                                       tmp.origin, tmp.cval, tmp.site, logical);
+  wave_fence();  // the subtree is read across the lanes below
   if (capped && gen.status == ST_CAPACITY) return;
   if (gen.status != ST_OK) { st.error = 7; return; }
   const CRow sub{tmp.origin, tmp.site, tmp.cval, gen.nodes, gen.constants};
