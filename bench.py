@@ -84,7 +84,8 @@ def profile(warm, steps):
 
 # The engine's timer names and the kernel symbols rocprofv3 records.
 PROFILED_NAME = {"k_vary": "k_vary<true, false>", "k_vary_global": "k_vary<false, false>",
-                 "k_vary_walks": "k_vary<true, true>", "k_vary_global_walks": "k_vary<false, true>",
+                 "k_vary_deferred": "k_vary<true, true>", "k_vary_global_deferred": "k_vary<false, true>",
+                 "k_lower": "k_lower<false>", "k_lower_walks": "k_lower<true>",
                  "k_eval": "k_eval<1>", "k_eval_general": "k_eval<0>", "k_place": "k_place<true>",
                  "k_place_hbm": "k_place<false>"}
 

@@ -30,7 +30,7 @@
 
 #include "engine.hpp"
 #include "population.hpp"
-#include "phase_wave.hpp"
+#include "vary_wave.hpp"
 #include "vm.hpp"
 
 namespace gagp_amd {
@@ -96,7 +96,7 @@ struct DSearch {
   GAS double* fitness;
   GAS unsigned *wrong, *nodes;
   GAS OpStats* stats;
-  GAS int* reuse;
+  GAS int* reuse;    // the member whose result the child takes, -1, or -2 until k_lower has lowered the child
   GAS double* c_fit;
   GAS unsigned *c_wrong, *c_nodes;
   GAS Ins* code;
@@ -131,6 +131,7 @@ struct DSearch {
   GAS int* elite;            // elite members of the current generation, best first
   int temp_slots;      // hidden-local slots per lane of the general VM (temporaries, grammar locals, input shadows)
   int input_shadow;    // the last input_shadow of them shadow stored inputs (statement input targets), else 0
+  int defer;           // programs may leave the straight-line VM: k_lower lowers what lower_row does not
   int walks;           // the grammar has traversals: lowering runs the kWalks instantiations
   int imported;        // the initial population is uploaded, not generated
   // Selection values of a caller-driven round (the owner seam): tournaments
@@ -206,14 +207,11 @@ __global__ __launch_bounds__(64 * kVaryWaves) void k_init_pop(DSearch* all, cons
 }
 
 // ---- lowering: one wavefront per row ----
-// kWalks: the lowering instantiation with traversals (grammars that have them).
-// Returns the code flags it stores (code_jumps).
-template <bool kWalks>
-__device__ __attribute__((always_inline)) inline int lower_into_w(const PhaseView& g, const DSearch& d, const CRow& row, int slot, WalkStore<kWalks>& ws) {
-  Ins* code = d.code + std::size_t(slot) * d.code_cap;
-  Val* pool = d.pool + std::size_t(slot) * d.pool_cap;
-  const LowerResult r =
-      lower_phase_w<kWalks>(g, row, d.local_types, d.n_locals, d.expected_type, code, d.code_cap, pool, d.pool_cap, ws);
+// Records the lowering `r` of a slot and decodes a looping program's steps;
+// returns the code flags it stores (code_jumps).
+__device__ __attribute__((always_inline)) inline int store_lowered(const DSearch& d, int slot, const LowerResult& r) {
+  const Ins* code = d.code + std::size_t(slot) * d.code_cap;
+  const Val* pool = d.pool + std::size_t(slot) * d.pool_cap;
   const bool ok = r.status == ST_OK && r.stack_bound >= 1 && r.stack_bound <= d.stack_slots &&
                   r.locals - d.n_locals <= d.temp_slots - d.input_shadow;
   // bit 0: jumps; bit 1: typed straight-line (vm_fast); bit 2: Bool result; bit 3: typed looping (vm_steps)
@@ -232,14 +230,40 @@ __device__ __attribute__((always_inline)) inline int lower_into_w(const PhaseVie
   }
   return flags;
 }
+// The node-by-node lowering of `row`, in memory, into `slot` (`source`: its
+// origins and constants, read into registers as they are needed). kWalks: the
+// instantiation with traversals (grammars that have them).
+template <bool kWalks>
+__device__ __attribute__((always_inline)) inline LowerResult lower_into_w(const PhaseView& g, const DSearch& d, const CRow& row, int slot,
+                                                                          WaveOrigins& source, WalkStore<kWalks>& ws) {
+  return lower_phase_w<kWalks>(g, row, d.local_types, d.n_locals, d.expected_type, d.code + std::size_t(slot) * d.code_cap, d.code_cap,
+                               d.pool + std::size_t(slot) * d.pool_cap, d.pool_cap, source, ws);
+}
 template <bool kWalks>
 __global__ __launch_bounds__(64 * kVaryWaves) void k_lower_members(DSearch* all, const BlockMap* map) {
   const BlockMap bm = map[blockIdx.x];
   const DSearch& d = all[bm.search];
   const int m = bm.block * kVaryWaves + wave_index();
   if (!d.active || (d.walks != 0) != kWalks || m >= d.P || *d.error) return;
+  __shared__ int row_lds[kVaryWaves][kWaveRow];
   __shared__ WalkStore<kWalks> walk_lds[kVaryWaves];
-  lower_into_w<kWalks>(view_of(d.g), d, member_row(d, m), m, walk_lds[wave_index()]);
+  const PhaseView g = view_of(d.g);
+  const CRow row = member_row(d, m);
+  LowerResult lowered;
+  WaveGrammar w;
+  bool done = false;
+  if (d.R <= kWaveRow && wave_grammar(g, w)) {
+    const std::size_t o = std::size_t(m) * d.R;
+    const WaveRow r = load_row(d.cur_origin + o, d.cur_site + o, d.cur_cval + o, d.R, row.n, row.nc);
+    done = (!d.slot.statement || locals_defined_row(g, w, r)) &&
+           lower_row<true>(w, r, d.local_types, d.n_locals, d.expected_type, d.code + std::size_t(m) * d.code_cap, d.code_cap,
+                           d.pool + std::size_t(m) * d.pool_cap, d.pool_cap, (LAS int*)row_lds[wave_index()], lowered);
+  }
+  if (!done) {
+    WaveOrigins source{row};
+    lowered = lower_into_w<kWalks>(g, d, row, m, source, walk_lds[wave_index()]);
+  }
+  store_lowered(d, m, lowered);
 }
 
 // ---- member hash table (parent_fitness_cache.cuh:11-58) ----
@@ -297,6 +321,22 @@ __device__ inline int find_member_w(const DSearch& d, const CRow& child, std::ui
   }
   return -1;
 }
+// find_member_w for a row in registers.
+__device__ inline int find_member_row(const DSearch& d, const WaveRow& child, std::uint64_t h) {
+  const std::uint64_t key = h | 1;
+  for (int probe = 0; probe <= d.table_mask; ++probe) {
+    const int slot = int((h + std::uint64_t(probe)) & std::uint64_t(d.table_mask));
+    const std::uint64_t k = d.table_key[slot];
+    if (k == 0) return -1;
+    if (k != key) continue;
+    const int m = __builtin_amdgcn_readfirstlane(d.table[slot]);
+    const std::size_t o = std::size_t(m) * d.R;
+    const std::uint64_t hash = d.member_hash[m];
+    const WaveRow member = load_row(d.cur_origin + o, d.cur_site + o, d.cur_cval + o, d.R, d.cur_n[m], d.cur_nc[m]);
+    return hash == h && same_rows(child, member) ? m : -1;
+  }
+  return -1;
+}
 // The evaluation kernel that scores a program: 1 the typed straight-line
 // path, 2 the typed looping path (both with an LDS score buffer, so only
 // where the cases fit it), 0 the general VM.
@@ -308,16 +348,28 @@ __device__ inline int eval_class(int code_flags, int C) {
 // straight-line ones from its back, the looping ones in [B, 2B).
 __device__ inline int pending_at(int B, int kind, int i) { return kind == 0 ? i : kind == 1 ? B - 1 - i : B + i; }
 
+// Puts a lowered child on its pending list.
+__device__ inline void pend_child(const DSearch& d, int c, int flags) {
+  if (wlane() != 0) return;
+  d.reuse[c] = -1;
+  const int k = eval_class(flags, d.cd.C);
+  d.pending[pending_at(d.B, k, atomicAdd(d.n_pending + k, 1))] = c;
+}
+
 // ---- reproduction: one wavefront per child (phase_operators.cuh:156-265) ----
 // kStaged: the block first copies the phase tables into LDS (searches whose
 // tables fit); otherwise the operators read them from global memory.
-// At most 64 vector registers, so eight wavefronts per SIMD: a population of
-// 8192 is resident at once.
-template <bool kStaged, bool kWalks>
-__global__ __launch_bounds__(64 * kVaryWaves) __attribute__((amdgpu_num_vgpr(64))) void k_vary(DSearch* all, const BlockMap* map) {
+// kDefer: rows that lower_row does not lower are left to k_lower (searches
+// whose programs may jump; those that may not have straight-line code, which
+// the small lowering here covers). The node-by-node lowering of a traversal is
+// 75-100 us of dependent steps, and its registers in this kernel cost one more
+// wavefront per SIMD: 8192 children of a list grammar took 352 us with it, and
+// take 164 plus 8 for the launch that finds nothing to lower.
+template <bool kStaged, bool kDefer>
+__global__ __launch_bounds__(64 * kVaryWaves) void k_vary(DSearch* all, const BlockMap* map) {
   const BlockMap bm = map[blockIdx.x];
   const DSearch& d = all[bm.search];
-  if (!search_live(d) || (d.stage_tables != 0) != kStaged || (d.walks != 0) != kWalks) return;  // uniform per block
+  if (!search_live(d) || (d.stage_tables != 0) != kStaged || (d.defer != 0) != kDefer) return;  // uniform per block
   extern __shared__ __attribute__((aligned(16))) unsigned char vary_lds[];
   const PhaseView g = kStaged ? stage_phase_tables<64 * kVaryWaves>(d.g, vary_lds) : view_of(d.g);
   const int c = bm.block * kVaryWaves + wave_index();
@@ -326,26 +378,59 @@ __global__ __launch_bounds__(64 * kVaryWaves) __attribute__((amdgpu_num_vgpr(64)
   const Keys keys = d.select ? Keys{d.select, nullptr, nullptr, 0} : Keys{d.fitness, d.wrong, d.nodes, d.has_wrong};
   const std::size_t o = std::size_t(c) * d.R;
   Row x{d.x_origin + o, d.x_site + o, d.x_cval + o, 0, 0};
+  Row tmp{d.t_origin + o, d.t_site + o, d.t_cval + o, 0, 0};
   OpStats st;
-  if (d.generational && c < d.elites) {
-    // Elite rows replace the first children after variation; a child's
-    // draws depend only on (seed, child), so the elite children skip theirs.
-    // An elite child is its source member and reuses its result.
-    const int src = d.elite[c];
-    copy_row_w(member_row(d, src), x);
-    st = OpStats{src, 0, 0, 0, 0, 0, 0, src, -1};
-    wave_fence();
+  // Elite rows replace the first children after variation; a child's draws
+  // depend only on (seed, child), so the elite children skip theirs. An elite
+  // child is its source member and reuses its result.
+  const int elite = d.generational && c < d.elites ? d.elite[c] : -1;
+  __shared__ int row_lds[kVaryWaves][kWaveRow];
+  LAS int* const hist = (LAS int*)row_lds[wave_index()];
+  WaveGrammar w;
+  // Rows of one node per lane stay in registers (vary_wave.hpp); wider rows
+  // and grammars are varied in memory.
+  const bool in_lanes = d.R <= kWaveRow && wave_grammar(g, w);
+  WaveRow child_row;
+  std::uint64_t h = 0;
+  if (in_lanes) {
+    const auto member = [&](int m) {
+      const std::size_t at = std::size_t(m) * d.R;
+      return load_row(d.cur_origin + at, d.cur_site + at, d.cur_cval + at, d.R, d.cur_n[m], d.cur_nc[m]);
+    };
+    if (elite >= 0) {
+      st = OpStats{elite, 0, 0, 0, 0, 0, 0, elite, -1};
+      child_row = member(elite);
+    } else {
+      st = OpStats{-1, 0, 0, 0, 0, 0, 0, -1, -1};
+      WaveDraws draws(seed ^ (0x617089e168ULL + std::uint64_t(c)));
+      tournament_rows(keys, d.P, d.pressure, draws, st.parent, st.donor);
+      const WaveRow parent = member(st.parent), donor = member(st.donor);
+      child_row = parent;
+      if (parent.n <= 0) st.error = 1;
+      else cross_rows(g, w, d.slot, parent, donor, child_row, draws, d.pol, hist, st);
+      mutate_row(g, w, d.slot, child_row, tmp, d.p_mut, seed ^ (0x124ab512bf01ULL + std::uint64_t(c)), d.pol, hist, st);
+      if (!st.error) compare_rows(parent, child_row, d.P, st);
+    }
+    if (!st.error) h = row_hash_row(child_row);
+    store_row(child_row, d.x_origin + o, d.x_site + o, d.x_cval + o);
+    x.n = child_row.n;
+    x.nc = child_row.nc;
   } else {
-    crossover_w(g, d.slot, c, [&](int m) { return member_row(d, m); }, x, keys, d.P, d.pressure, seed, d.pol, st);
-    wave_fence();
-    Row tmp{d.t_origin + o, d.t_site + o, d.t_cval + o, 0, 0};
-    Row spl{d.s_origin + o, d.s_site + o, d.s_cval + o, 0, 0};
-    mutate_w(g, d.slot, c, x, tmp, spl, d.p_mut, seed, d.pol, st);
-    wave_fence();
-    if (!st.error) compare_w(member_row(d, st.parent), as_const(x), d.P, st);
+    if (elite >= 0) {
+      copy_row_w(member_row(d, elite), x);
+      st = OpStats{elite, 0, 0, 0, 0, 0, 0, elite, -1};
+      wave_fence();
+    } else {
+      crossover_w(g, d.slot, c, [&](int m) { return member_row(d, m); }, x, keys, d.P, d.pressure, seed, d.pol, st);
+      wave_fence();
+      Row spl{d.s_origin + o, d.s_site + o, d.s_cval + o, 0, 0};
+      mutate_w(g, d.slot, c, x, tmp, spl, d.p_mut, seed, d.pol, st);
+      wave_fence();
+      if (!st.error) compare_w(member_row(d, st.parent), as_const(x), d.P, st);
+    }
+    if (!st.error) h = row_hash_w(as_const(x));
   }
   const CRow child = as_const(x);
-  const std::uint64_t h = st.error ? 0 : row_hash_w(child);
   if (wlane() == 0) {
     d.x_n[c] = x.n;
     d.x_nc[c] = x.nc;
@@ -357,7 +442,7 @@ __global__ __launch_bounds__(64 * kVaryWaves) __attribute__((amdgpu_num_vgpr(64)
   // A child identical to its parent, or to any member, takes that member's
   // completed result and is neither lowered nor evaluated. Results are
   // fixed before any placement of the round.
-  const int r = st.reusable_parent >= 0 ? st.reusable_parent : find_member_w(d, child, h);
+  const int r = st.reusable_parent >= 0 ? st.reusable_parent : in_lanes ? find_member_row(d, child_row, h) : find_member_w(d, child, h);
   if (r >= 0) {
     if (wlane() == 0) {
       d.code_len[c] = 0;
@@ -369,23 +454,61 @@ __global__ __launch_bounds__(64 * kVaryWaves) __attribute__((amdgpu_num_vgpr(64)
     }
     return;
   }
-  __shared__ WalkStore<kWalks> walk_lds[kVaryWaves];
-  const int flags = lower_into_w<kWalks>(g, d, child, c, walk_lds[wave_index()]);
   unsigned n;
-  if (d.grammar_sites) {
+  if (!d.grammar_sites) {
+    n = unsigned(d.fixed_nodes) + unsigned(child.n);
+  } else if (in_lanes) {
+    n = unsigned(__popcll(__ballot(child_row.site >= 0)));
+  } else {
     unsigned mine = 0;
     for (int i = wlane(); i < child.n; i += 64) mine += child.site[i] >= 0;
     for (int off = 32; off > 0; off >>= 1) mine += __shfl_xor(mine, off, 64);
     n = mine;
-  } else {
-    n = unsigned(d.fixed_nodes) + unsigned(child.n);
   }
-  if (wlane() == 0) {
-    d.reuse[c] = -1;
-    d.c_nodes[c] = n;
-    const int k = eval_class(flags, d.cd.C);
-    d.pending[pending_at(d.B, k, atomicAdd(d.n_pending + k, 1))] = c;
+  if (wlane() == 0) d.c_nodes[c] = n;
+  LowerResult lowered;
+  const bool done = in_lanes && lower_row<kDefer>(w, child_row, d.local_types, d.n_locals, d.expected_type, d.code + std::size_t(c) * d.code_cap,
+                                          d.code_cap, d.pool + std::size_t(c) * d.pool_cap, d.pool_cap, hist, lowered);
+  if (kDefer && !done) {
+    if (wlane() == 0) d.reuse[c] = -2;
+    return;
   }
+  if (!done) {
+    WaveOrigins source{child};
+    if (in_lanes) {
+      source.tile = source.constants = 0;
+      source.tile_origin = child_row.origin;
+      source.c0 = child_row.c0;
+      source.c1 = child_row.c1;
+      source.ct = child_row.ct;
+    }
+    WalkStore<false> ws;
+    lowered = lower_into_w<false>(g, d, child, c, source, ws);
+  }
+  pend_child(d, c, store_lowered(d, c, lowered));
+}
+// Lowers the children k_vary left, a wavefront each. The grammar's nodes are
+// held in lanes where they fit, else its tables are staged.
+template <bool kWalks>
+__global__ __launch_bounds__(64 * kVaryWaves) void k_lower(DSearch* all, const BlockMap* map) {
+  const BlockMap bm = map[blockIdx.x];
+  const DSearch& d = all[bm.search];
+  if (!search_live(d) || !d.defer || (d.walks != 0) != kWalks) return;  // uniform per block
+  extern __shared__ __attribute__((aligned(16))) unsigned char vary_lds[];
+  const PhaseView tables = view_of(d.g);
+  WaveGrammar w;
+  const bool packed = wave_grammar(tables, w);
+  const PhaseView g = packed || !d.stage_tables ? tables : stage_phase_tables<64 * kVaryWaves>(d.g, vary_lds);
+  const int c = bm.block * kVaryWaves + wave_index();
+  if (c >= d.B || __builtin_amdgcn_readfirstlane(d.reuse[c]) != -2) return;
+  __shared__ WalkStore<kWalks> walk_lds[kVaryWaves];
+  const CRow row = child_row(d, c);
+  WaveOrigins source{row};
+  source.packed = packed;
+  source.node = w.node;
+  source.node2 = w.node2;
+  const int flags = store_lowered(d, c, lower_into_w<kWalks>(g, d, row, c, source, walk_lds[wave_index()]));
+  pend_child(d, c, flags);
 }
 
 // ---- evaluation: one wavefront per program ----
@@ -2074,7 +2197,7 @@ struct Batch::Impl {
   // Flat grids: every search contributes exactly its own blocks.
   struct Grid { GAS BlockMap* map = nullptr; int blocks = 0; };
   DeviceArena map_arena;
-  Grid g_init, g_lower, g_eval_init, g_vary_staged, g_vary_global, g_vary_staged_w, g_vary_global_w, g_table, g_member,
+  Grid g_init, g_lower, g_eval_init, g_vary_staged, g_vary_global, g_vary_staged_d, g_vary_global_d, g_lower_c, g_lower_w, g_table, g_member,
       g_eval, g_eval_tiles, g_eval_general, g_eval_loop, g_finish, g_member_w;
   // Evaluation launch shapes of the round (the autotuner's choice, or the
   // fixed default: one program per wavefront, one 64-case tile per item).
@@ -2111,15 +2234,22 @@ struct Batch::Impl {
   static int up(int x, int k) { return (x + k - 1) / k; }
   void build_round_grids() {
     map_arena.release();
-    const auto vary = [&](bool staged, bool walks) {
+    const auto vary = [&](bool staged, bool defer) {
       return build_grid(map_arena, live, [&](const SearchState& s) {
-        return (s.d.stage_tables != 0) == staged && (s.d.walks != 0) == walks ? up(s.B, kVaryWaves) : 0;
+        return (s.d.stage_tables != 0) == staged && (s.d.defer != 0) == defer ? up(s.B, kVaryWaves) : 0;
+      });
+    };
+    const auto lower = [&](bool walks) {
+      return build_grid(map_arena, live, [&](const SearchState& s) {
+        return s.d.defer && (s.d.walks != 0) == walks ? up(s.B, kVaryWaves) : 0;
       });
     };
     g_vary_staged = vary(true, false);
     g_vary_global = vary(false, false);
-    g_vary_staged_w = vary(true, true);
-    g_vary_global_w = vary(false, true);
+    g_vary_staged_d = vary(true, true);
+    g_vary_global_d = vary(false, true);
+    g_lower_c = lower(false);
+    g_lower_w = lower(true);
     g_table = build_grid(map_arena, live, [&](const SearchState& s) { return up(s.d.table_mask + 1, 256); });
     g_member = build_grid(map_arena, live, [&](const SearchState& s) { return up(s.P, 128); });
     // one wavefront per child / member
@@ -2161,6 +2291,7 @@ struct Batch::Impl {
     s.configured = true;
     s.allocate();
     s.d.profile = timer.on ? 1 : 0;
+    s.d.defer = s.may_jump;
     s.d.stage_tables = phase_tables_bytes(s.d.g) <= kStageLimit;
     const std::size_t stacks = std::size_t(kWavesPerBlock) * (s.d.stack_slots + s.d.temp_slots) * 64 * 10;
     const std::size_t score_buf = std::size_t(kWavesPerBlock) * 8 * s.d.cd.C;
@@ -2197,11 +2328,13 @@ struct Batch::Impl {
       max_table = std::max(max_table, x.d.table_mask + 1);
     }
     const auto attr = [](const void* k, std::size_t bytes) {
-      if (bytes > 65536) HIP_OK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)));
+      if (bytes > 48 * 1024) HIP_OK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)));
     };
     attr(reinterpret_cast<const void*>(&k_init_pop<true>), vary_lds_bytes);
     attr(reinterpret_cast<const void*>(&k_vary<true, false>), vary_lds_bytes);
     attr(reinterpret_cast<const void*>(&k_vary<true, true>), vary_lds_bytes);
+    attr(reinterpret_cast<const void*>(&k_lower<false>), vary_lds_bytes);
+    attr(reinterpret_cast<const void*>(&k_lower<true>), vary_lds_bytes);
     attr(reinterpret_cast<const void*>(&k_eval<0>), eval_general_lds);
     attr(reinterpret_cast<const void*>(&k_eval<1>), eval_fast_lds);
     attr(reinterpret_cast<const void*>(&k_eval_tiles), eval_tiles_lds);
@@ -2507,17 +2640,17 @@ struct Batch::Impl {
     if (any_generational && !seam)
       timer.time("k_gen_begin", stream, [&] { hipLaunchKernelGGL(k_gen_begin, dim3(n), dim3(256), 0, stream, d_all); });
     if (!seam) timer.time("k_record", stream, [&] { hipLaunchKernelGGL(k_record, dim3(n), dim3(256), 0, stream, d_all); });
-    // Three independent branches: the reproduction of searches without and
-    // with traversal walks (disjoint searches) and the genotype index of the
-    // current members (read by nothing reproduction writes); the pending
-    // lists need all three.
+    // Two independent branches: the searches whose programs may jump, with
+    // the lowering that leaves, and the others (disjoint searches).
     branches({[&](hipStream_t s) {
-                launch_on(s, "k_vary", g_vary_staged, k_vary<true, false>, 64 * kVaryWaves, vary_lds_bytes);
-                launch_on(s, "k_vary_global", g_vary_global, k_vary<false, false>, 64 * kVaryWaves, 0);
+                launch_on(s, "k_vary_deferred", g_vary_staged_d, k_vary<true, true>, 64 * kVaryWaves, vary_lds_bytes);
+                launch_on(s, "k_vary_global_deferred", g_vary_global_d, k_vary<false, true>, 64 * kVaryWaves, 0);
+                launch_on(s, "k_lower_walks", g_lower_w, k_lower<true>, 64 * kVaryWaves, vary_lds_bytes);
+                launch_on(s, "k_lower", g_lower_c, k_lower<false>, 64 * kVaryWaves, vary_lds_bytes);
               },
               [&](hipStream_t s) {
-                launch_on(s, "k_vary_walks", g_vary_staged_w, k_vary<true, true>, 64 * kVaryWaves, vary_lds_bytes);
-                launch_on(s, "k_vary_global_walks", g_vary_global_w, k_vary<false, true>, 64 * kVaryWaves, 0);
+                launch_on(s, "k_vary", g_vary_staged, k_vary<true, false>, 64 * kVaryWaves, vary_lds_bytes);
+                launch_on(s, "k_vary_global", g_vary_global, k_vary<false, false>, 64 * kVaryWaves, 0);
               }});
   }
   void enqueue_eval() {

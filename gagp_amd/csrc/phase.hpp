@@ -308,6 +308,13 @@ struct SlotInfo {
   int statement;     // the phase is a statement program: variation checks definite assignment
 };
 
+// Constant k of the row being lowered, and the node of an expression (a reader
+// that holds them elsewhere has its own overloads).
+template <class OriginAt>
+GHD inline Val constant_of(const OriginAt&, const CRow& t, int k) { return t.cval[k]; }
+template <class OriginAt>
+GHD inline const PNode& node_of(const OriginAt&, const PhaseView& g, int origin) { return g.expr[origin].node; }
+
 // Definite assignment of grammar locals (phase_compile.cuh:170-200): a local
 // is readable after an assign to it, inside a for_range body that names it,
 // and after an if_stmt only when both branches assigned it; a for_range
@@ -321,7 +328,7 @@ GHD inline bool locals_defined_with(const PhaseView& g, int n, OriginAt origin_a
   const auto bit = [](int operand) { return operand >= 0 && operand < 16 ? 1u << operand : 0u; };
   for (int i = 0; i < n; ++i) {
     const int o = origin_at(i);
-    const PNode& node = g.expr[o].node;
+    const PNode& node = node_of(origin_at, g, o);
     if (node.kind == TK_VAR && !(mask & bit(node.operand))) return false;
     if (node.arity > 0) {
       if (depth == 64) return false;
@@ -330,7 +337,7 @@ GHD inline bool locals_defined_with(const PhaseView& g, int n, OriginAt origin_a
     }
     while (depth) {
       DefFrame f = frames.get(depth - 1);
-      const PNode& owner = g.expr[f.origin].node;
+      const PNode& owner = node_of(origin_at, g, f.origin);
       ++f.seen;
       if (owner.kind == TK_FOR_RANGE && f.seen == 1) {
         f.saved = mask;
@@ -689,11 +696,10 @@ GHD inline LowerResult lower_phase_with(const PhaseView& g, const CRow& t, Origi
     if (!have_value) {
       if (cursor >= t.n) return out;
       const int o = origin_at(cursor++);
-      const PExpr& x = g.expr[o];
-      const PNode& node = x.node;
+      const PNode& node = node_of(origin_at, g, o);
       if (node.kind == TK_CONSTANT) {
         if (cconst >= t.nc) return out;
-        const Val& src = t.cval[cconst++];
+        const Val src = constant_of(origin_at, t, cconst++);
         Val v{};  // fields only: the padding never leaves the row
         v.i = src.i;
         v.b = src.b;
@@ -823,7 +829,7 @@ GHD inline LowerResult lower_phase_with(const PhaseView& g, const CRow& t, Origi
       return out;
     }
     Frame f = frames.get(depth - 1);
-    const PNode& node = g.expr[f.origin].node;
+    const PNode& node = node_of(origin_at, g, f.origin);
     // Constant indices keep the frame in registers.
     if (f.seen == 0) f.args[0] = std::uint8_t(completed);
     else if (f.seen == 1) f.args[1] = std::uint8_t(completed);

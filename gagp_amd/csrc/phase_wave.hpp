@@ -178,13 +178,27 @@ struct WaveGrammar {
   unsigned expr;                  // kind [2:0], arity [6:3], scope count [10:7], BOUND well formed [11], target [31:16]
   unsigned c01, c23, c45, c67;    // children, two per register
   unsigned scopes;                // 4 bits per child: its scope count + 1, 0 to inherit
-  unsigned nt;                    // production offset [7:0], count [15:8], scope count [23:16], normalized [24]
+  unsigned node, node2;           // tree kind [4:0], opcode [9:5], arity [13:10], operand [31:16]; type [7:0], fuel [15:8], merge fuel [23:16]
+  unsigned nt;                    // production offset [7:0], count [15:8], scope count [23:16], normalized [24], fixed sites [25]
   int prod;                       // the production's expression
   double weight;
 };
+// The node of expression `origin` (uniform).
+__device__ inline PNode unpack_node(unsigned node, unsigned node2, int origin) {
+  const unsigned a = unsigned(rdlane(int(node), origin)), b = unsigned(rdlane(int(node2), origin));
+  PNode n;
+  n.kind = int(a & 31u);
+  n.opcode = int((a >> 5) & 31u);
+  n.operand = int(a) >> 16;
+  n.arity = int((a >> 10) & 15u);
+  n.fuel = (b >> 8) & 255u;
+  n.merge_fuel = (b >> 16) & 255u;
+  n.type = int(b & 255u);
+  return n;
+}
 // Fills `w`; false when the grammar does not fit.
 __device__ inline bool wave_grammar(const PhaseView& g, WaveGrammar& w) {
-  w = WaveGrammar{0, 0, 0, 0, 0, 0, 0, -1, 0.0};
+  w = WaveGrammar{0, 0, 0, 0, 0, 0, 0, 0, 0, -1, 0.0};
   if (g.n_expr > 64 || g.n_nt > 64 || g.n_prod > 64 || g.n_dom > 64 || g.depth_count > 256 || g.logical_count > 256) return false;
   const int lane = wlane();
   bool bad = false;
@@ -202,13 +216,18 @@ __device__ inline bool wave_grammar(const PhaseView& g, WaveGrammar& w) {
       w.scopes |= unsigned((x.child_scope[k] + 1) & 15) << (4 * k);
       bad = bad || x.child_scope[k] > 14;
     }
+    const PNode& t = x.node;
+    w.node = unsigned(t.kind & 31) | unsigned(t.opcode & 31) << 5 | unsigned(t.arity & 15) << 10 | unsigned(t.operand & 0xffff) << 16;
+    w.node2 = unsigned(t.type & 255) | (t.fuel & 255u) << 8 | (t.merge_fuel & 255u) << 16;
+    bad = bad || t.kind < 0 || t.kind > 31 || t.opcode < 0 || t.opcode > 31 || t.operand < -0x8000 || t.operand > 0x7fff || t.type < 0 ||
+          t.type > 255 || t.fuel > 255 || t.merge_fuel > 255;
     bad = bad || x.kind < 0 || x.kind > 7 || x.node.arity < 0 || x.node.arity > kMaxArity || x.scope_count < 0 || x.scope_count > 15 ||
           x.target < -1 || x.target > 64;
   }
   if (lane < g.n_nt) {
     const PNt n = g.nt[lane];
     w.nt = unsigned(n.production_offset) | unsigned(n.production_count) << 8 | unsigned(n.scope_count & 255) << 16 |
-           unsigned(n.normalized != 0) << 24;
+           unsigned(n.normalized != 0) << 24 | unsigned(n.fixed != 0) << 25;
   }
   if (lane < g.n_prod) {
     const PProd p = g.prod[lane];
@@ -268,8 +287,9 @@ struct WaveDraws {
 // dozen scalar instructions: a subtree of 31 nodes takes about 45 us where the
 // general form took 80, and the initial population of 1500 statement programs
 // (up to 256 attempts a member) 5.9 ms instead of 10.0.
+template <class Sink>
 __device__ inline bool derive_w(const PhaseView& g, const WaveGrammar& w, int root_expression, int scope_count, int depth, int capacity,
-                                std::uint64_t seed, int* origins, Val* constants, int* sites, int logical_depth, GenResult& r) {
+                                std::uint64_t seed, Sink& sink, int logical_depth, GenResult& r) {
   r = GenResult{ST_INVALID, 0, 0, 0};
   if (root_expression < 0 || root_expression >= g.n_expr || scope_count < 0 || scope_count > 15 || depth <= 0 ||
       depth >= g.depth_count || depth > 64 || logical_depth < 0 || logical_depth >= g.logical_count || capacity <= 0 ||
@@ -285,7 +305,7 @@ __device__ inline bool derive_w(const PhaseView& g, const WaveGrammar& w, int ro
   int e = root_expression, d = depth, sc = scope_count, l = logical_depth;
   unsigned required = reserved;
   unsigned ta = 0, tb = 0;
-  int next_site = -1, node_origin = 0, node_site = -1;
+  int next_site = -1;
   WaveDraws draws(seed);
   const int spend = g.site_depth ? 1 : 0;
   while (status == kRunning) {
@@ -301,7 +321,7 @@ __device__ inline bool derive_w(const PhaseView& g, const WaveGrammar& w, int ro
         const unsigned nt = target >= 0 && target < g.n_nt ? unsigned(rdlane(int(w.nt), target)) : 0u;
         const int offset = int(nt & 255u), productions = int((nt >> 8) & 255u);
         if (productions == 0 || int((nt >> 16) & 255u) != scopes || scopes > 8 || offset + productions > g.n_prod ||
-            (sites && next_site >= 0)) {
+            next_site >= 0) {
           status = ST_INVALID;
         } else if ((spend && l == 0) || reserved > unsigned(capacity - nodes)) {
           status = ST_CAPACITY;
@@ -316,7 +336,7 @@ __device__ inline bool derive_w(const PhaseView& g, const WaveGrammar& w, int ro
           const bool eligible = in && cost <= available;
           double weight = eligible ? w.weight : 0.0;
           bool positive = true;
-          if (!(nt >> 24 & 1u)) {
+          if ((nt >> 24 & 1u) == 0) {
             double most = 0;
             for (int k = 0; k < productions; ++k) {
               const double o = rdlane_d(weight, offset + k);
@@ -381,18 +401,12 @@ __device__ inline bool derive_w(const PhaseView& g, const WaveGrammar& w, int ro
               }
             }
             if (status == kRunning && (v.tag == TAG_INVALID || v.tag == TAG_FALLBACK)) status = ST_INVALID;
-            if (status == kRunning) constants[n_constants++] = v;
+            if (status == kRunning) sink.constant(n_constants++, v);
           }
           if (status == kRunning) {
-            const int at = nodes & 63;
-            node_origin = lane == at ? e : node_origin;
-            node_site = lane == at ? next_site : node_site;
+            sink.node(nodes, e, next_site);
             next_site = -1;
             ++nodes;
-            if (at == 63) {
-              origins[nodes - 64 + lane] = node_origin;
-              if (sites) sites[nodes - 64 + lane] = node_site;
-            }
             if (count + arity > 64) {
               status = kOther;
             } else if (arity > 0) {
@@ -440,16 +454,29 @@ __device__ inline bool derive_w(const PhaseView& g, const WaveGrammar& w, int ro
     }
   }
   if (status == kOther) return false;
-  if (nodes & 63) {
-    const int base = nodes & ~63, k = nodes & 63;
-    if (lane < k) {
-      origins[base + lane] = node_origin;
-      if (sites) sites[base + lane] = node_site;
-    }
-  }
+  sink.finish(nodes);
   r = GenResult{status, nodes, n_constants, steps};
   return true;
 }
+// A derivation's row in memory: nodes collect one per lane and are stored 64
+// at a time, constants as they come.
+struct MemorySink {
+  int* origins;
+  Val* constants;
+  int* sites;
+  int origin = 0, site = -1;
+  __device__ void node(int k, int o, int s) {
+    const bool mine = wlane() == (k & 63);
+    origin = mine ? o : origin;
+    site = mine ? s : site;
+    if ((k & 63) == 63) put(k - 63, 64);
+  }
+  __device__ void constant(int k, const Val& v) { constants[k] = v; }
+  __device__ void finish(int n) { put(n & ~63, n & 63); }
+  __device__ void put(int base, int count) {
+    if (wlane() < count) { origins[base + wlane()] = origin; sites[base + wlane()] = site; }
+  }
+};
 // The derivation of a wavefront: in lane registers where the grammar and its
 // pending stack fit, else the general one. The row is stored across the
 // lanes: readers of other lanes' nodes fence first.
@@ -457,8 +484,8 @@ __device__ inline GenResult derive_phase_w(const PhaseView& g, int root_expressi
                                            std::uint64_t seed, int* origins, Val* constants, int* sites, int logical_depth) {
   GenResult r{ST_INVALID, 0, 0, 0};
   WaveGrammar w;
-  if (wave_grammar(g, w) && derive_w(g, w, root_expression, scope_count, depth, capacity, seed, origins, constants, sites, logical_depth, r))
-    return r;
+  MemorySink sink{origins, constants, sites};
+  if (wave_grammar(g, w) && derive_w(g, w, root_expression, scope_count, depth, capacity, seed, sink, logical_depth, r)) return r;
   WaveTasks pending;
   return generate_phase_with(g, root_expression, scope_count, depth, capacity, seed, origins, constants, sites, logical_depth, pending);
 }
@@ -759,6 +786,12 @@ __device__ inline GenResult splice_w(const PhaseView& g, const CRow& base, int d
 struct WaveOrigins {
   const CRow& t;
   int tile = -64, tile_origin = 0;
+  // The row's constants likewise, for the lowering: payload, tag | flag << 8.
+  int constants = -64;
+  unsigned c0 = 0, c1 = 0, ct = 0;
+  // The nodes of a grammar held in lanes (WaveGrammar), else in the tables.
+  bool packed = false;
+  unsigned node = 0, node2 = 0;
   __device__ int operator()(int i) {
     if (i - tile >= 64 || i < tile) {
       tile = i & ~63;
@@ -768,6 +801,28 @@ struct WaveOrigins {
     return rdlane(tile_origin, i - tile);
   }
 };
+__device__ inline PNode node_of(const WaveOrigins& r, const PhaseView& g, int origin) {
+  return r.packed ? unpack_node(r.node, r.node2, origin) : g.expr[origin].node;
+}
+__device__ inline Val constant_of(WaveOrigins& r, const CRow& t, int k) {
+  if (k - r.constants >= 64 || k < r.constants) {
+    r.constants = k & ~63;
+    const int mine = r.constants + wlane();
+    if (mine < t.nc) {
+      const std::uint64_t v = std::uint64_t(t.cval[mine].i);
+      r.c0 = unsigned(v);
+      r.c1 = unsigned(v >> 32);
+      r.ct = unsigned(t.cval[mine].tag) | unsigned(t.cval[mine].b) << 8;
+    }
+  }
+  const int at = k - r.constants;
+  const unsigned tag = unsigned(rdlane(int(r.ct), at));
+  Val v{};
+  v.i = std::int64_t(std::uint64_t(unsigned(rdlane(int(r.c1), at))) << 32 | unsigned(rdlane(int(r.c0), at)));
+  v.tag = std::uint8_t(tag);
+  v.b = std::uint8_t(tag >> 8);
+  return v;
+}
 // locals_defined by the whole wavefront (phase_operators.cuh:148-154).
 __device__ inline bool locals_defined_w(const PhaseView& g, const CRow& t) {
   wave_fence();
@@ -928,9 +983,8 @@ __device__ inline std::uint64_t row_hash_w(const CRow& r) {
 template <bool kWalks = false>
 __device__ inline LowerResult lower_phase_w(const PhaseView& g, const CRow& t, const std::uint8_t* local_types, int local_count,
                                             int expected_type, Ins* code, int code_capacity, Val* pool, int pool_capacity,
-                                            WalkStore<kWalks>& ws) {
+                                            WaveOrigins& origin_at, WalkStore<kWalks>& ws) {
   WaveFrames frames;
-  WaveOrigins origin_at{t};
   return lower_phase_with<WaveFrames, WaveOrigins&, kWalks>(g, t, origin_at, local_types, local_count, expected_type, code,
                                                             code_capacity, pool, pool_capacity, frames, ws);
 }
