@@ -1230,21 +1230,44 @@ __global__ void k_status(DSearch* all, int n, int* out) {
 
 // ---- placement (evolve.cpp:378-422) ----
 // The reference draws victims one group of `replacement_size` words at a
-// time. Here one wavefront examines up to W consecutive groups at once
-// against the keys as they stand at the start of the chunk, then commits the
-// longest prefix of groups whose outcome cannot differ from the sequential
-// order. A chunk ends before the first group that drew a member replaced by
-// an earlier group of the chunk, after the first group whose child becomes
-// the new best (the redraw test and the best tracking change there), and
-// after the group that places the last child. Group 0 is always committed.
-constexpr int kRing = 1024;        // tempered generator words, a power of two
-constexpr int kPlaceWords = 512;   // words examined per chunk at most
+// time: the worst member drawn takes the next child, unless it is the best.
+// Here a thread takes one of up to 1024 consecutive groups, and the chunk's
+// victims are found as the fixpoint of the sequential rule: given everyone's
+// victim, a group compares the members it drew with the keys they hold by its
+// turn (the child of the last earlier group that took the member, else the
+// member's own). A group depends on earlier ones alone, so every pass settles
+// at least the first unsettled group, and an unchanged pass is the sequential
+// outcome; most groups share no member with an earlier one, and a chunk takes
+// as many passes as its longest chain of such groups. The chunk ends after the
+// first group whose child becomes the best (the test against the best and its
+// tracking change there) and after the first that places nothing (the children
+// shift by one).
+// Bound by the passes' chain of LDS reads and barriers in one block a search.
+// One wavefront taking the longest prefix of 64 groups without a shared member
+// needed a chunk of 1.1 us for every 30 to 60 groups. us a round before and
+// after: 47 and 22 for 1024 groups of two draws among 1024 members, 111 and 47
+// for 4096, 194 and 85 for 8192; 512 threads take 22, 54 and 100. Of the 47,
+// 10 are 26 twists of the generator, 5 the launch and 30 four or five chunks
+// of three to four passes. Twisting between the passes' barriers instead took
+// 52: the last wavefronts then keep the block waiting.
+constexpr int kRing = 4096;          // tempered generator words, a power of two
+constexpr int kLeftWords = 1024;     // unconsumed words kept between rounds (at most 311)
+constexpr int kPlaceThreads = 1024;  // groups per chunk at most
+constexpr int kPlaceBuckets = 2048;  // lists of groups by victim, a power of two
+static_assert(kPlaceThreads <= 1024, "a bucket holds a group in 10 bits");
+// Dynamic LDS of a placement block: the generator's ring and two states, the
+// chunk's child keys (a packed order has 4 bytes in LDS, 8 otherwise), the
+// victim lists, then with keys in LDS 12 bytes per member.
+constexpr std::size_t place_bytes(bool lds, int members) {
+  return 8 * std::size_t(kRing) + 16 * 312 + (lds ? 12 : 16) * std::size_t(kPlaceThreads) + 4 * std::size_t(kPlaceBuckets) +
+         4 * std::size_t(kPlaceThreads) + (lds ? 12 * std::size_t(members) : 0);
+}
 
 template <bool kLds>
 struct PlaceKeys {
   // kLds: fitness and (wrong << 12 | nodes) staged in LDS; otherwise the
-  // member arrays in HBM, read past the L1 so every lane sees the stores of
-  // the previous chunk. Fields are copied out of the search state so that
+  // member arrays in HBM, read past the L1 so every wavefront sees the stores
+  // of the previous chunk. Fields are copied out of the search state so that
   // stores to the keys never force it to be re-read.
   GAS double* fitness;
   GAS unsigned* wrong;
@@ -1259,20 +1282,15 @@ struct PlaceKeys {
     return __longlong_as_double((long long)bits);
   }
   __device__ std::uint64_t order(int m) const {
+    if (!has_wrong) return 0;
     if (kLds) return wn[m];
     const unsigned w = __hip_atomic_load(wrong + m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const unsigned n = __hip_atomic_load(nodes + m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return std::uint64_t(w) << 32 | n;
   }
-  __device__ std::uint64_t pack(unsigned w, unsigned n) const { return kLds ? std::uint64_t(w << 12 | n) : std::uint64_t(w) << 32 | n; }
-  // `better` (fitness desc, wrong asc, nodes asc, index asc) of a key against member b.
-  __device__ bool key_better(double fa, std::uint64_t oa, int a, int b) const {
-    const double fb = fit(b);
-    if (fa != fb) return fa > fb;
-    if (has_wrong) { const std::uint64_t ob = order(b); if (oa != ob) return oa < ob; }
-    return a < b;
+  __device__ std::uint64_t pack(unsigned w, unsigned n) const {
+    return !has_wrong ? 0 : kLds ? std::uint64_t(w << 12 | n) : std::uint64_t(w) << 32 | n;
   }
-  __device__ bool better(int a, int b) const { return key_better(fit(a), has_wrong ? order(a) : 0, a, b); }
   __device__ void store(int m, double fv, unsigned w, unsigned n) const {
     if (kLds) { f[m] = fv; wn[m] = w << 12 | n; }
     fitness[m] = fv;
@@ -1280,208 +1298,215 @@ struct PlaceKeys {
     nodes[m] = n;
   }
 };
+// `better` (fitness desc, wrong asc, nodes asc, index asc) of two keys.
+__device__ inline bool key_better(double fa, std::uint64_t oa, int a, double fb, std::uint64_t ob, int b) {
+  if (fa != fb) return fa > fb;
+  if (oa != ob) return oa < ob;
+  return a < b;
+}
 
-// The block's four wavefronts stage the keys and refill the generator ring
-// together; wavefront 0 alone runs the chunks (their LDS ordering needs only
-// workgroup fences, not barriers). Children's keys are prefetched into two
-// 64-child register windows one window ahead of use.
-constexpr int kPlaceThreads = 256;
 template <bool kLds>
 __global__ __launch_bounds__(kPlaceThreads) void k_place(DSearch* all) {
   const DSearch& d = all[blockIdx.x];
   if (!search_live(d) || d.generational || d.place_lds != int(kLds)) return;
   extern __shared__ __attribute__((aligned(16))) unsigned char place_smem[];
-  __shared__ std::uint64_t ring[kRing];
-  __shared__ unsigned ridx[kRing];
+  std::uint64_t* const ring = reinterpret_cast<std::uint64_t*>(place_smem);
   // Generator state, double-buffered: a twist reads one buffer and writes
   // the other (`cur` is the buffer holding the current state).
-  __shared__ std::uint64_t mt[2][312];
-  __shared__ int s_head, s_b, s_best;
+  std::uint64_t* const mt = ring + kRing;
+  double* const child_f = reinterpret_cast<double*>(mt + 2 * 312);
+  using Order = std::conditional_t<kLds, unsigned, std::uint64_t>;
+  Order* const child_o = reinterpret_cast<Order*>(child_f + kPlaceThreads);
+  // bucket: pass << 10 | last group entered; link: victim << 11 | (next group + 1).
+  unsigned* const bucket = reinterpret_cast<unsigned*>(child_o + kPlaceThreads);
+  unsigned* const link = bucket + kPlaceBuckets;
+  double* const member_f = reinterpret_cast<double*>(link + kPlaceThreads);
+  __shared__ int s_cut, s_best, s_kept, s_moved[3];
+  __shared__ double s_best_f;
+  __shared__ std::uint64_t s_best_o;
   const int t = threadIdx.x, lane = t & 63;
-  const bool leader = wave_index() == 0;
   const int P = d.P, B = d.B, rs = d.replacement_size, has_wrong = d.has_wrong;
   const std::uint64_t P64 = std::uint64_t(P);
   GAS const double* const c_fit = d.c_fit;
   GAS const unsigned* const c_wrong = d.c_wrong;
   GAS const unsigned* const c_nodes = d.c_nodes;
   GAS int* const placed = d.placed;
-  PlaceKeys<kLds> keys{d.fitness, d.wrong, d.nodes, has_wrong, reinterpret_cast<double*>(place_smem),
-                       reinterpret_cast<unsigned*>(place_smem + (kLds ? 8 * std::size_t(P) : 0))};
-  unsigned* mark = reinterpret_cast<unsigned*>(place_smem + (kLds ? 12 * std::size_t(P) : 0));
+  const PlaceKeys<kLds> keys{d.fitness, d.wrong, d.nodes, has_wrong, member_f, reinterpret_cast<unsigned*>(member_f + (kLds ? P : 0))};
   // x mod P by a Barrett step: q = mulhi(x, floor((2^64-1)/P)) is
   // floor(x/P) or one less, so one conditional subtraction is exact.
   const std::uint64_t barrett = ~0ull / P64;
   const auto mod_p = [&](std::uint64_t x) {
     std::uint64_t r = x - __umul64hi(x, barrett) * P64;
-    return unsigned(r >= P64 ? r - P64 : r);
+    return int(r >= P64 ? r - P64 : r);
   };
-  constexpr int kStage = 8;  // loads in flight per thread while staging keys
-  for (int m0 = 0; m0 < P; m0 += kPlaceThreads * kStage) {
-    double f[kStage];
-    unsigned w[kStage], n[kStage];
+  // Child keys of this thread's group, loaded a chunk ahead.
+  double cf = 0;
+  unsigned cw = 0, cn = 0;
+  const auto fetch = [&](int c) {
+    if (c < B) { cf = c_fit[c]; cw = c_wrong[c]; cn = c_nodes[c]; }
+  };
+  fetch(t);
+  if (kLds) {
+    constexpr int kStage = 8;  // loads in flight per thread while staging keys
+    for (int m0 = 0; m0 < P; m0 += kPlaceThreads * kStage) {
+      double f[kStage];
+      unsigned w[kStage], n[kStage];
 #pragma unroll
-    for (int k = 0; k < kStage; ++k) {
-      const int m = m0 + k * kPlaceThreads + t;
-      if (kLds && m < P) { f[k] = keys.fitness[m]; w[k] = keys.wrong[m]; n[k] = keys.nodes[m]; }
-    }
+      for (int k = 0; k < kStage; ++k) {
+        const int m = m0 + k * kPlaceThreads + t;
+        if (m < P) { f[k] = keys.fitness[m]; w[k] = keys.wrong[m]; n[k] = keys.nodes[m]; }
+      }
 #pragma unroll
-    for (int k = 0; k < kStage; ++k) {
-      const int m = m0 + k * kPlaceThreads + t;
-      if (m < P) {
-        if (kLds) { keys.f[m] = f[k]; keys.wn[m] = has_wrong ? w[k] << 12 | n[k] : 0u; }
-        mark[m] = 0;
+      for (int k = 0; k < kStage; ++k) {
+        const int m = m0 + k * kPlaceThreads + t;
+        if (m < P) { keys.f[m] = f[k]; keys.wn[m] = w[k] << 12 | n[k]; }
       }
     }
   }
+  for (int i = t; i < kPlaceBuckets; i += kPlaceThreads) bucket[i] = 0;
+  if (t < 3) s_moved[t] = 0;
   int cur = 0;
-  for (int i = t; i < 312; i += kPlaceThreads) mt[0][i] = d.mt[i];
+  for (int i = t; i < 312; i += kPlaceThreads) mt[i] = d.mt[i];
   int head = 0, tail = *d.n_left;
-  for (int i = t; i < tail; i += kPlaceThreads) {
-    const std::uint64_t x = d.mt_left[i];
-    ring[i] = x;
-    ridx[i] = mod_p(x);
-  }
+  for (int i = t; i < tail; i += kPlaceThreads) ring[i] = d.mt_left[i];
   __syncthreads();
   // Every thread, uniformly: the next state into the other buffer and its
   // 312 tempered words at the ring's tail. Words 0..155 read only the old
   // state; 156..310 read the new word i-156, and 311 the new words 0 and 155.
   const auto twist = [&] {
-    const int nxt = cur ^ 1;
+    const std::uint64_t* const old = mt + 312 * cur;
+    std::uint64_t* const now = mt + 312 * (cur ^ 1);
     const auto put = [&](int i, std::uint64_t w) {
-      mt[nxt][i] = w;
-      const std::uint64_t x = mt_temper(w);
-      ring[(tail + i) & (kRing - 1)] = x;
-      ridx[(tail + i) & (kRing - 1)] = mod_p(x);
+      now[i] = w;
+      ring[(tail + i) & (kRing - 1)] = mt_temper(w);
     };
-    for (int i = t; i < 156; i += kPlaceThreads) put(i, mt_next_word(mt[cur][i], mt[cur][i + 1], mt[cur][i + 156]));
+    if (t < 156) put(t, mt_next_word(old[t], old[t + 1], old[t + 156]));
     __syncthreads();
-    for (int i = 156 + t; i < 312; i += kPlaceThreads)
-      put(i, mt_next_word(mt[cur][i], i == 311 ? mt[nxt][0] : mt[cur][i + 1], mt[nxt][i - 156]));
+    if (t < 156) put(t + 156, mt_next_word(old[t + 156], t == 155 ? now[0] : old[t + 157], now[t]));
     __syncthreads();
-    cur = nxt;
+    cur ^= 1;
     tail += 312;
   };
-  const auto refill = [&](int need) {
-    while (tail - head < need) twist();
-  };
-  const int W = rs < kPlaceWords / 64 ? 64 : kPlaceWords / rs;
-  const std::uint64_t below = (1ull << lane) - 1;
+  const int W = min(kPlaceThreads, (kRing - 312) / rs);
   int b = 0, best = *d.best;
   double best_f = keys.fit(best);
-  std::uint64_t best_o = has_wrong ? keys.order(best) : 0;
-  unsigned chunk = 0;
-  const unsigned chunk_limit = 4u * unsigned(B) + 4096u;
-  // Child-key windows [win, win+64) and [win+64, win+128), lane l holding child win+l.
-  int win = 0;
-  double f0 = 0, f1 = 0;
-  unsigned w0 = 0, n0 = 0, w1 = 0, n1 = 0;
-  if (leader) {
-    if (lane < B) { f0 = c_fit[lane]; w0 = c_wrong[lane]; n0 = c_nodes[lane]; }
-    if (64 + lane < B) { f1 = c_fit[64 + lane]; w1 = c_wrong[64 + lane]; n1 = c_nodes[64 + lane]; }
-  }
+  std::uint64_t best_o = keys.order(best);
+  unsigned pass = 0;
+  int chunk = 0;
+  const int chunk_limit = 4 * B + 4096;
   while (b < B) {
-    // The ring is filled with whole twists (at least kRing - 311 unconsumed
-    // words, above one chunk's W * rs <= kPlaceWords), and the leader runs
-    // chunks until fewer words than a chunk's are left, so the block meets
-    // at a barrier once per fill rather than once per chunk.
-    while (tail - head + 312 <= kRing) twist();
-    bool stop = false;
-    while (leader && !stop && b < B && tail - head >= W * rs) {
-      stop = ++chunk > chunk_limit;
-      if (stop && lane == 0) raise(d, 500);
-      while (!stop && b >= win + 64) {  // slide the windows
-        f0 = f1; w0 = w1; n0 = n1;
-        win += 64;
-        const int next = win + 64 + lane;
-        f1 = 0; w1 = 0; n1 = 0;
-        if (next < B) { f1 = c_fit[next]; w1 = c_wrong[next]; n1 = c_nodes[next]; }
+    if (++chunk > chunk_limit) {
+      if (t == 0) raise(d, 500);
+      break;
+    }
+    const int n = min(W, B - b);
+    while (tail - head < n * rs) twist();
+    const bool active = t < n;
+    const int base = head + t * rs;
+    const std::uint64_t co = keys.pack(cw, cn);
+    child_f[t] = cf;
+    child_o[t] = Order(co);
+    if (t == 0) s_cut = n;
+    // The first draws and their members' keys stay in registers (named ones:
+    // a dynamically indexed array would spill).
+    int m0 = 0, m1 = 0, m2 = 0;
+    double f0 = 0, f1 = 0, f2 = 0;
+    std::uint64_t o0 = 0, o1 = 0, o2 = 0;
+    const auto drawn = [&](int k) { return mod_p(ring[(base + k) & (kRing - 1)]); };
+    if (active) {
+      m0 = drawn(0);
+      f0 = keys.fit(m0);
+      o0 = keys.order(m0);
+      if (rs > 1) { m1 = drawn(1); f1 = keys.fit(m1); o1 = keys.order(m1); }
+      if (rs > 2) { m2 = drawn(2); f2 = keys.fit(m2); o2 = keys.order(m2); }
+    }
+    // The worst member drawn; `settled` reads the lists of the last pass.
+    const auto pick = [&](bool settled) {
+      int worst = -1;
+      double wf = 0;
+      std::uint64_t wo = 0;
+      const auto consider = [&](int m, double f, std::uint64_t o) {
+        if (settled) {
+          const unsigned first = bucket[m & (kPlaceBuckets - 1)];
+          int found = -1;
+          if (first >> 10 == pass)
+            for (int j = int(first & 1023u); j >= 0;) {
+              const unsigned l = link[j];
+              if (int(l >> 11) == m && j < t && j > found) found = j;
+              j = int(l & 2047u) - 1;
+            }
+          if (found >= 0) { f = child_f[found]; o = child_o[found]; }
+        }
+        if (worst < 0 || key_better(wf, wo, worst, f, o, m)) { worst = m; wf = f; wo = o; }
+      };
+      consider(m0, f0, o0);
+      if (rs > 1) consider(m1, f1, o1);
+      if (rs > 2) consider(m2, f2, o2);
+      for (int k = 3; k < rs; ++k) {
+        const int m = drawn(k);
+        consider(m, keys.fit(m), keys.order(m));
       }
-      if (!stop) {
-        const bool active = lane < W;
-        const int base = head + lane * rs;
-        int worst = -1;
-        // The first four draws stay in registers for the conflict test
-        // (named registers: a dynamically indexed array would spill).
-        int d0 = 0, d1 = 0, d2 = 0, d3 = 0;
-        if (active) {
-          worst = int(ridx[base & (kRing - 1)]);
-          d0 = worst;
-          for (int i = 1; i < rs; ++i) {
-            const int c = int(ridx[(base + i) & (kRing - 1)]);
-            d1 = i == 1 ? c : d1;
-            d2 = i == 2 ? c : d2;
-            d3 = i == 3 ? c : d3;
-            if (keys.better(worst, c)) worst = c;
-          }
-        }
-        const bool place = active && worst != best;
-        const std::uint64_t pmask = __ballot(place);
-        const int rank = __popcll(pmask & below);
-        const int child = b + rank;
-        const bool fills = place && child < B;
-        const int k = child - win;  // 0 <= k < 128
-        // Both windows are read by every lane before the select: a shuffle
-        // under a divergent branch reads 0 from the lanes that branch masks off.
-        const double a0 = __shfl(f0, k & 63, 64), a1 = __shfl(f1, k & 63, 64);
-        const int b0 = __shfl(int(w0), k & 63, 64), b1 = __shfl(int(w1), k & 63, 64);
-        const int c0 = __shfl(int(n0), k & 63, 64), c1 = __shfl(int(n1), k & 63, 64);
-        const double cf = k < 64 ? a0 : a1;
-        const unsigned cw = unsigned(k < 64 ? b0 : b1);
-        const unsigned cn = unsigned(k < 64 ? c0 : c1);
-        if (place) atomicMax(&mark[worst], chunk * 64u + unsigned(63 - lane));
-        // LDS operations of one wavefront complete in issue order, so the
-        // mark reads below see every lane's maximum without a wait between
-        // them; keys in HBM need the fence.
-        if constexpr (!kLds) __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-        __builtin_amdgcn_wave_barrier();
-        bool conflict = false;
-        if (active)
-          for (int i = 0; i < rs; ++i) {
-            const int drawn = i == 0 ? d0 : i == 1 ? d1 : i == 2 ? d2 : i == 3 ? d3 : int(ridx[(base + i) & (kRing - 1)]);
-            const unsigned m = mark[drawn];
-            conflict = conflict || ((m >> 6) == chunk && int(63u - (m & 63u)) < lane);
-          }
-        // `better` of the child (at the victim's index) against the best
-        // member, whose keys stay in registers: the best is never a victim,
-        // so they change only when a child becomes the best.
-        const std::uint64_t co = keys.pack(cw, cn);
-        const bool raises = fills && (cf != best_f ? cf > best_f : has_wrong && co != best_o ? co < best_o : worst < best);
-        int cut = W;
-        const std::uint64_t last = __ballot(fills && child == B - 1);
-        if (last) cut = min(cut, __ffsll((long long)last));
-        const std::uint64_t clash = __ballot(active && conflict);
-        if (clash) cut = min(cut, __ffsll((long long)clash) - 1);
-        const std::uint64_t lifts = __ballot(raises);
-        const int lifter = lifts ? __ffsll((long long)lifts) - 1 : 64;
-        if (lifter < cut) cut = lifter + 1;
-        if (fills && lane < cut) {
-          keys.store(worst, cf, cw, cn);
-          placed[worst] = child;
-        }
-        if (lifter < cut) {
-          best = __shfl(worst, lifter, 64);
-          best_f = __shfl(cf, lifter, 64);
-          best_o = __shfl(co, lifter, 64);
-        }
-        b += __popcll(cut >= 64 ? pmask : pmask & ((1ull << cut) - 1));
-        head += cut * rs;
-        if constexpr (!kLds) __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-        __builtin_amdgcn_wave_barrier();
+      return worst;
+    };
+    int worst = active ? pick(false) : -1;
+    for (int settled = 0; settled <= n; ++settled) {
+      ++pass;
+      if (active) {
+        const unsigned old = atomicExch(&bucket[worst & (kPlaceBuckets - 1)], pass << 10 | unsigned(t));
+        link[t] = unsigned(worst) << 11 | (old >> 10 == pass ? (old & 1023u) + 1u : 0u);
+      }
+      __syncthreads();
+      const int now = active ? pick(true) : -1;
+      const std::uint64_t moved = __ballot(now != worst);
+      worst = now;
+      // Three flags in turn: the next is cleared two barriers before its use.
+      if (moved && lane == 0) s_moved[pass % 3] = 1;
+      if (t == 0) s_moved[(pass + 1) % 3] = 0;
+      __syncthreads();
+      if (!s_moved[pass % 3]) break;
+    }
+    // `better` of the child (at the victim's index) against the best member,
+    // which is no victim before the chunk's end.
+    const bool place = active && worst != best;
+    const bool raises = place && key_better(cf, co, worst, best_f, best_o, best);
+    const std::uint64_t ends = __ballot(active && (!place || raises));
+    if (ends && lane == 0) atomicMin(&s_cut, (t & ~63) + wave_first(ends) + 1);
+    __syncthreads();
+    const int cut = s_cut;
+    if (place && t < cut) {
+      // The last group of the chunk that took the member leaves its child there.
+      bool last = true;
+      for (int j = int(bucket[worst & (kPlaceBuckets - 1)] & 1023u); j >= 0;) {
+        const unsigned l = link[j];
+        last = last && !(int(l >> 11) == worst && j > t && j < cut);
+        j = int(l & 2047u) - 1;
+      }
+      if (last) {
+        keys.store(worst, cf, cw, cn);
+        placed[worst] = b + t;
       }
     }
-    if (leader && lane == 0) { s_head = head; s_b = stop ? B : b; s_best = best; }
+    if (t == cut - 1) {
+      s_kept = place ? cut : cut - 1;
+      s_best = raises ? worst : best;
+      s_best_f = raises ? cf : best_f;
+      s_best_o = raises ? co : best_o;
+    }
+    if (!kLds) __threadfence();
     __syncthreads();
-    head = s_head;
-    b = s_b;
+    b += s_kept;
     best = s_best;
-    __syncthreads();
+    best_f = s_best_f;
+    best_o = s_best_o;
+    head += cut * rs;
+    fetch(b + t);
   }
-  refill(1);
+  while (tail - head < 1) twist();
   const std::uint64_t next_seed = ring[head & (kRing - 1)];
   ++head;
   const int left = tail - head;
-  for (int i = t; i < left; i += kPlaceThreads) d.mt_left[i] = ring[(head + i) & (kRing - 1)];
-  for (int i = t; i < 312; i += kPlaceThreads) d.mt[i] = mt[cur][i];
+  for (int i = t; i < left && i < kLeftWords; i += kPlaceThreads) d.mt_left[i] = ring[(head + i) & (kRing - 1)];
+  for (int i = t; i < 312; i += kPlaceThreads) d.mt[i] = mt[312 * cur + i];
   if (t == 0) {
     *d.n_left = left;
     *d.round_seed = next_seed;
@@ -2053,10 +2078,10 @@ struct SearchState {
     x.pending = a.alloc<int>(2 * std::size_t(B)); x.n_pending = a.alloc<int>(3);
     const int tsize = next_pow2(2 * P);
     x.table_key = a.alloc<std::uint64_t>(tsize); x.table = a.alloc<int>(tsize); x.table_mask = tsize - 1;
-    x.mt = a.alloc<std::uint64_t>(312); x.mt_left = a.alloc<std::uint64_t>(kRing); x.n_left = a.alloc<int>(1);
+    x.mt = a.alloc<std::uint64_t>(312); x.mt_left = a.alloc<std::uint64_t>(kLeftWords); x.n_left = a.alloc<int>(1);
     x.round_seed = a.alloc<std::uint64_t>(1);
     x.member_hash = a.alloc<std::uint64_t>(P);
-    // Placement keys (fitness, wrong << 12 | nodes) and victim marks in LDS.
+    // Placement keys (fitness, wrong << 12 | nodes) in LDS.
     x.place_lds = P <= 8192 && train.n < (1 << 20) && int(layout.fixed_nodes) + R < 4096;
     x.round = a.alloc<int>(1); x.best = a.alloc<int>(1); x.placed = a.alloc<int>(P);
     x.hist_origin = a.alloc<int>(std::size_t(G) * R); x.hist_cval = a.alloc<Val>(std::size_t(G) * R);
@@ -2319,8 +2344,8 @@ struct Batch::Impl {
       if (x.d.typed_tiles) eval_tiles_lds = std::max(eval_tiles_lds, std::size_t(8) * x.d.cd.C);
       if (x.d.stage_tables) vary_lds_bytes = std::max(vary_lds_bytes, phase_tables_bytes(x.d.g));
       else vary_global = true;
-      if (x.d.place_lds) place_lds_bytes = std::max(place_lds_bytes, std::size_t(16) * x.P);
-      else place_hbm_bytes = std::max(place_hbm_bytes, std::size_t(4) * x.P);
+      if (x.d.place_lds) place_lds_bytes = std::max(place_lds_bytes, place_bytes(true, x.P));
+      else place_hbm_bytes = place_bytes(false, x.P);
       any_generational = any_generational || x.d.generational;
       max_P = std::max(max_P, x.P);
       max_B = std::max(max_B, x.B);
