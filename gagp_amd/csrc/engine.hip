@@ -207,10 +207,12 @@ __global__ __launch_bounds__(64 * kVaryWaves) void k_init_pop(DSearch* all, cons
 }
 
 // ---- lowering: one wavefront per row ----
-// Records the lowering `r` of a slot and decodes a looping program's steps;
-// returns the code flags it stores (code_jumps).
-__device__ __attribute__((always_inline)) inline int store_lowered(const DSearch& d, int slot, const LowerResult& r) {
-  const Ins* code = d.code + std::size_t(slot) * d.code_cap;
+// Records the lowering `r` of a slot and decodes a looping program's steps,
+// from `code` and `values` where the caller has them at hand; returns the code
+// flags it stores (code_jumps).
+__device__ __attribute__((always_inline)) inline int store_lowered(const DSearch& d, int slot, const LowerResult& r,
+                                                                   const Ins* code = nullptr, const std::int64_t* values = nullptr) {
+  if (!code) code = d.code + std::size_t(slot) * d.code_cap;
   const Val* pool = d.pool + std::size_t(slot) * d.pool_cap;
   const bool ok = r.status == ST_OK && r.stack_bound >= 1 && r.stack_bound <= d.stack_slots &&
                   r.locals - d.n_locals <= d.temp_slots - d.input_shadow;
@@ -218,8 +220,8 @@ __device__ __attribute__((always_inline)) inline int store_lowered(const DSearch
   const int flags = r.jumps | (r.fast ? 2 : 0) | (r.result_type == TAG_BOOL ? 4 : 0) | (r.loop ? 8 : 0);
   int steps = 0;
   if (ok && r.loop && d.steps) {
-    wave_fence();  // the code and pool stored above are read across the lanes
-    steps = decode_steps_w(code, r.code, pool, d.n_locals, d.steps + std::size_t(slot) * d.step_cap);
+    if (!values) wave_fence();  // the code and pool stored above are read across the lanes
+    steps = decode_steps_w(code, r.code, pool, values, d.n_locals, d.steps + std::size_t(slot) * d.step_cap);
   }
   if (wlane() == 0) {
     if (!ok) raise(d, 200 + r.status);
@@ -245,8 +247,9 @@ __global__ __launch_bounds__(64 * kVaryWaves) void k_lower_members(DSearch* all,
   const DSearch& d = all[bm.search];
   const int m = bm.block * kVaryWaves + wave_index();
   if (!d.active || (d.walks != 0) != kWalks || m >= d.P || *d.error) return;
-  __shared__ int row_lds[kVaryWaves][kWaveRow];
+  __shared__ LaneStore<true> row_lds[kVaryWaves];
   __shared__ WalkStore<kWalks> walk_lds[kVaryWaves];
+  LaneStore<true>& store = row_lds[wave_index()];
   const PhaseView g = view_of(d.g);
   const CRow row = member_row(d, m);
   LowerResult lowered;
@@ -257,13 +260,14 @@ __global__ __launch_bounds__(64 * kVaryWaves) void k_lower_members(DSearch* all,
     const WaveRow r = load_row(d.cur_origin + o, d.cur_site + o, d.cur_cval + o, d.R, row.n, row.nc);
     done = (!d.slot.statement || locals_defined_row(g, w, r)) &&
            lower_row<true>(w, r, d.local_types, d.n_locals, d.expected_type, d.code + std::size_t(m) * d.code_cap, d.code_cap,
-                           d.pool + std::size_t(m) * d.pool_cap, d.pool_cap, (LAS int*)row_lds[wave_index()], lowered);
+                           d.pool + std::size_t(m) * d.pool_cap, d.pool_cap, (LAS LaneStore<true>*)&store, lowered);
   }
   if (!done) {
     WaveOrigins source{row};
     lowered = lower_into_w<kWalks>(g, d, row, m, source, walk_lds[wave_index()]);
   }
-  store_lowered(d, m, lowered);
+  if (done) store_lowered(d, m, lowered, store.code, store.values);
+  else store_lowered(d, m, lowered);
 }
 
 // ---- member hash table (parent_fitness_cache.cuh:11-58) ----
@@ -364,9 +368,10 @@ __device__ inline void pend_child(const DSearch& d, int c, int flags) {
 // the small lowering here covers). The node-by-node lowering of a traversal is
 // 75-100 us of dependent steps, and its registers in this kernel cost one more
 // wavefront per SIMD: 8192 children of a list grammar took 352 us with it, and
-// take 164 plus 8 for the launch that finds nothing to lower.
+// take 158 plus 8 for the launch that finds nothing to lower. At most 80 vector
+// registers, so six wavefronts per SIMD and not five.
 template <bool kStaged, bool kDefer>
-__global__ __launch_bounds__(64 * kVaryWaves) void k_vary(DSearch* all, const BlockMap* map) {
+__global__ __launch_bounds__(64 * kVaryWaves) __attribute__((amdgpu_waves_per_eu(6))) void k_vary(DSearch* all, const BlockMap* map) {
   const BlockMap bm = map[blockIdx.x];
   const DSearch& d = all[bm.search];
   if (!search_live(d) || (d.stage_tables != 0) != kStaged || (d.defer != 0) != kDefer) return;  // uniform per block
@@ -384,8 +389,9 @@ __global__ __launch_bounds__(64 * kVaryWaves) void k_vary(DSearch* all, const Bl
   // depend only on (seed, child), so the elite children skip theirs. An elite
   // child is its source member and reuses its result.
   const int elite = d.generational && c < d.elites ? d.elite[c] : -1;
-  __shared__ int row_lds[kVaryWaves][kWaveRow];
-  LAS int* const hist = (LAS int*)row_lds[wave_index()];
+  __shared__ LaneStore<kDefer> row_lds[kVaryWaves];
+  LaneStore<kDefer>& store = row_lds[wave_index()];
+  LAS int* const hist = (LAS int*)store.sums;
   WaveGrammar w;
   // Rows of one node per lane stay in registers (vary_wave.hpp); wider rows
   // and grammars are varied in memory.
@@ -468,9 +474,10 @@ __global__ __launch_bounds__(64 * kVaryWaves) void k_vary(DSearch* all, const Bl
   if (wlane() == 0) d.c_nodes[c] = n;
   LowerResult lowered;
   const bool done = in_lanes && lower_row<kDefer>(w, child_row, d.local_types, d.n_locals, d.expected_type, d.code + std::size_t(c) * d.code_cap,
-                                          d.code_cap, d.pool + std::size_t(c) * d.pool_cap, d.pool_cap, hist, lowered);
-  if (kDefer && !done) {
-    if (wlane() == 0) d.reuse[c] = -2;
+                                          d.code_cap, d.pool + std::size_t(c) * d.pool_cap, d.pool_cap, (LAS LaneStore<kDefer>*)&store, lowered);
+  if constexpr (kDefer) {
+    if (done) pend_child(d, c, store_lowered(d, c, lowered, store.code, store.values));
+    else if (wlane() == 0) d.reuse[c] = -2;
     return;
   }
   if (!done) {

@@ -4,6 +4,8 @@
 #include "identity.hpp"
 
 #include <algorithm>
+#include <cmath>
+#include <cstring>
 #include <fstream>
 #include <functional>
 #include <map>
@@ -539,6 +541,38 @@ Grammar load_grammar_text(const std::string& text) {
 }
 Grammar load_grammar_file(const std::string& path) { return load_grammar_text(read_file(path)); }
 
+// The choice among all of a nonterminal's productions (choose_production_in_order)
+// as bounds: it subtracts the weights in order, each step rounded and so
+// monotone in the choice, until the choice is negative; `below` is the least
+// choice that is not, found by halving the doubles' bit patterns.
+void production_bounds(PProd* p, PNt& nt) {
+  double maximum = nt.normalized ? 1 : 0, total = 0;
+  if (!nt.normalized)
+    for (int i = 0; i < nt.production_count; ++i) maximum = std::max(maximum, p[i].weight);
+  if (!(maximum > 0) || !std::isfinite(maximum)) return;
+  const auto weight = [&](int i) { return nt.normalized ? p[i].weight : p[i].weight / maximum; };
+  for (int i = 0; i < nt.production_count; ++i) total += weight(i);
+  if (!std::isfinite(total)) return;
+  nt.total = total;
+  for (int i = 0; i < nt.production_count; ++i) {
+    const auto negative = [&](double choice) {
+      for (int k = 0; k <= i; ++k) choice -= weight(k);
+      return choice < 0;
+    };
+    const double top = 2 * total + 1;
+    std::uint64_t lo = 0, hi;  // negative below lo, not negative at hi
+    std::memcpy(&hi, &top, sizeof(hi));
+    while (lo < hi) {
+      const std::uint64_t middle = lo + (hi - lo) / 2;
+      double choice;
+      std::memcpy(&choice, &middle, sizeof(choice));
+      if (negative(choice)) lo = middle + 1;
+      else hi = middle;
+    }
+    std::memcpy(&p[i].below, &hi, sizeof(hi));
+  }
+}
+
 PhaseGrammar compile_phase(const Grammar& g, unsigned root, unsigned max_depth, unsigned site_depth,
                            const std::vector<std::string>& input_order) {
   const auto fail = [](const std::string& why) -> void { throw Unsupported("GPU phase construction: " + why); };
@@ -901,6 +935,7 @@ PhaseGrammar compile_phase(const Grammar& g, unsigned root, unsigned max_depth, 
     for (int i = 0; i < nt.production_count; ++i) out.prods[nt.production_offset + i].weight /= maximum;
     nt.normalized = 1;
   }
+  for (auto& nt : out.nts) production_bounds(out.prods.data() + nt.production_offset, nt);
   return out;
 }
 

@@ -133,8 +133,13 @@ struct PExpr {
   int scope_count = 0;
   signed char child_scope[kMaxArity] = {-1, -1, -1, -1, -1, -1, -1, -1};
 };
-struct PProd { int expression; double weight; };
-struct PNt { int production_offset = 0, production_count = 0, scope_count = 0, normalized = 0, fixed = 0; };
+// `below`: with every production of its nonterminal eligible, a choice of less
+// takes this one or an earlier one.
+struct PProd { int expression; double weight; double below = 0; };
+// `total`: the sum a choice is scaled by with every production eligible, 0 if none can be chosen.
+struct PNt { int production_offset = 0, production_count = 0, scope_count = 0, normalized = 0, fixed = 0; double total = 0; };
+// Sets `below` of a nonterminal's productions `p` and its `total`.
+void production_bounds(PProd* p, PNt& nt);
 struct PDomain { int value_offset = 0, value_count = 0, integer_range = 0; std::int64_t minimum = 0, maximum = 0; };
 
 struct PhaseGrammar {

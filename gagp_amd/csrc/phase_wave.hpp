@@ -181,7 +181,8 @@ struct WaveGrammar {
   unsigned node, node2;           // tree kind [4:0], opcode [9:5], arity [13:10], operand [31:16]; type [7:0], fuel [15:8], merge fuel [23:16]
   unsigned nt;                    // production offset [7:0], count [15:8], scope count [23:16], normalized [24], fixed sites [25]
   int prod;                       // the production's expression
-  double weight;
+  double weight, below;           // and its weight and bound
+  double total;                   // the nonterminal's
 };
 // The node of expression `origin` (uniform).
 __device__ inline PNode unpack_node(unsigned node, unsigned node2, int origin) {
@@ -198,7 +199,7 @@ __device__ inline PNode unpack_node(unsigned node, unsigned node2, int origin) {
 }
 // Fills `w`; false when the grammar does not fit.
 __device__ inline bool wave_grammar(const PhaseView& g, WaveGrammar& w) {
-  w = WaveGrammar{0, 0, 0, 0, 0, 0, 0, 0, 0, -1, 0.0};
+  w = WaveGrammar{0, 0, 0, 0, 0, 0, 0, 0, 0, -1, 0.0, 0.0, 0.0};
   if (g.n_expr > 64 || g.n_nt > 64 || g.n_prod > 64 || g.n_dom > 64 || g.depth_count > 256 || g.logical_count > 256) return false;
   const int lane = wlane();
   bool bad = false;
@@ -228,11 +229,13 @@ __device__ inline bool wave_grammar(const PhaseView& g, WaveGrammar& w) {
     const PNt n = g.nt[lane];
     w.nt = unsigned(n.production_offset) | unsigned(n.production_count) << 8 | unsigned(n.scope_count & 255) << 16 |
            unsigned(n.normalized != 0) << 24 | unsigned(n.fixed != 0) << 25;
+    w.total = n.total;
   }
   if (lane < g.n_prod) {
     const PProd p = g.prod[lane];
     w.prod = p.expression;
     w.weight = p.weight;
+    w.below = p.below;
   }
   return __ballot(bad) == 0;
 }
@@ -286,7 +289,8 @@ struct WaveDraws {
 // Bound by its chain of dependent steps, each one LDS round trip and a few
 // dozen scalar instructions: a subtree of 31 nodes takes about 45 us where the
 // general form took 80, and the initial population of 1500 statement programs
-// (up to 256 attempts a member) 5.9 ms instead of 10.0.
+// (up to 256 attempts a member) 5.3 ms instead of 10.0. Scanning the weights
+// instead of comparing with the bounds took 5.9.
 template <class Sink>
 __device__ inline bool derive_w(const PhaseView& g, const WaveGrammar& w, int root_expression, int scope_count, int depth, int capacity,
                                 std::uint64_t seed, Sink& sink, int logical_depth, GenResult& r) {
@@ -334,40 +338,49 @@ __device__ inline bool derive_w(const PhaseView& g, const WaveGrammar& w, int ro
           const bool in = lane >= offset && lane < offset + productions;
           const unsigned cost = in ? g_minimum(g, w.prod, d, nl) : 0xffffffffu;
           const bool eligible = in && cost <= available;
-          double weight = eligible ? w.weight : 0.0;
-          bool positive = true;
-          if ((nt >> 24 & 1u) == 0) {
-            double most = 0;
-            for (int k = 0; k < productions; ++k) {
-              const double o = rdlane_d(weight, offset + k);
-              most = o > most ? o : most;
-            }
-            positive = most > 0;
-            weight = positive ? weight / most : 0.0;
-          }
-          double total = 0;
-          for (int k = 0; k < productions; ++k) total += rdlane_d(weight, offset + k);
-          const std::uint64_t mask = __ballot(eligible);
-          if (!positive) {
-            status = ST_CAPACITY;
+          // Every production eligible, as away from the limits: the choice is
+          // one comparison a lane (production_bounds).
+          const double whole = rdlane_d(w.total, target);
+          int chosen = -1;
+          if (__ballot(in && !eligible) == 0 && whole > 0) {
+            const double choice = draws.unit() * whole;
+            const std::uint64_t under = __ballot(in && choice < w.below);
+            chosen = under ? wave_first(under) : offset + productions - 1;
           } else {
-            double left = draws.unit() * total;
-            // Lane offset + j holds the choice less productions 0..j.
-            for (int k = 0; k < productions; ++k) {
-              const double o = rdlane_d(weight, offset + k);
-              left -= lane >= offset + k ? o : 0.0;
+            double weight = eligible ? w.weight : 0.0;
+            bool positive = true;
+            if ((nt >> 24 & 1u) == 0) {
+              double most = 0;
+              for (int k = 0; k < productions; ++k) {
+                const double o = rdlane_d(weight, offset + k);
+                most = o > most ? o : most;
+              }
+              positive = most > 0;
+              weight = positive ? weight / most : 0.0;
             }
-            const std::uint64_t under = __ballot(eligible && left < 0);
-            if (mask == 0) {
-              status = ST_INVALID;
+            double total = 0;
+            for (int k = 0; k < productions; ++k) total += rdlane_d(weight, offset + k);
+            const std::uint64_t mask = __ballot(eligible);
+            if (!positive) {
+              status = ST_CAPACITY;
             } else {
-              const int chosen = under ? wave_first(under) : 63 - __clzll((long long)mask);
-              e = rdlane(w.prod, chosen);
-              required = unsigned(rdlane(int(cost), chosen));
-              reserved += required;
-              sc = scopes;
-              l = nl;
+              double left = draws.unit() * total;
+              // Lane offset + j holds the choice less productions 0..j.
+              for (int k = 0; k < productions; ++k) {
+                const double o = rdlane_d(weight, offset + k);
+                left -= lane >= offset + k ? o : 0.0;
+              }
+              const std::uint64_t under = __ballot(eligible && left < 0);
+              if (mask == 0) status = ST_INVALID;
+              else chosen = under ? wave_first(under) : 63 - __clzll((long long)mask);
             }
+          }
+          if (chosen >= 0) {
+            e = rdlane(w.prod, chosen);
+            required = unsigned(rdlane(int(cost), chosen));
+            reserved += required;
+            sc = scopes;
+            l = nl;
           }
         }
       } else {

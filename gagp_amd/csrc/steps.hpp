@@ -112,6 +112,7 @@ struct StepSource {
   const Ins* code;
   int len;
   const Val* pool;
+  const std::int64_t* values;  // the pool's payloads (a Bool's flag), where the caller has them, else null
   int n_inputs;
   bool tagged;
   CodeBits target;    // instructions some jump enters
@@ -216,6 +217,7 @@ STEP_FN Step step_at(const StepSource& s, int j, const CodeBits& starts, int n) 
   const auto element = [&](int k) { return unsigned(stack + (k < 0 ? 0 : k < kStepStack ? k : kStepStack - 1)); };
   const auto step_of = [&](int t) { return unsigned(t >= s.len ? n : starts.below(t)); };
   const auto constant = [&](const Ins& x) {
+    if (s.values) return s.values[x.a];
     const Val v = s.pool[x.a];
     return v.tag == TAG_BOOL ? std::int64_t(v.b != 0) : v.i;
   };
@@ -352,7 +354,7 @@ STEP_FN Step step_at(const StepSource& s, int j, const CodeBits& starts, int n) 
 // Host decoding of a certified looping program of at most kLoopCode
 // instructions; returns the number of steps written.
 inline int decode_steps(const Ins* code, int len, const Val* pool, int n_inputs, bool tagged, Step* out) {
-  StepSource s{code, len, pool, n_inputs, tagged, {{0, 0, 0, 0}}, {{0, 0, 0, 0}}};
+  StepSource s{code, len, pool, nullptr, n_inputs, tagged, {{0, 0, 0, 0}}, {{0, 0, 0, 0}}};
   for (int i = 0; i < len; ++i) {
     if (jump_op(code[i].op)) s.target.set(code[i].a, 1);
     if (tagged && !s.sequence.at(i) && sequence_length(code[i])) s.sequence.set(i, sequence_length(code[i]));
@@ -368,9 +370,10 @@ inline int decode_steps(const Ins* code, int len, const Val* pool, int n_inputs,
 
 #if defined(__HIPCC__)
 // The same by one wavefront, a lane per instruction.
-__device__ __attribute__((always_inline)) inline int decode_steps_w(const Ins* code, int len, const Val* pool, int n_inputs, Step* out) {
+__device__ __attribute__((always_inline)) inline int decode_steps_w(const Ins* code, int len, const Val* pool, const std::int64_t* values,
+                                                                        int n_inputs, Step* out) {
   const int lane = int(threadIdx.x & 63u);
-  StepSource s{code, len, pool, n_inputs, true, {{0, 0, 0, 0}}, {{0, 0, 0, 0}}};
+  StepSource s{code, len, pool, values, n_inputs, true, {{0, 0, 0, 0}}, {{0, 0, 0, 0}}};
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
     if (64 * g >= len) break;

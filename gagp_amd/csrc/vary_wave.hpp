@@ -14,15 +14,24 @@
 // about 78 global and 85 LDS loads a child, each a dependent round trip. Here
 // a child reads its tournament keys, its two rows at once, and its member
 // probe; what is left is the chain of the derivation and of the draws. A round
-// of 4096 children of the quintic grammar takes 62 us where it took 139, 1024
-// of a polynomial 41 for 78, 8192 of a list grammar 172 for 300, 2000 of a
-// statement grammar 109 for 183.
+// of 4096 children of the quintic grammar takes 59 us where it took 139, 1024
+// of a polynomial 39 for 78, 8192 of a list grammar 166 for 300, 1500 of a
+// statement grammar 105 for 183.
 #pragma once
 #include "phase_wave.hpp"
 
 namespace gagp_amd {
 
 constexpr int kWaveRow = 64;
+constexpr int kLaneValues = 64;  // pool entries of a program lowered with jumps
+// LDS of a wavefront that lowers rows: exchange words and, with jumps, the
+// program, which is decoded from here and stored in order.
+template <bool kJumps> struct LaneStore { int sums[64]; };
+template <> struct LaneStore<true> {
+  int sums[64];
+  Ins code[kLoopCode];
+  std::int64_t values[kLaneValues];  // payloads, a Bool's flag
+};
 
 // ---- wavefront reductions and scans in the data-parallel shifts (all lanes active) ----
 template <int kControl, int kRows>
@@ -406,14 +415,17 @@ __device__ inline std::uint64_t row_hash_row(const WaveRow& r) {
 // of use stored, unless every check of lower_phase_with passes on the types
 // the grammar declares; the node-by-node lowering then decides.
 // kJumps: all kinds; otherwise constants, inputs and operations only.
-// A statement row has been checked for definite assignment. `sums`: 64 LDS
-// words of this wavefront.
-// Node by node a child took 1.2 us a node, and 75-100 us with traversals.
+// A statement row has been checked for definite assignment. `store`: this
+// wavefront's LDS, which keeps the code and the pool's payloads (kJumps).
+// Node by node a child took 1.2 us a node, and 75-100 us with traversals; a
+// row takes 3 us here, 6 with jumps. The program stays in LDS for the decoding,
+// which read its neighbours' words from global memory in 20 us and takes half.
 template <bool kJumps>
 __device__ inline bool lower_row(const WaveGrammar& w, const WaveRow& r, GAS const std::uint8_t* local_types, int local_count,
                                  int expected_type, GAS Ins* code, int code_capacity, GAS Val* pool, int pool_capacity,
-                                 LAS int* sums, LowerResult& out) {
+                                 LAS LaneStore<kJumps>* store, LowerResult& out) {
   const int lane = wlane(), n = r.n;
+  LAS int* const sums = store->sums;
   if (n <= 0 || n > 64) return false;
   const bool live = lane < n, statement = kJumps && expected_type == kStatementType;
   const int x = lane_of(int(w.node), r.origin), x2 = lane_of(int(w.node2), r.origin);
@@ -506,7 +518,7 @@ __device__ inline bool lower_row(const WaveGrammar& w, const WaveRow& r, GAS con
     base = over_ancestors(under) + under;
   }
   const int bound = wave_max(live ? (s.arity == 0 && !nil ? base + 1 : walk || range ? base + 2 : logic ? base + 1 : 0) : 0);
-  if (words > code_capacity || entries > pool_capacity) return false;
+  if (words > code_capacity || entries > pool_capacity || (kJumps && (words > kLoopCode || entries > kLaneValues))) return false;
 
   // Types: each node's, as the grammar declares it or its rule gives it, and
   // the rules checked against the operands' below.
@@ -635,10 +647,12 @@ __device__ inline bool lower_row(const WaveGrammar& w, const WaveRow& r, GAS con
 
   // ---- the instructions ----
   const auto put = [&](int to, int op, int argc, int sp, unsigned cost, int a) {
-    *(GAS std::uint64_t*)(code + to) =
-        std::uint64_t(unsigned(op) | unsigned(argc) << 8 | unsigned(sp) << 16 | cost << 24) | std::uint64_t(unsigned(a)) << 32;
+    const std::uint64_t word = std::uint64_t(unsigned(op) | unsigned(argc) << 8 | unsigned(sp) << 16 | cost << 24) | std::uint64_t(unsigned(a)) << 32;
+    if constexpr (kJumps) *(LAS std::uint64_t*)(store->code + to) = word;
+    else *(GAS std::uint64_t*)(code + to) = word;
   };
   const auto put_value = [&](int to, std::uint64_t v, unsigned tag, unsigned flag) {
+    if constexpr (kJumps) store->values[to] = std::int64_t(tag == unsigned(TAG_BOOL) ? flag : v);
     pool[to].i = std::int64_t(v);
     *(GAS std::uint64_t*)(&pool[to].b) = std::uint64_t(flag) | std::uint64_t(tag) << 8;
   };
@@ -790,6 +804,10 @@ __device__ inline bool lower_row(const WaveGrammar& w, const WaveRow& r, GAS con
     }
   }
   if (!statement && lane == 0) put(words - 1, OP_RETURN, 0, 1, 1, 0);
+  if constexpr (kJumps) {
+    lanes_meet();
+    for (int k = lane; k < words; k += 64) *(GAS std::uint64_t*)(code + k) = *(LAS std::uint64_t*)(store->code + k);
+  }
   const bool straight = __ballot(live && (!fast || branch || logic || walk || bind || let)) == 0 && !statement;
   const bool few = local_count <= kFastInputs;
   const int value = statement ? returned : root;
