@@ -8,6 +8,7 @@
 #include <string>
 
 #include "engine.hpp"
+#include "parallel.hpp"
 #include "serve.hpp"
 
 using namespace gagp_amd;
@@ -52,21 +53,22 @@ int copy_out(const std::string& text, char* buf, size_t cap, size_t* needed) {
 ProgramIn program_in(const gagp_program& p) {
   if (p.code_len <= 0 || !p.code) throw std::invalid_argument("empty program");
   ProgramIn out;
-  for (int i = 0; i < p.code_len; ++i) {
-    out.op.push_back(p.code[i].op);
-    out.has_a.push_back(p.code[i].has_a);
-    out.has_b.push_back(p.code[i].has_b);
-    out.a.push_back(p.code[i].a);
-    out.b.push_back(p.code[i].b);
-    if (p.fuel) out.fuel.push_back(p.fuel[i]);
-  }
-  for (int i = 0; i < p.n_consts; ++i) {
-    Val v{};
-    std::memcpy(&v, &p.consts[i], sizeof v);
-    out.consts.push_back(v);
+  out.code.resize(std::size_t(p.code_len));
+  for (int i = 0; i < p.code_len; ++i)
+    out.code[std::size_t(i)] = CodeIn{p.code[i].op, p.code[i].has_a, p.code[i].has_b, p.code[i].a, p.code[i].b, p.fuel ? p.fuel[i] : 1u};
+  if (p.n_consts > 0) {
+    out.consts.resize(std::size_t(p.n_consts));
+    std::memcpy(static_cast<void*>(out.consts.data()), p.consts, sizeof(Val) * std::size_t(p.n_consts));
   }
   out.n_locals = p.n_locals;
   return out;
+}
+std::vector<ProgramIn> programs_in(const gagp_program* programs, int32_t n) {
+  std::vector<ProgramIn> in(static_cast<std::size_t>(n));
+  parallel_ranges(in.size(), 512, [&](std::size_t begin, std::size_t end) {
+    for (std::size_t i = begin; i < end; ++i) in[i] = program_in(programs[i]);
+  });
+  return in;
 }
 }  // namespace
 
@@ -113,9 +115,7 @@ int gagp_session_eval(gagp_session* s, const gagp_program* programs, int32_t n, 
                       uint32_t* out_counts) {
   return guarded([&] {
     if (!s || n < 0 || (n && (!programs || !out_fitness))) throw std::invalid_argument("invalid eval arguments");
-    std::vector<ProgramIn> in;
-    in.reserve(std::size_t(n));
-    for (int i = 0; i < n; ++i) in.push_back(program_in(programs[i]));
+    const std::vector<ProgramIn> in = programs_in(programs, n);
     s->s->eval(in, out_fitness, out_wrong, out_counts);
   });
 }
@@ -124,9 +124,7 @@ int gagp_session_eval_static(gagp_session* s, const gagp_program* programs, int3
                              uint32_t* out_counts) {
   return guarded([&] {
     if (!s || n < 0 || (n && (!programs || !out_fitness))) throw std::invalid_argument("invalid eval arguments");
-    std::vector<ProgramIn> in;
-    in.reserve(std::size_t(n));
-    for (int i = 0; i < n; ++i) in.push_back(program_in(programs[i]));
+    const std::vector<ProgramIn> in = programs_in(programs, n);
     s->s->eval_static(in, out_fitness, out_wrong, out_counts);
   });
 }
@@ -191,7 +189,7 @@ int gagp_batch_run(gagp_batch* b, int32_t use_graph) {
     b->b.run(use_graph != 0);
     b->prepared = b->ran = true;
     b->results.clear();
-    for (std::size_t i = 0; i < b->b.size(); ++i) b->results.push_back(b->b.result(int(i), false));
+    b->b.results(b->results);
   });
 }
 
@@ -223,7 +221,7 @@ int gagp_batch_finish(gagp_batch* b) {
     b->b.finish();
     b->ran = true;
     b->results.clear();
-    for (std::size_t i = 0; i < b->b.size(); ++i) b->results.push_back(b->b.result(int(i), false));
+    b->b.results(b->results);
   });
 }
 

@@ -29,6 +29,7 @@
 #include <stdexcept>
 
 #include "engine.hpp"
+#include "parallel.hpp"
 #include "population.hpp"
 #include "vary_wave.hpp"
 #include "vm.hpp"
@@ -1992,7 +1993,13 @@ struct SearchState {
   }
 
   // Allocates every device array of the search in its arena.
-  void allocate() { d = build(arena); }
+  // One device block of exactly the search's bytes.
+  void allocate() {
+    DeviceArena count(true);
+    (void)build(count);
+    arena.next_chunk = count.bytes;
+    d = build(arena);
+  }
   // Device bytes the search holds once allocated (its arena's chunks),
   // computed without allocating.
   std::size_t planned_bytes() const {
@@ -3171,14 +3178,9 @@ json::Value judge(const SearchState& s, const Cases& test, int fuel, const std::
   ProgramIn p;
   for (int i = 0; i < lr.code; ++i) {
     const Ins& x = code[i];
-    p.op.push_back(x.op);
     const bool a = x.op == OP_PUSH_CONST || x.op == OP_LOAD || x.op == OP_STORE || x.op == OP_JMP || x.op == OP_JMP_IF_FALSE ||
                    x.op == OP_JMP_IF_TRUE || x.op == OP_CALL_BUILTIN;
-    p.has_a.push_back(a);
-    p.has_b.push_back(x.op == OP_CALL_BUILTIN);
-    p.a.push_back(x.a);
-    p.b.push_back(x.argc);
-    p.fuel.push_back(x.fuel);
+    p.code.push_back(CodeIn{x.op, a, x.op == OP_CALL_BUILTIN, x.a, x.argc, x.fuel});
   }
   p.consts.assign(pool.begin(), pool.begin() + lr.constants);
   p.n_locals = lr.locals;
@@ -3247,6 +3249,29 @@ json::Value evaluate_program(const std::string& task_path, const std::string& pr
   v.obj["task"] = json::make_string(s.task.name);
   v.obj["split"] = json::make_string(split);
   return v;
+}
+
+void Batch::results(std::vector<SearchResult>& out) {
+  int device = 0;
+  HIP_OK(hipGetDevice(&device));
+  const std::size_t n = size();
+  std::vector<SearchResult> made(n);
+  std::vector<std::exception_ptr> failed(n);
+  parallel_ranges(n, 1, [&](std::size_t begin, std::size_t end) {
+    HIP_OK(hipSetDevice(device));  // a new thread's device is the first
+    for (std::size_t i = begin; i < end; ++i) {
+      try {
+        made[i] = result(int(i), false);
+      } catch (...) {
+        failed[i] = std::current_exception();
+        return;
+      }
+    }
+  });
+  for (std::size_t i = 0; i < n; ++i) {
+    if (failed[i]) std::rethrow_exception(failed[i]);
+    out.push_back(std::move(made[i]));
+  }
 }
 
 SearchResult Batch::result(int index, bool save_all) {
@@ -3388,11 +3413,8 @@ namespace {
 // pass, cpp/src/runtime/bytecode_verify.cpp): every instruction gets one
 // height; joins must agree; operand/constant/jump domains are checked.
 std::vector<Ins> verify_program(const ProgramIn& p, int n_inputs, int& max_stack, bool& jumps, bool* input_stores = nullptr) {
-  const int n = int(p.op.size());
+  const int n = int(p.code.size());
   if (n == 0) throw std::invalid_argument("empty program");
-  if (p.a.size() != std::size_t(n) || p.b.size() != std::size_t(n) || p.has_a.size() != std::size_t(n) ||
-      p.has_b.size() != std::size_t(n) || (!p.fuel.empty() && p.fuel.size() != std::size_t(n)))
-    throw std::invalid_argument("program arrays disagree in length");
   std::vector<int> height(std::size_t(n) + 1, -1);
   std::vector<int> work{0};
   height[0] = 0;
@@ -3404,14 +3426,14 @@ std::vector<Ins> verify_program(const ProgramIn& p, int n_inputs, int& max_stack
   // jump targets the NEG.
   std::vector<char> targeted(std::size_t(n) + 1, 0);
   for (int i = 0; i < n; ++i)
-    if ((p.op[i] == OP_JMP || p.op[i] == OP_JMP_IF_FALSE || p.op[i] == OP_JMP_IF_TRUE) && p.has_a[i] && p.a[i] >= 0 &&
-        p.a[i] <= n)
-      targeted[std::size_t(p.a[i])] = 1;
+    if ((p.code[i].op == OP_JMP || p.code[i].op == OP_JMP_IF_FALSE || p.code[i].op == OP_JMP_IF_TRUE) && p.code[i].has_a && p.code[i].a >= 0 &&
+        p.code[i].a <= n)
+      targeted[std::size_t(p.code[i].a)] = 1;
   const auto failing_neg = [&](int ip) {
-    if (ip == 0 || targeted[std::size_t(ip)] || p.op[ip - 1] != OP_PUSH_CONST || !p.has_a[ip - 1] || p.a[ip - 1] < 0 ||
-        p.a[ip - 1] >= int(p.consts.size()))
+    if (ip == 0 || targeted[std::size_t(ip)] || p.code[ip - 1].op != OP_PUSH_CONST || !p.code[ip - 1].has_a || p.code[ip - 1].a < 0 ||
+        p.code[ip - 1].a >= int(p.consts.size()))
       return false;
-    const int tag = p.consts[std::size_t(p.a[ip - 1])].tag;
+    const int tag = p.consts[std::size_t(p.code[ip - 1].a)].tag;
     return tag != TAG_INT && tag != TAG_FLOAT;
   };
   const auto flow = [&](int to, int h) {
@@ -3424,35 +3446,35 @@ std::vector<Ins> verify_program(const ProgramIn& p, int n_inputs, int& max_stack
     work.pop_back();
     if (ip == n) continue;
     const int h = height[ip];
-    const int op = p.op[ip];
+    const int op = p.code[ip].op;
     int pop = 0, push = 0;
     bool falls = true;
     switch (op) {
       case OP_PUSH_CONST:
-        if (!p.has_a[ip] || p.a[ip] < 0 || p.a[ip] >= int(p.consts.size())) throw std::invalid_argument("const index out of range");
+        if (!p.code[ip].has_a || p.code[ip].a < 0 || p.code[ip].a >= int(p.consts.size())) throw std::invalid_argument("const index out of range");
         push = 1; break;
       case OP_LOAD:
-        if (!p.has_a[ip] || p.a[ip] < 0 || p.a[ip] >= 64) throw std::invalid_argument("local index out of range");
+        if (!p.code[ip].has_a || p.code[ip].a < 0 || p.code[ip].a >= 64) throw std::invalid_argument("local index out of range");
         push = 1; break;
       case OP_STORE:
-        if (!p.has_a[ip] || p.a[ip] < 0 || p.a[ip] >= 64) throw std::invalid_argument("local index out of range");
+        if (!p.code[ip].has_a || p.code[ip].a < 0 || p.code[ip].a >= 64) throw std::invalid_argument("local index out of range");
         // A store into an input slot: the evaluators shadow it per execution.
-        if (p.a[ip] < n_inputs && input_stores) *input_stores = true;
+        if (p.code[ip].a < n_inputs && input_stores) *input_stores = true;
         pop = 1; break;
       case OP_NEG: pop = 1; push = 1; falls = !failing_neg(ip); break;
       case OP_NOT: case OP_CHECK_INT: case OP_CHECK_LIST: pop = 1; push = 1; break;
       case OP_ADD: case OP_SUB: case OP_MUL: case OP_DIV: case OP_MOD:
       case OP_LT: case OP_LE: case OP_GT: case OP_GE: case OP_EQ: case OP_NE: pop = 2; push = 1; break;
-      case OP_JMP: jumps = true; if (!p.has_a[ip]) throw std::invalid_argument("jump target missing"); flow(p.a[ip], h); falls = false; break;
+      case OP_JMP: jumps = true; if (!p.code[ip].has_a) throw std::invalid_argument("jump target missing"); flow(p.code[ip].a, h); falls = false; break;
       case OP_JMP_IF_FALSE: case OP_JMP_IF_TRUE:
         jumps = true;
-        if (!p.has_a[ip]) throw std::invalid_argument("jump target missing");
+        if (!p.code[ip].has_a) throw std::invalid_argument("jump target missing");
         if (h < 1) throw std::invalid_argument("stack underflow");
-        flow(p.a[ip], h - 1);
+        flow(p.code[ip].a, h - 1);
         pop = 1; break;
       case OP_CALL_BUILTIN:
-        if (!p.has_b[ip] || p.b[ip] < 0 || p.b[ip] > 8) throw std::invalid_argument("invalid builtin argc");
-        pop = p.b[ip]; push = 1; break;
+        if (!p.code[ip].has_b || p.code[ip].b < 0 || p.code[ip].b > 8) throw std::invalid_argument("invalid builtin argc");
+        pop = p.code[ip].b; push = 1; break;
       case OP_RETURN: if (h < 1) throw std::invalid_argument("return requires value on stack"); falls = false; break;
       default: throw Unsupported("opcode outside the device VM: " + std::to_string(op));
     }
@@ -3464,10 +3486,10 @@ std::vector<Ins> verify_program(const ProgramIn& p, int n_inputs, int& max_stack
   }
   std::vector<Ins> out(static_cast<std::size_t>(n));
   for (int i = 0; i < n; ++i) {
-    const std::uint32_t f = p.fuel.empty() ? 1u : p.fuel[i];
+    const std::uint32_t f = p.code[i].fuel;
     if (f > 255) throw Unsupported("instruction fuel charges above 255");
     const int h = height[i] < 0 ? 0 : height[i];  // unreachable instructions never run
-    out[i] = Ins{p.op[i], std::uint8_t(p.b[i]), std::uint8_t(h), std::uint8_t(f), p.a[i]};
+    out[i] = Ins{p.code[i].op, std::uint8_t(p.code[i].b), std::uint8_t(h), std::uint8_t(f), p.code[i].a};
   }
   return out;
 }
@@ -3709,40 +3731,56 @@ float Session::last_kernel_ms() const { return impl_->last_ms; }
 
 PackedPrograms Session::Impl::pack(const std::vector<ProgramIn>& programs, bool decode) const {
   const auto& I = *this;
+  struct Item {
+    std::vector<Ins> code;
+    std::vector<Step> steps;
+    int max_stack = 0, kind = 0, result = TAG_INVALID;
+    bool jumps = false, stores = false;  // stores: into an input
+  };
+  std::vector<Item> items(programs.size());
+  parallel_ranges(items.size(), 512, [&](std::size_t begin, std::size_t end) {
+    for (std::size_t i = begin; i < end; ++i) {
+      const ProgramIn& p = programs[i];
+      Item& x = items[i];
+      x.code = verify_program(p, I.cases.cd.n_inputs, x.max_stack, x.jumps, &x.stores);
+      for (const auto& v : p.consts) check_view(v, I.arena_len);
+      const FastCert cert = certify_fast(x.code, p.consts, I.input_tags, p.n_locals, x.max_stack, x.jumps, I.cases.cd.C);
+      x.kind = cert.fast ? 1 : 0;
+      x.result = cert.result_tag;
+      if (x.kind || !decode) continue;
+      const bool unit = std::all_of(x.code.begin(), x.code.end(), [](const Ins& y) { return y.fuel == 1; });
+      const LoopCert loop = certify_loop(x.code, p.consts, I.input_tags, p.n_locals, x.max_stack, unit, I.cases.cd.C);
+      if (!loop.loop) continue;
+      x.kind = 2;
+      x.result = loop.result_tag;
+      Step steps[kStepMax];
+      const int n = decode_steps(x.code.data(), int(x.code.size()), p.consts.data(), I.cases.cd.n_inputs, false, steps);
+      x.steps.assign(steps, steps + n);
+    }
+  });
   PackedPrograms k;
   bool stores = false;  // some program stores into an input
-  for (const auto& p : programs) {
+  for (std::size_t i = 0; i < items.size(); ++i) {
+    const ProgramIn& p = programs[i];
+    const Item& x = items[i];
     k.temps = std::max(k.temps, std::min(64, p.n_locals) - I.cases.cd.n_inputs);
-    int ms = 0;
-    bool j = false;
-    const auto ins = verify_program(p, I.cases.cd.n_inputs, ms, j, &stores);
-    for (const auto& v : p.consts) check_view(v, I.arena_len);
-    const FastCert cert = certify_fast(ins, p.consts, I.input_tags, p.n_locals, ms, j, I.cases.cd.C);
-    int kind = cert.fast ? 1 : 0, result = cert.result_tag;
-    if (!kind && decode) {
-      const bool unit = std::all_of(ins.begin(), ins.end(), [](const Ins& x) { return x.fuel == 1; });
-      const LoopCert loop = certify_loop(ins, p.consts, I.input_tags, p.n_locals, ms, unit, I.cases.cd.C);
-      if (loop.loop) {
-        kind = 2;
-        result = loop.result_tag;
-        Step steps[kStepMax];
-        const int n = decode_steps(ins.data(), int(ins.size()), p.consts.data(), I.cases.cd.n_inputs, false, steps);
-        k.step_off.push_back(k.steps.size());
-        k.step_n.push_back(n);
-        k.step_index.push_back(int(k.fast.size()));
-        k.steps.insert(k.steps.end(), steps, steps + n);
-      }
+    stores = stores || x.stores;
+    if (x.kind == 2) {
+      k.step_off.push_back(k.steps.size());
+      k.step_n.push_back(int(x.steps.size()));
+      k.step_index.push_back(int(i));
+      k.steps.insert(k.steps.end(), x.steps.begin(), x.steps.end());
     }
-    k.slots = std::max(k.slots, ms + 1);
-    k.fast.push_back(kind);
-    k.result.push_back(result);
+    k.slots = std::max(k.slots, x.max_stack + 1);
+    k.fast.push_back(x.kind);
+    k.result.push_back(x.result);
     k.pool_n.push_back(int(p.consts.size()));
     k.code_off.push_back(k.code.size());
     k.pool_off.push_back(k.pool.size());
-    k.code.insert(k.code.end(), ins.begin(), ins.end());
+    k.code.insert(k.code.end(), x.code.begin(), x.code.end());
     k.pool.insert(k.pool.end(), p.consts.begin(), p.consts.end());
-    k.lens.push_back(int(ins.size()));
-    k.jumps.push_back(j);
+    k.lens.push_back(int(x.code.size()));
+    k.jumps.push_back(x.jumps);
     k.locals.push_back(p.n_locals);
   }
   if (k.pool.empty()) k.pool.push_back(val_invalid());
@@ -3805,28 +3843,52 @@ void Session::eval(const std::vector<ProgramIn>& programs, double* fitness, std:
   const int n = int(programs.size());
   if (!n) return;
   const PackedPrograms k = I.pack(programs, true);
-  DeviceArena tmp;
-  auto dcode = tmp.upload(k.code);
-  auto dpool = tmp.upload(k.pool);
-  auto dprogs = tmp.upload(I.program_table(k, dcode, dpool));
-  auto dsteps = tmp.upload(k.steps);
-  auto dloops = tmp.upload(I.step_table(k, dsteps));
-  auto dfit = tmp.alloc<double>(std::size_t(n));
-  auto dwrong = tmp.alloc<unsigned>(std::size_t(n));
-  auto dcounts = tmp.alloc<unsigned>(std::size_t(n) * 3);
-  hipEvent_t a, b;
-  HIP_OK(hipEventCreate(&a));
-  HIP_OK(hipEventCreate(&b));
-  HIP_OK(hipEventRecord(a, nullptr));
-  I.launch(k, (const DProg*)dprogs, (const StepProg*)dloops, n, (double*)dfit, (unsigned*)dwrong, (unsigned*)dcounts);
-  HIP_OK(hipEventRecord(b, nullptr));
-  HIP_OK(hipEventSynchronize(b));
-  HIP_OK(hipEventElapsedTime(&I.last_ms, a, b));
-  (void)hipEventDestroy(a);
-  (void)hipEventDestroy(b);
-  HIP_OK(hipMemcpy(fitness, (const void*)dfit, sizeof(double) * n, hipMemcpyDeviceToHost));
-  if (wrong) HIP_OK(hipMemcpy(wrong, (const void*)dwrong, sizeof(unsigned) * n, hipMemcpyDeviceToHost));
-  if (counts) HIP_OK(hipMemcpy(counts, (const void*)dcounts, sizeof(unsigned) * 3 * n, hipMemcpyDeviceToHost));
+  // One allocation and one copy each way: the launch's inputs back to back,
+  // then its results.
+  std::size_t bytes = 0;
+  const auto place = [&](std::size_t size) {
+    const std::size_t at = bytes;
+    bytes += (size + 255) & ~std::size_t(255);
+    return at;
+  };
+  const std::size_t o_progs = place(sizeof(DProg) * std::size_t(n)), o_code = place(sizeof(Ins) * k.code.size()),
+                    o_pool = place(sizeof(Val) * k.pool.size()), o_steps = place(sizeof(Step) * k.steps.size()),
+                    o_loops = place(sizeof(StepProg) * k.step_n.size()), inputs = bytes;
+  const std::size_t o_fit = place(sizeof(double) * std::size_t(n)), o_wrong = place(sizeof(unsigned) * std::size_t(n)),
+                    o_counts = place(sizeof(unsigned) * 3 * std::size_t(n));
+  struct Block {
+    unsigned char* p = nullptr;
+    ~Block() { (void)hipFree(p); }
+  } block;
+  HIP_OK(hipMalloc(&block.p, bytes));
+  unsigned char* const base = block.p;
+  std::vector<unsigned char> staged(std::max(inputs, bytes - inputs));
+  const auto put = [&](std::size_t at, const auto& v) {
+    if (!v.empty()) std::memcpy(staged.data() + at, static_cast<const void*>(v.data()), v.size() * sizeof(v[0]));
+  };
+  put(o_progs, I.program_table(k, gbl(reinterpret_cast<const Ins*>(base + o_code)), gbl(reinterpret_cast<const Val*>(base + o_pool))));
+  put(o_code, k.code);
+  put(o_pool, k.pool);
+  put(o_steps, k.steps);
+  put(o_loops, I.step_table(k, gbl(reinterpret_cast<const Step*>(base + o_steps))));
+  HIP_OK(hipMemcpy(base, staged.data(), inputs, hipMemcpyHostToDevice));
+  struct Event {
+    hipEvent_t e = nullptr;
+    ~Event() { if (e) (void)hipEventDestroy(e); }
+  } a, b;
+  HIP_OK(hipEventCreate(&a.e));
+  HIP_OK(hipEventCreate(&b.e));
+  HIP_OK(hipEventRecord(a.e, nullptr));
+  I.launch(k, reinterpret_cast<const DProg*>(base + o_progs), reinterpret_cast<const StepProg*>(base + o_loops), n,
+           reinterpret_cast<double*>(base + o_fit), reinterpret_cast<unsigned*>(base + o_wrong), reinterpret_cast<unsigned*>(base + o_counts));
+  HIP_OK(hipEventRecord(b.e, nullptr));
+  HIP_OK(hipMemcpy(staged.data(), base + inputs, bytes - inputs, hipMemcpyDeviceToHost));
+  HIP_OK(hipEventSynchronize(b.e));
+  HIP_OK(hipEventElapsedTime(&I.last_ms, a.e, b.e));
+  const auto take = [&](void* to, std::size_t at, std::size_t size) { std::memcpy(to, staged.data() + (at - inputs), size); };
+  take(fitness, o_fit, sizeof(double) * std::size_t(n));
+  if (wrong) take(wrong, o_wrong, sizeof(unsigned) * std::size_t(n));
+  if (counts) take(counts, o_counts, sizeof(unsigned) * 3 * std::size_t(n));
 }
 
 // ---- allocation-free evaluation ----

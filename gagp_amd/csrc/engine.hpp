@@ -67,6 +67,9 @@ class Batch {
   // Device counters of search `index` (see gagp_batch_counters).
   std::vector<std::uint64_t> counters(int index) const;
   double init_ms() const;
+  // Appends every search's result, in order, up to the first that fails (its
+  // exception leaves).
+  void results(std::vector<SearchResult>& out);
   SearchResult result(int index, bool save_all);
   std::size_t size() const;
   std::size_t device_bytes() const;
@@ -171,10 +174,13 @@ constexpr std::size_t kStaticScratchBytes = std::size_t(16) << 20;
 
 // Evaluation session: the FitnessSessionGpu boundary (fixed case set,
 // arbitrary verified bytecode programs).
+struct CodeIn {
+  std::uint8_t op, has_a, has_b;
+  std::int32_t a, b;
+  std::uint32_t fuel;
+};
 struct ProgramIn {
-  std::vector<std::uint8_t> op, has_a, has_b;
-  std::vector<std::int32_t> a, b;
-  std::vector<std::uint32_t> fuel;  // empty: unit schedule
+  std::vector<CodeIn> code;
   std::vector<Val> consts;
   int n_locals = 0;
 };
