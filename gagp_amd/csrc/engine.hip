@@ -607,6 +607,44 @@ __device__ inline FastInputs staged_inputs(const StagedCases& sc, int C, int n_i
   return in;
 }
 
+// The canonical total of C case scores held in `scores`, computed by one
+// wavefront: L logical lanes over contiguous case chunks with 48-bit rounding,
+// then 32-lane groups and the total (the legacy metric sums the lane partials
+// directly). `sums`: kReplayWords doubles of this wavefront's LDS. 512 logical
+// lanes at a time leave their partials there, 33 words a group so that the
+// groups' reads fall into different banks, and a lane adds up each group.
+// Bound by the chain of rounded additions, now 48 and not 528 for 512 lanes;
+// with every addition on all lanes, each behind a shuffle, a program took about
+// 30 us and the launch of 540 programs on 600 discounted cases 127 us, now 47.
+constexpr int kReplayLanes = 512, kReplayWords = kReplayLanes / 32 * 33;
+__device__ inline double canonical_from_scores(const EvalParams& e, int C, const double* scores, int lane, double* sums) {
+  const int L = e.lanes;
+  double total = 0;
+  for (int chunk = 0; chunk < L; chunk += kReplayLanes) {
+    const int count = min(kReplayLanes, L - chunk);
+    for (int base = 0; base < count; base += 64) {
+      const int l = chunk + base + lane, at = base + lane;
+      const bool own = l < L;
+      const int begin = own ? int((std::int64_t(C) * l) / L) : 0;
+      const int end = own ? int((std::int64_t(C) * (l + 1)) / L) : 0;
+      double local = 0;
+      for (int c = begin; c < end; ++c) local = canon48(local + scores[c]);
+      sums[at + at / 32] = local;
+    }
+    wave_fence();
+    if (e.policy.metric == METRIC_LEGACY) {
+      for (int k = 0; k < count; ++k) total = canon48(total + sums[k + k / 32]);
+    } else {
+      const int groups = (count + 31) / 32, mine = min(32, count - 32 * lane);
+      double group = 0;
+      for (int k = 0; k < mine; ++k) group = canon48(group + sums[33 * lane + k]);
+      for (int k = 0; k < groups; ++k) total = canon48(total + rdlane_d(group, k));
+    }
+    wave_fence();
+  }
+  return total;
+}
+
 // Scores one program over all cases with the canonical reduction
 // (fitness_cpu.cpp:97-171: L logical lanes over contiguous case chunks,
 // 48-bit rounding after every addition, 32-lane groups then the total).
@@ -617,9 +655,10 @@ __device__ inline FastInputs staged_inputs(const StagedCases& sc, int C, int n_i
 // otherwise the general VM runs it with its stack in LDS.
 // `scores` (this wavefront's LDS buffer of C doubles, or null) keeps every
 // case score of the first pass, so the canonical order is replayed from it
-// instead of by running the program again; the fast kernel always has it.
+// instead of by running the program again; the fast kernel always has it, and `sums`
+// (canonical_from_scores).
 template <int kKind>
-__device__ EvalOut eval_program(const EvalParams& e, const ProgView& pv, WaveStack& st, double* scores, int lane,
+__device__ EvalOut eval_program(const EvalParams& e, const ProgView& pv, WaveStack& st, double* scores, int lane, double* sums,
                                 StagedCases staged = StagedCases{}) {
   static_assert(kKind == 0 || kKind == 1, "the looping path has its own kernel");
   constexpr bool kFast = kKind != 0;  // a typed path: scores in LDS, inputs untagged
@@ -679,6 +718,10 @@ __device__ EvalOut eval_program(const EvalParams& e, const ProgView& pv, WaveSta
   // Canonical order: lane j owns logical lanes j, j+64, ... of L.
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");  // scores[] of other lanes
   __builtin_amdgcn_wave_barrier();
+  if constexpr (kFast) {
+    out.fitness = canonical_from_scores(e, C, scores, lane, sums);
+    return out;
+  }
   const int L = e.lanes;
   double group_total = 0;
   for (int base = 0; base < L; base += 64) {
@@ -692,9 +735,7 @@ __device__ EvalOut eval_program(const EvalParams& e, const ProgView& pv, WaveSta
     for (int s = 0; s < longest; ++s) {
       const int c = begin + s;
       const bool active = c < end;
-      if constexpr (kFast) {
-        if (active) local = canon48(local + scores[c]);
-      } else if (scores) {
+      if (scores) {
         if (active) local = canon48(local + scores[c]);
       } else {
         const LaneResult r = run(active ? c : 0, active);
@@ -727,42 +768,6 @@ __device__ EvalOut eval_program(const EvalParams& e, const ProgView& pv, WaveSta
   }
   out.fitness = group_total;
   return out;
-}
-
-// The canonical total of C case scores held in `scores` (LDS), computed by
-// one wavefront: L logical lanes over contiguous case chunks with 48-bit
-// rounding, then 32-lane groups and the total (the legacy metric sums the
-// lane partials directly), as eval_program's replay.
-__device__ inline double canonical_from_scores(const EvalParams& e, int C, const double* scores, int lane) {
-  const int L = e.lanes;
-  double group_total = 0;
-  for (int base = 0; base < L; base += 64) {
-    const int l = base + lane;
-    const bool own = l < L;
-    const int begin = own ? int((std::int64_t(C) * l) / L) : 0;
-    const int end = own ? int((std::int64_t(C) * (l + 1)) / L) : 0;
-    int longest = end - begin;
-    for (int off = 32; off > 0; off >>= 1) { const int y = __shfl_xor(longest, off, 64); longest = y > longest ? y : longest; }
-    double local = 0;
-    for (int k = 0; k < longest; ++k) {
-      const int c = begin + k;
-      if (c < end) local = canon48(local + scores[c]);
-    }
-    for (int half = 0; half < 2; ++half) {
-      if (base + half * 32 >= L) break;
-      double group = 0;
-      for (int k = 0; k < 32; ++k) {
-        const int src = half * 32 + k;
-        const double v = __shfl(local, src, 64);
-        if (base + src < L) {
-          if (e.policy.metric == METRIC_LEGACY) group_total = canon48(group_total + v);
-          else group = canon48(group + v);
-        }
-      }
-      if (e.policy.metric != METRIC_LEGACY) group_total = canon48(group_total + group);
-    }
-  }
-  return group_total;
 }
 
 // Items of the looping kernel: (program, group of `group` consecutive
@@ -851,7 +856,9 @@ __global__ __launch_bounds__(64) void k_eval_loop(DSearch* all, const BlockMap* 
       continue;
     }
     wave_fence();  // the canonical replay reads the other lanes' scores
-    const double fitness = frac ? canonical_from_scores(e, C, scores, lane) : double(total);
+    // The program has ended: its slots hold the replay's partials.
+    static_assert((kLoopLocals + kStepStack) * 64 >= kReplayWords, "slots of a program without inputs");
+    const double fitness = frac ? canonical_from_scores(e, C, scores, lane, (double*)slots) : double(total);
     if (lane == 0) {
       // Ranking rounds every published fitness to a 40-bit mantissa.
       if (mode == 1) { d.c_fit[slot] = canon40(fitness); d.c_wrong[slot] = tw; }
@@ -874,6 +881,7 @@ __global__ __launch_bounds__(kEvalThreads) void k_loop_finish(DSearch* all, cons
   if (mode == 1 ? !search_live(d) : (!d.active || *d.error)) return;
   const int C = d.cd.C, tiles = (C + 63) / 64, groups = (tiles + group - 1) / group;
   if (groups <= 1 || C > kScoreCases) return;
+  __shared__ double replay[kWavesPerBlock][kReplayWords];
   const int lane = threadIdx.x % 64, part = lane % 16;
   const EvalParams e{d.cd, d.fuel, d.lanes, d.penalty, d.policy};
   const int count = mode == 1 ? d.n_pending[2] : d.P;
@@ -895,7 +903,7 @@ __global__ __launch_bounds__(kEvalThreads) void k_loop_finish(DSearch* all, cons
     double fitness = double(t.sum);
     for (unsigned long long m = __ballot(mine && part == 0 && t.fractional); m; m &= m - 1) {
       const int from = wave_first(m);
-      const double total = canonical_from_scores(e, C, d.loop_scores + std::size_t(rdlane(slot, from)) * C, lane);
+      const double total = canonical_from_scores(e, C, d.loop_scores + std::size_t(rdlane(slot, from)) * C, lane, replay[wave_index()]);
       if (lane == from) fitness = total;
     }
     if (mine && part == 0) {
@@ -929,6 +937,7 @@ __global__ __launch_bounds__(kEvalThreads) void k_eval(DSearch* all, const Block
   if (mode == 1 ? !search_live(d) : (!d.active || *d.error)) return;
   if (kFast && d.typed_tiles) return;  // k_eval_tiles scores them
   extern __shared__ unsigned char smem[];
+  __shared__ double replay[kFast ? kWavesPerBlock : 1][kFast ? kReplayWords : 1];
   const int wave = wave_index(), lane = threadIdx.x % 64;
   WaveStack st = stack_of(smem, kFast ? 0 : d.stack_slots, kFast ? 0 : d.temp_slots, wave, kFast ? 0 : d.input_shadow);
   // Score buffers follow the stacks of the block's wavefronts.
@@ -951,7 +960,7 @@ __global__ __launch_bounds__(kEvalThreads) void k_eval(DSearch* all, const Block
     if (mode == 0 && eval_class(pmode, d.cd.C) != kKind) continue;  // another kernel scores it
     const ProgView pv{d.code + std::size_t(slot) * d.code_cap, d.pool + std::size_t(slot) * d.pool_cap, d.code_len[slot],
                       d.n_locals, pmode & 1, (pmode >> 1) & 1, d.pool_len[slot], (pmode & 4) ? TAG_BOOL : TAG_INT};
-    const EvalOut r = eval_program<kKind>(e, pv, st, scores, lane, staged);
+    const EvalOut r = eval_program<kKind>(e, pv, st, scores, lane, replay[kKind == 0 ? 0 : wave], staged);
     if (lane == 0) {
       // Ranking rounds every published fitness to a 40-bit mantissa.
       if (mode == 1) { d.c_fit[slot] = canon40(r.fitness); d.c_wrong[slot] = r.wrong; }
@@ -979,7 +988,7 @@ __global__ __launch_bounds__(kEvalThreads) void k_eval_tiles(DSearch* all, const
   if (!d.typed_tiles) return;  // uniform per block
   extern __shared__ unsigned char smem[];
   double* const scores = reinterpret_cast<double*>(smem);  // [C]
-  __shared__ double part_sum[kWavesPerBlock];
+  __shared__ double part_sum[kWavesPerBlock], replay[kReplayWords];
   __shared__ unsigned part_count[kWavesPerBlock][4];  // wrong, errors, timeouts, integral
   __shared__ unsigned long long part_fuel[kWavesPerBlock];
   const int wave = wave_index(), lane = threadIdx.x % 64;
@@ -1039,7 +1048,7 @@ __global__ __launch_bounds__(kEvalThreads) void k_eval_tiles(DSearch* all, const
         all_integral = all_integral && part_count[k][3] != 0;
         tf += part_fuel[k];
       }
-      const double fitness = all_integral ? total : canonical_from_scores(e, C, scores, lane);
+      const double fitness = all_integral ? total : canonical_from_scores(e, C, scores, lane, replay);
       if (lane == 0) {
         // Ranking rounds every published fitness to a 40-bit mantissa.
         if (mode == 1) { d.c_fit[slot] = canon40(fitness); d.c_wrong[slot] = tw; }
@@ -1647,13 +1656,14 @@ template <bool kFast>
 __global__ __launch_bounds__(kEvalThreads) void k_eval_programs(const DProg* progs, int n, EvalParams e, int slots, int temps,
                                                                  int shadow, double* fitness, unsigned* wrong, unsigned* counts) {
   extern __shared__ unsigned char smem[];
+  __shared__ double replay[kFast ? kWavesPerBlock : 1][kFast ? kReplayWords : 1];
   const int wave = wave_index(), lane = threadIdx.x % 64;
   WaveStack st = stack_of(smem, kFast ? 0 : slots, kFast ? 0 : temps, wave, kFast ? 0 : shadow);
   double* scores = kFast ? reinterpret_cast<double*>(smem) + std::size_t(wave) * e.cd.C : nullptr;
   for (int i = blockIdx.x * kWavesPerBlock + wave; i < n; i += gridDim.x * kWavesPerBlock) {
     const DProg p = progs[i];
     if (p.fast != int(kFast)) continue;  // 2: k_eval_steps scores it
-    const EvalOut r = eval_program<kFast ? 1 : 0>(e, view_of(p), st, scores, lane);
+    const EvalOut r = eval_program<kFast ? 1 : 0>(e, view_of(p), st, scores, lane, replay[kFast ? wave : 0]);
     if (lane == 0) {
       fitness[i] = r.fitness;
       wrong[i] = e.policy.metric == METRIC_LEGACY ? 0 : r.wrong;
@@ -1674,7 +1684,7 @@ struct StepProg { GAS const Step* steps; int n_steps, index, result_tag; };
 __global__ __launch_bounds__(kEvalThreads) void k_eval_steps(const StepProg* progs, int n, EvalParams e, double* fitness,
                                                               unsigned* wrong, unsigned* counts) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  __shared__ double part_sum[kWavesPerBlock];
+  __shared__ double part_sum[kWavesPerBlock], replay[kReplayWords];
   __shared__ unsigned part_count[kWavesPerBlock][4];  // wrong, errors, timeouts, integral
   const int waves = int(blockDim.x) / 64, wave = wave_index(), lane = threadIdx.x % 64;
   const int C = e.cd.C, n_in = e.cd.n_inputs, slots = step_slots(n_in);
@@ -1725,7 +1735,7 @@ __global__ __launch_bounds__(kEvalThreads) void k_eval_steps(const StepProg* pro
         tt += part_count[k][2];
         all_integral = all_integral && part_count[k][3] != 0;
       }
-      const double f = all_integral ? total : canonical_from_scores(e, C, scores, lane);
+      const double f = all_integral ? total : canonical_from_scores(e, C, scores, lane, replay);
       if (lane == 0) {
         fitness[p.index] = f;
         wrong[p.index] = e.policy.metric == METRIC_LEGACY ? 0 : tw;
@@ -2352,7 +2362,7 @@ struct Batch::Impl {
       eval_general_lds = std::max(eval_general_lds, stacks + (x.d.general_scores ? score_buf : 0));
       const std::size_t cases = x.d.stage_cases ? staged_case_bytes(x.d.cd.C, staged_inputs_of(x.d.n_locals, x.d.cd.n_inputs)) : 0;
       if (x.d.cd.C <= kScoreCases) {
-        eval_fast_lds = std::max(eval_fast_lds, score_buf + cases);
+        if (!x.d.typed_tiles) eval_fast_lds = std::max(eval_fast_lds, score_buf + cases);
         eval_loop_lds = std::max(eval_loop_lds, std::size_t(step_slots(staged_inputs_of(x.d.n_locals, x.d.cd.n_inputs))) * 64 * 8);
       }
       if (x.d.typed_tiles) eval_tiles_lds = std::max(eval_tiles_lds, std::size_t(8) * x.d.cd.C);
