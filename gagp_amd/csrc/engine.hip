@@ -6,8 +6,9 @@
 //   k_record  history row of generation r/per_epoch (best row, fitness vector)
 //   k_vary    tournaments, crossover, mutation, compare, completed-result
 //             reuse through the member table, lowering, pending lists
-//             (wavefront/child)
-//   k_eval    bytecode VM + canonical reduction (wavefront/program)
+//             (wavefront/child); k_lower lowers what it leaves
+//   k_eval    the bytecode VMs + canonical reduction (k_eval, k_eval_tiles,
+//             k_eval_loop with k_loop_finish)
 //   k_place   mt19937_64 inverse-tournament placement (block/search), with
 //             k_clear emptying the member table beside it
 //   k_commit  placed children overwrite their members; every member is
