@@ -860,12 +860,12 @@ __device__ inline LaneResult vm_steps(const StepProgram& f, const FastInputs& in
             sl[a * 64] = wrap_add(counter, 1);
             next = target;
           } else {
-            // Leaving lanes keep the variable.
+            // Leaving lanes keep the variable, and an unset input unset.
             const std::int64_t limit = sl[b * 64], old = sl[p * 64];
             const bool more = counter < limit;
             const unsigned long long stay = __ballot(more), group = __ballot(true);
             sl[p * 64] = more ? counter : old;
-            sink_slot = unsigned(p);
+            sink_slot = stay != 0 ? unsigned(p) : kStepNoSlot;
             mask = stay;
             event = stay != 0 && stay != group ? EV_TEST : EV_NONE;
             next = stay == 0 ? target : next;
