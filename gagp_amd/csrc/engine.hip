@@ -218,8 +218,9 @@ __device__ __attribute__((always_inline)) inline int store_lowered(const DSearch
   const Val* pool = d.pool + std::size_t(slot) * d.pool_cap;
   const bool ok = r.status == ST_OK && r.stack_bound >= 1 && r.stack_bound <= d.stack_slots &&
                   r.locals - d.n_locals <= d.temp_slots - d.input_shadow;
-  // bit 0: jumps; bit 1: typed straight-line (vm_fast); bit 2: Bool result; bit 3: typed looping (vm_steps)
-  const int flags = r.jumps | (r.fast ? 2 : 0) | (r.result_type == TAG_BOOL ? 4 : 0) | (r.loop ? 8 : 0);
+  // bit 0: jumps; bit 1: typed straight-line (vm_fast); bit 2: Bool result; bit 3: typed looping (vm_steps, where
+  // the search has that path; else the general VM scores the program)
+  const int flags = r.jumps | (r.fast ? 2 : 0) | (r.result_type == TAG_BOOL ? 4 : 0) | (r.loop && d.steps ? 8 : 0);
   int steps = 0;
   if (ok && r.loop && d.steps) {
     if (!values) wave_fence();  // the code and pool stored above are read across the lanes
@@ -1925,7 +1926,7 @@ struct SearchState {
   int stepped = 0;  // rounds the host has stepped this search (it idles past `rounds`)
   int fuel = 0;
   double penalty = 0;
-  bool may_jump = false;   // programs may go to the looping path: if/and/or, traversals, statements, lets
+  bool may_jump = false;   // programs may go to the looping path (leaves_straight_line)
   bool statement = false;  // a Program entry: statement programs with grammar locals
   // The export name table: the names the first initial member uses, in
   // declaration order (the layout prototype of phase_population_cpu.cpp:195),
@@ -1983,18 +1984,8 @@ struct SearchState {
     layout = whole_program_layout(grammar);
     phase = compile_phase(grammar, grammar.entry, grammar.max_depth, unsigned(cfg.site_depth), train.input_names);
     R = std::min<int>(kPhaseCapacity, int(layout.max_variable_nodes));
-    for (const auto& x : phase.exprs)
-      may_jump = may_jump || x.node.kind == TK_IF || x.node.kind == TK_AND || x.node.kind == TK_OR || x.node.kind == TK_TRAVERSE ||
-                 x.node.kind == TK_FOR_RANGE;
     statement = grammar.nts[grammar.entry].cat == Cat::Program;
-    // Hidden locals (statements, lets) also make programs for the looping
-    // path, with or without jumps, and so does straight-line code beyond the
-    // straight-line VM's limits: one instruction per node plus RETURN, and a
-    // stack of at most (arity - 1) pending operands per level plus one.
-    int arity = 1;
-    for (const auto& x : phase.exprs) arity = std::max(arity, x.node.arity);
-    may_jump = may_jump || statement || phase.has_let || R + 1 > kFastCode ||
-               (arity - 1) * int(layout.slot_max_depth) + 1 > kFastStack;
+    may_jump = leaves_straight_line(phase, train.input_types, layout, R, statement);
     if (!s.init_path.empty()) {
       imported = load_population(s.init_path, grammar, phase, unsigned(cfg.site_depth), R, std::size_t(P));
       has_import = true;

@@ -12,6 +12,9 @@
 //   compile_phase_tree    .../device/phase_compile.cuh:206-895 (expressions,
 //                         traversals and statements)
 #pragma once
+#include <algorithm>
+#include <vector>
+
 #include "core.hpp"
 #include "grammar.hpp"
 
@@ -468,6 +471,25 @@ GHD inline bool loop_operation(int opcode, int builtin, int arity, int a0, int a
       return arity == 2 && a0 == TAG_INT_LIST && a1 == TAG_INT;
   }
   return fast_operation(opcode, builtin, arity, a0, a1, a2);
+}
+
+// Whether programs of a grammar may leave the straight-line path for the
+// looping one: branches, loops and hidden locals (statements, lets); values
+// the straight-line path does not hold (an IntList input, which len and
+// indexing read without a jump); and code beyond its limits, one instruction
+// per node plus RETURN, and a stack of at most (arity - 1) pending operands
+// per level plus one. `rows`: nodes of a row.
+inline bool leaves_straight_line(const PhaseGrammar& g, const std::vector<std::uint8_t>& input_types, const Layout& layout, int rows,
+                                 bool statement) {
+  bool leaves = statement || g.has_let || rows + 1 > kFastCode;
+  int arity = 1;
+  for (const auto& x : g.exprs) {
+    const int kind = x.node.kind;
+    leaves = leaves || kind == TK_IF || kind == TK_AND || kind == TK_OR || kind == TK_TRAVERSE || kind == TK_FOR_RANGE;
+    arity = std::max(arity, x.node.arity);
+  }
+  for (const std::uint8_t type : input_types) leaves = leaves || type == TAG_INT_LIST;
+  return leaves || (arity - 1) * int(layout.slot_max_depth) + 1 > kFastStack;
 }
 
 // An open operation of the post-order walk: its node, operands seen so far,

@@ -1,6 +1,7 @@
-"""Programs of a search whose cases leave inputs out, scored by the owner seam
-twice: on the task's cases, where the looping path runs them, and on the same
-cases repeated to above 4096, where the general VM does. The draws do not read the cases, so
+"""Programs of a search whose cases leave inputs out, and of a grammar whose
+only list operations are len and index, scored by the owner seam twice: on the
+task's cases, where the looping path runs them, and on the same cases repeated
+to above 4096, where the general VM does. The draws do not read the cases, so
 the programs are the same, and with integer losses every score and count is
 the repetition's multiple. Initial population and one batch of children."""
 import json
@@ -9,7 +10,8 @@ import os
 import pytest
 
 import gagp_amd
-from _util import GOLDEN
+from _util import GOLDEN, strip_timing
+from test_looping_grammar import reads_only
 
 pytestmark = pytest.mark.gpu
 REPEAT = 42  # 100 cases: two tiles, the second part full
@@ -72,3 +74,24 @@ def unset(name):
 def test_unset_inputs_score_as_in_the_general_vm(task, name, population, tmp_path):
     print("two paths", task, flush=True)
     same_scores(*task_of(tmp_path, task, unset(name)), population)
+
+
+def reads(grammar, cases):
+    grammar.clear()
+    grammar.update(reads_only())
+
+
+def test_list_reads_without_a_jump_score_as_in_the_general_vm(tmp_path):
+    print("two paths reads", flush=True)
+    short, long = task_of(tmp_path, "list_sum_even", reads)
+    same_scores(short, long, 300)
+    # Alone and beside a search with loops, straight and batched rounds publish the same.
+    results = []
+    for beside in (None, os.path.join(GOLDEN, "tasks", "list_sum_even", "task.json")):
+        batch = gagp_amd.Batch()
+        batch.add(short, None, 300, 6, 5)
+        if beside:
+            batch.add(beside, None, 300, 6, 5)
+        batch.run()
+        results.append(strip_timing(batch.result(0)))
+    assert results[0] == results[1]
