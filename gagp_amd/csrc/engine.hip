@@ -60,10 +60,10 @@ struct Counters {
   unsigned long long children, child_nodes, child_consts, parent_nodes, parent_consts, child_code_words, child_pool_words;
 };
 
-// Totals of one work item of the looping kernel (a program on one tile
-// group), combined per program by k_loop_finish.
-struct alignas(16) LoopPart {
-  long long sum;            // of the integral scores
+// Totals of one program's tile groups in the looping kernel (device atomics),
+// taken and cleared by k_loop_finish.
+struct alignas(16) LoopAcc {
+  unsigned long long sum;   // of the integral scores, two's complement
   unsigned long long fuel;  // charged fuel
   unsigned wrong, errors, timeouts, fractional;
 };
@@ -101,9 +101,9 @@ struct DSearch {
   GAS int* reuse;    // the member whose result the child takes, -1, or -2 until k_lower has lowered the child
   GAS double* c_fit;
   GAS unsigned *c_wrong, *c_nodes;
-  GAS Ins* code;
+  GAS Ins* code;     // of a program of the looping path its packed steps, in the same words
   GAS Val* pool;
-  GAS int *code_len, *pool_len, *code_jumps;
+  GAS int *code_len, *pool_len, *code_jumps;  // code_jumps: flags, and the number of packed steps << 8
   GAS std::uint64_t* child_hash;
   // pending[2B]: children to score, general ones from the front of [0, B),
   // vm_fast ones from its back, vm_steps ones in [B, 2B); n_pending[3] counts each.
@@ -141,10 +141,8 @@ struct DSearch {
   GAS const double* select;
   int general_scores;  // the general evaluation kernel has an LDS score buffer for this search
   GAS double* loop_scores;  // the looping kernel's case scores: C per program slot
-  GAS LoopPart* loop_part;  // the looping kernel's totals: one per 64-case tile and program slot
-  GAS Step* steps;          // decoded steps of the programs of the looping path, step_cap per slot
-  GAS int* step_n;
-  int step_cap;
+  GAS LoopAcc* loop_acc;    // the looping kernel's totals per program slot (zero between evaluations)
+  int looping;              // the search has the looping path: its programs' packed steps replace their code
   int stage_cases;     // the typed evaluation kernel stages the case set in LDS
   int typed_tiles;     // typed programs go to k_eval_tiles (more than one 64-case tile, C <= kScoreCases)
 };
@@ -209,26 +207,28 @@ __global__ __launch_bounds__(64 * kVaryWaves) void k_init_pop(DSearch* all, cons
 }
 
 // ---- lowering: one wavefront per row ----
-// Records the lowering `r` of a slot and decodes a looping program's steps,
-// from `code` and `values` where the caller has them at hand; returns the code
-// flags it stores (code_jumps).
+// Records the lowering `r` of a slot, whose code is in the slot or, where
+// `kept` is not null, in this wavefront's LDS: a looping program's is decoded
+// into the slot, any other stands there. Returns the code flags it stores
+// (code_jumps).
 __device__ __attribute__((always_inline)) inline int store_lowered(const DSearch& d, int slot, const LowerResult& r,
-                                                                   const Ins* code = nullptr, const std::int64_t* values = nullptr) {
-  if (!code) code = d.code + std::size_t(slot) * d.code_cap;
-  const Val* pool = d.pool + std::size_t(slot) * d.pool_cap;
+                                                                   const Ins* kept = nullptr) {
+  Ins* const code = d.code + std::size_t(slot) * d.code_cap;
   const bool ok = r.status == ST_OK && r.stack_bound >= 1 && r.stack_bound <= d.stack_slots &&
-                  r.locals - d.n_locals <= d.temp_slots - d.input_shadow;
+                   r.locals - d.n_locals <= d.temp_slots - d.input_shadow;
+  const bool steps = ok && r.loop && d.looping;
+  int n = 0;
+  if (steps) {
+    if (!kept) wave_fence();  // the code stored above is read across the lanes
+    n = decode_steps_w(kept ? kept : code, r.code, d.n_locals, reinterpret_cast<std::uint64_t*>(code));
+  } else if (kept) {
+    for (int k = wlane(); k < r.code; k += 64) code[k] = kept[k];
+  }
   // bit 0: jumps; bit 1: typed straight-line (vm_fast); bit 2: Bool result; bit 3: typed looping (vm_steps, where
   // the search has that path; else the general VM scores the program)
-  const int flags = r.jumps | (r.fast ? 2 : 0) | (r.result_type == TAG_BOOL ? 4 : 0) | (r.loop && d.steps ? 8 : 0);
-  int steps = 0;
-  if (ok && r.loop && d.steps) {
-    if (!values) wave_fence();  // the code and pool stored above are read across the lanes
-    steps = decode_steps_w(code, r.code, pool, values, d.n_locals, d.steps + std::size_t(slot) * d.step_cap);
-  }
+  const int flags = r.jumps | (r.fast ? 2 : 0) | (r.result_type == TAG_BOOL ? 4 : 0) | (steps ? 8 : 0) | n << 8;
   if (wlane() == 0) {
     if (!ok) raise(d, 200 + r.status);
-    if (d.steps) d.step_n[slot] = steps;
     d.code_len[slot] = ok ? r.code : 0;
     d.pool_len[slot] = ok ? r.constants : 0;
     d.code_jumps[slot] = flags;
@@ -269,7 +269,7 @@ __global__ __launch_bounds__(64 * kVaryWaves) void k_lower_members(DSearch* all,
     WaveOrigins source{row};
     lowered = lower_into_w<kWalks>(g, d, row, m, source, walk_lds[wave_index()]);
   }
-  if (done) store_lowered(d, m, lowered, store.code, store.values);
+  if (done) store_lowered(d, m, lowered, store.code);
   else store_lowered(d, m, lowered);
 }
 
@@ -479,7 +479,7 @@ __global__ __launch_bounds__(64 * kVaryWaves) __attribute__((amdgpu_waves_per_eu
   const bool done = in_lanes && lower_row<kDefer>(w, child_row, d.local_types, d.n_locals, d.expected_type, d.code + std::size_t(c) * d.code_cap,
                                           d.code_cap, d.pool + std::size_t(c) * d.pool_cap, d.pool_cap, (LAS LaneStore<kDefer>*)&store, lowered);
   if constexpr (kDefer) {
-    if (done) pend_child(d, c, store_lowered(d, c, lowered, store.code, store.values));
+    if (done) pend_child(d, c, store_lowered(d, c, lowered, store.code));
     else if (wlane() == 0) d.reuse[c] = -2;
     return;
   }
@@ -788,10 +788,11 @@ __host__ __device__ inline int loop_blocks(int C, int n, int group = 1) {
 // by descending list length, so the longest items of all programs start
 // first and the launch ends with the shortest.
 // Scores go to the program's row of loop_scores (HBM). A program with one
-// group is finished by its wavefront; otherwise every group writes its totals
-// to its own LoopPart and k_loop_finish, the next launch, combines them: no
-// fence or atomic orders the items of one program. LDS: step_slots(n_inputs)
-// slots of 64 lanes, independent of the case count.
+// group is finished by its wavefront; otherwise every group adds its totals
+// (whole numbers, so their order is free) to the program's LoopAcc, and
+// k_loop_finish, the next launch, takes them: no fence orders the items of one
+// program. LDS: step_slots(n_inputs) slots of 64 lanes, independent of the
+// case count.
 // kGrouped false is the one-tile instantiation (group 1): its loop-carried
 // totals fold away.
 // Bound by instruction issue of the step loop (scalar decode and branches).
@@ -819,7 +820,8 @@ __global__ __launch_bounds__(64) void k_eval_loop(DSearch* all, const BlockMap* 
     const int pmode = d.code_jumps[slot];
     if (mode == 0 && eval_class(pmode, C) != 2) continue;  // another kernel scores it (uniform per wavefront)
     const int n_in = staged_inputs_of(d.n_locals, e.cd.n_inputs), result_tag = (pmode & 4) ? TAG_BOOL : TAG_INT;
-    const StepProgram sp = steps_load(d.steps + std::size_t(slot) * d.step_cap, d.step_n[slot], lane);
+    const StepProgram sp = steps_load((GAS const std::uint64_t*)(d.code + std::size_t(slot) * d.code_cap),
+                                      d.pool + std::size_t(slot) * d.pool_cap, pmode >> 8, lane);
     GAS double* const scores = d.loop_scores + std::size_t(slot) * C;
     long long total = 0;  // exact while no score is fractional
     bool frac = false;
@@ -853,8 +855,15 @@ __global__ __launch_bounds__(64) void k_eval_loop(DSearch* all, const BlockMap* 
       tf += wave_sum_u64(active ? unsigned(r.fuel_used) : 0u);
     }
     if (groups > 1) {
-      if (lane == 0)
-        d.loop_part[std::size_t(slot) * tiles + q0] = LoopPart{frac ? 0 : total, tf, tw, te, tt, unsigned(frac)};
+      if (lane == 0) {
+        GAS LoopAcc* const acc = d.loop_acc + slot;
+        if (frac) atomicOr(&acc->fractional, 1u);
+        else atomicAdd(&acc->sum, (unsigned long long)total);
+        atomicAdd(&acc->fuel, tf);
+        if (tw) atomicAdd(&acc->wrong, tw);
+        if (te) atomicAdd(&acc->errors, te);
+        if (tt) atomicAdd(&acc->timeouts, tt);
+      }
       continue;
     }
     wave_fence();  // the canonical replay reads the other lanes' scores
@@ -872,8 +881,8 @@ __global__ __launch_bounds__(64) void k_eval_loop(DSearch* all, const BlockMap* 
   }
 }
 
-// Combines the LoopParts of every program of more than one tile group: 16
-// lanes per program and four programs per wavefront, the canonical replay
+// Takes and clears the LoopAcc of every program of more than one tile group:
+// 16 lanes per program and four programs per wavefront, the canonical replay
 // over the program's scores by the whole wavefront where some tile had a
 // non-integral one.
 constexpr int kFinishPrograms = 4 * kWavesPerBlock;  // programs per block
@@ -891,18 +900,15 @@ __global__ __launch_bounds__(kEvalThreads) void k_loop_finish(DSearch* all, cons
     const int i = base + lane / 16;
     const int slot = i >= count ? -1 : mode == 1 ? d.pending[pending_at(d.B, 2, i)] : i;
     const bool mine = slot >= 0 && (mode == 1 || eval_class(d.code_jumps[slot], C) == 2);
-    LoopPart t{0, 0, 0, 0, 0, 0};
-    for (int q = part; mine && q < groups; q += 16) {
-      const LoopPart x = d.loop_part[std::size_t(slot) * tiles + q];
-      t.sum += x.sum; t.fuel += x.fuel;
-      t.wrong += x.wrong; t.errors += x.errors; t.timeouts += x.timeouts; t.fractional |= x.fractional;
+    LoopAcc t{0, 0, 0, 0, 0, 0};
+    if (mine && part == 0) {
+      GAS LoopAcc* const acc = d.loop_acc + slot;
+      t.sum = acc->sum; t.fuel = acc->fuel;
+      t.wrong = acc->wrong; t.errors = acc->errors; t.timeouts = acc->timeouts; t.fractional = acc->fractional;
+      acc->sum = acc->fuel = 0;
+      acc->wrong = acc->errors = acc->timeouts = acc->fractional = 0;
     }
-    for (int off = 8; off > 0; off >>= 1) {
-      t.sum += __shfl_xor(t.sum, off, 64); t.fuel += __shfl_xor(t.fuel, off, 64);
-      t.wrong += __shfl_xor(t.wrong, off, 64); t.errors += __shfl_xor(t.errors, off, 64);
-      t.timeouts += __shfl_xor(t.timeouts, off, 64); t.fractional |= __shfl_xor(t.fractional, off, 64);
-    }
-    double fitness = double(t.sum);
+    double fitness = double((long long)t.sum);
     for (unsigned long long m = __ballot(mine && part == 0 && t.fractional); m; m &= m - 1) {
       const int from = wave_first(m);
       const double total = canonical_from_scores(e, C, d.loop_scores + std::size_t(rdlane(slot, from)) * C, lane, replay[wave_index()]);
@@ -2002,8 +2008,9 @@ struct SearchState {
     arena.next_chunk = count.bytes;
     d = build(arena);
   }
-  // Device bytes the search holds once allocated (its arena's chunks),
-  // computed without allocating.
+  // Device bytes the search is admitted by: its arrays in chunks doubling from
+  // 1 MiB, never less than the one block they are allocated as; computed
+  // without allocating.
   std::size_t planned_bytes() const {
     DeviceArena count(true);
     (void)build(count);
@@ -2070,11 +2077,10 @@ struct SearchState {
     x.cd = dc.cd;
     const std::size_t slots = std::size_t(std::max(P, B));
     if (x.cd.C <= kScoreCases) x.loop_scores = a.alloc<double>(slots * std::size_t(x.cd.C));
-    if (x.cd.C <= kScoreCases && may_jump) {
-      x.loop_part = a.alloc<LoopPart>(slots * std::size_t((x.cd.C + 63) / 64));
-      x.step_cap = std::min(x.code_cap, kStepMax);
-      x.steps = a.alloc<Step>(slots * std::size_t(x.step_cap));
-      x.step_n = a.alloc<int>(slots);
+    x.looping = x.cd.C <= kScoreCases && may_jump;
+    if (x.looping) {
+      x.loop_acc = a.alloc<LoopAcc>(slots);
+      a.zero(x.loop_acc, slots);
     }
     const std::size_t rows = std::size_t(P) * R, crows = std::size_t(B) * R;
     x.cur_origin = a.alloc<int>(rows); x.cur_site = a.alloc<int>(rows); x.cur_cval = a.alloc<Val>(rows);
@@ -2319,11 +2325,11 @@ struct Batch::Impl {
   }
   Grid finish_grid(DeviceArena& arena, const std::vector<int>& table, bool members) {
     return build_grid(arena, table, [&](const SearchState& s) {
-      return s.may_jump && s.d.cd.C > 64 && s.d.cd.C <= kScoreCases ? up(members ? s.P : s.B, kFinishPrograms) : 0;
+      return s.d.looping && s.d.cd.C > 64 ? up(members ? s.P : s.B, kFinishPrograms) : 0;
     });
   }
   Grid loop_grid(DeviceArena& arena, int group) {
-    return build_grid(arena, live, [&](const SearchState& s) { return s.may_jump && s.d.steps ? loop_blocks(s.d.cd.C, s.B, group) : 0; });
+    return build_grid(arena, live, [&](const SearchState& s) { return s.d.looping ? loop_blocks(s.d.cd.C, s.B, group) : 0; });
   }
 
   // Allocates one search and fixes its kernel variants and LDS needs.
@@ -2451,7 +2457,7 @@ struct Batch::Impl {
       });
     if (any_jumps(ids))
       timer.time("k_eval_init_loop", stream, [&] {
-        const Grid gp = build_grid(tmp, ids, [&](const SearchState& x) { return x.may_jump && x.d.steps ? loop_blocks(x.d.cd.C, x.P) : 0; });
+        const Grid gp = build_grid(tmp, ids, [&](const SearchState& x) { return x.d.looping ? loop_blocks(x.d.cd.C, x.P) : 0; });
         if (gp.blocks) hipLaunchKernelGGL(k_eval_loop<false>, dim3(gp.blocks), dim3(64), eval_loop_lds, stream, t, gp.map, 0, 1);
         const Grid gf = finish_grid(tmp, ids, true);
         if (gf.blocks) hipLaunchKernelGGL(k_loop_finish, dim3(gf.blocks), dim3(kEvalThreads), 0, stream, t, gf.map, 0, 1);
@@ -2522,9 +2528,9 @@ struct Batch::Impl {
   // Measures the evaluation kernels over the current round's pending
   // programs under each candidate launch shape and keeps the fastest.
   // Re-running an evaluation kernel over the same pending list rewrites the
-  // same results (each program's fitness, wrong count and tallies; the
-  // looping kernel's per-program totals are cleared by the program's last
-  // item), so tuning changes no search. Call between enqueue_front and
+  // same results (each program's fitness, wrong count and tallies; k_loop_finish
+  // takes the looping kernel's totals after every launch), so tuning changes no
+  // search. Call between enqueue_front and
   // enqueue_eval of a round, with the stream idle.
   void tune_launches() {
     const std::string key = shape_key();
@@ -2554,12 +2560,14 @@ struct Batch::Impl {
     // The first candidate of each kernel runs twice (its first launch warms
     // code and caches), every other candidate once.
     int reps = 2;
-    const auto measure = [&](auto launch) {
+    // `after`, not timed, follows every launch.
+    const auto measure = [&](auto launch, auto after) {
       float best = 1e30f;
       for (int rep = 0; rep < reps; ++rep) {
         HIP_OK(hipEventRecord(a, stream));
         launch();
         HIP_OK(hipEventRecord(b, stream));
+        after();
         HIP_OK(hipEventSynchronize(b));
         float ms = 0;
         HIP_OK(hipEventElapsedTime(&ms, a, b));
@@ -2594,7 +2602,7 @@ struct Batch::Impl {
       const Grid g = typed_grid(tmp, k);
       return g.blocks ? measure([&] {
         hipLaunchKernelGGL(k_eval<1>, dim3(g.blocks), dim3(kEvalThreads), eval_fast_lds, stream, d_all, g.map, 1);
-      }) : 0.f;
+      }, [] {}) : 0.f;
     });
     if (loop_kernel) {
       choice.loop_group = pick("loop", {1, 2, 4}, [&](int group) {
@@ -2605,6 +2613,8 @@ struct Batch::Impl {
             hipLaunchKernelGGL(k_eval_loop<false>, dim3(g.blocks), dim3(64), eval_loop_lds, stream, d_all, g.map, 1, 1);
           else
             hipLaunchKernelGGL(k_eval_loop<true>, dim3(g.blocks), dim3(64), eval_loop_lds, stream, d_all, g.map, 1, group);
+        }, [&] {
+          if (g_finish.blocks) hipLaunchKernelGGL(k_loop_finish, dim3(g_finish.blocks), dim3(kEvalThreads), 0, stream, d_all, g_finish.map, 1, group);
         }) : 0.f;
       });
     }

@@ -55,6 +55,30 @@ struct alignas(16) Step {
 static_assert(sizeof(Step) == 16, "a step is one 16-byte load");
 constexpr std::uint32_t kStepPush = 1u << 6, kStepX = 1u << 7, kStepPop = 1u << 13;
 constexpr int kStepMax = kLoopCode;  // steps of a program: at most one per instruction
+// A step in 8 bytes, as a search keeps it where the instructions were: the
+// constant by its pool index (or a WALK_NEXT's direction) in w0 [23:16], which
+// a step leaves free; a WALK_TEST's three further slots and direction in w0
+// [21:6]. Kept beside the code at 16 bytes each, a search of 8192 list programs
+// asked for 164 MB instead of 144, and a server refused some it had admitted.
+// Reading them takes a second round trip, for the constants: k_eval_loop on
+// 4096 list programs x 200 cases 440 and 453 us.
+static_assert(sizeof(Ins) == sizeof(std::uint64_t) && kLoopPool <= 256, "a packed step replaces an instruction");
+STEP_FN std::uint64_t pack_step(const Step& s) {
+  const unsigned c = unsigned(std::uint64_t(s.c));
+  const unsigned more = (s.w0 & 63u) == unsigned(SO_WALK_TEST) ? (c & 31u) << 6 | (c >> 8 & 31u) << 11 | (c >> 16 & 31u) << 16 | (c >> 24 & 1u) << 21
+                                                               : (c & 0xffu) << 16;
+  return std::uint64_t(s.w1) << 32 | (s.w0 | more);
+}
+// The step again, a constant still its pool index.
+STEP_FN Step unpack_step(std::uint64_t word) {
+  const unsigned lo = unsigned(word);
+  const bool walk = (lo & 63u) == unsigned(SO_WALK_TEST);
+  const unsigned c = walk ? (lo >> 6 & 31u) | (lo >> 11 & 31u) << 8 | (lo >> 16 & 31u) << 16 | (lo >> 21 & 1u) << 24 : lo >> 16 & 0xffu;
+  return Step{lo & (walk ? 0xff00003fu : 0xff00ffffu), unsigned(word >> 32), std::int64_t(c)};
+}
+// Whether an unpacked step's constant is a pool index.
+STEP_FN bool step_indexes(const Step& s) { return (s.w0 & 63u) < unsigned(kStepControl) && (s.w0 >> 8 & 3u) == 2; }
+STEP_FN std::int64_t pool_payload(const Val& v) { return v.tag == TAG_BOOL ? std::int64_t(v.b != 0) : v.i; }
 
 // Slots of a lane: the evaluator inputs, the hidden locals, then the operand
 // stack's elements below the register top.
@@ -111,8 +135,7 @@ STEP_FN bool jump_op(int op) { return op == OP_JMP || op == OP_JMP_IF_FALSE || o
 struct StepSource {
   const Ins* code;
   int len;
-  const Val* pool;
-  const std::int64_t* values;  // the pool's payloads (a Bool's flag), where the caller has them, else null
+  const Val* pool;  // null: a step's constant is the pool index
   int n_inputs;
   bool tagged;
   CodeBits target;    // instructions some jump enters
@@ -217,9 +240,7 @@ STEP_FN Step step_at(const StepSource& s, int j, const CodeBits& starts, int n) 
   const auto element = [&](int k) { return unsigned(stack + (k < 0 ? 0 : k < kStepStack ? k : kStepStack - 1)); };
   const auto step_of = [&](int t) { return unsigned(t >= s.len ? n : starts.below(t)); };
   const auto constant = [&](const Ins& x) {
-    if (s.values) return s.values[x.a];
-    const Val v = s.pool[x.a];
-    return v.tag == TAG_BOOL ? std::int64_t(v.b != 0) : v.i;
+    return s.pool ? pool_payload(s.pool[x.a]) : std::int64_t(x.a);
   };
   const auto pack = [](unsigned op, unsigned flags, unsigned y, unsigned sink, unsigned loads, unsigned cost) {
     return op | flags | y << 8 | sink << 10 | loads << 14 | cost << 24;
@@ -354,7 +375,7 @@ STEP_FN Step step_at(const StepSource& s, int j, const CodeBits& starts, int n) 
 // Host decoding of a certified looping program of at most kLoopCode
 // instructions; returns the number of steps written.
 inline int decode_steps(const Ins* code, int len, const Val* pool, int n_inputs, bool tagged, Step* out) {
-  StepSource s{code, len, pool, nullptr, n_inputs, tagged, {{0, 0, 0, 0}}, {{0, 0, 0, 0}}};
+  StepSource s{code, len, pool, n_inputs, tagged, {{0, 0, 0, 0}}, {{0, 0, 0, 0}}};
   for (int i = 0; i < len; ++i) {
     if (jump_op(code[i].op)) s.target.set(code[i].a, 1);
     if (tagged && !s.sequence.at(i) && sequence_length(code[i])) s.sequence.set(i, sequence_length(code[i]));
@@ -369,11 +390,12 @@ inline int decode_steps(const Ins* code, int len, const Val* pool, int n_inputs,
 }
 
 #if defined(__HIPCC__)
-// The same by one wavefront, a lane per instruction.
-__device__ __attribute__((always_inline)) inline int decode_steps_w(const Ins* code, int len, const Val* pool, const std::int64_t* values,
-                                                                        int n_inputs, Step* out) {
+// Lowered code to packed steps by one wavefront, a lane per instruction.
+// `out` may be the code itself: the steps of 64 instructions are stored when
+// every lane has them, and replace none that a later one reads.
+__device__ __attribute__((always_inline)) inline int decode_steps_w(const Ins* code, int len, int n_inputs, std::uint64_t* out) {
   const int lane = int(threadIdx.x & 63u);
-  StepSource s{code, len, pool, values, n_inputs, true, {{0, 0, 0, 0}}, {{0, 0, 0, 0}}};
+  StepSource s{code, len, nullptr, n_inputs, true, {{0, 0, 0, 0}}, {{0, 0, 0, 0}}};
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
     if (64 * g >= len) break;
@@ -400,7 +422,11 @@ __device__ __attribute__((always_inline)) inline int decode_steps_w(const Ins* c
   for (int g = 0; g < 4; ++g) {
     if (64 * g >= len) break;
     const int j = 64 * g + lane;
-    if (j < len && starts.at(j)) out[starts.below(j)] = step_at(s, j, starts, n);
+    const bool mine = j < len && starts.at(j);
+    const std::uint64_t word = mine ? pack_step(step_at(s, j, starts, n)) : 0;
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    if (mine) out[starts.below(j)] = word;
   }
   return n;
 }

@@ -25,12 +25,11 @@ namespace gagp_amd {
 constexpr int kWaveRow = 64;
 constexpr int kLaneValues = 64;  // pool entries of a program lowered with jumps
 // LDS of a wavefront that lowers rows: exchange words and, with jumps, the
-// program, which is decoded from here and stored in order.
+// program, which the caller decodes from here or stores in order.
 template <bool kJumps> struct LaneStore { int sums[64]; };
 template <> struct LaneStore<true> {
   int sums[64];
   Ins code[kLoopCode];
-  std::int64_t values[kLaneValues];  // payloads, a Bool's flag
 };
 
 // ---- wavefront reductions and scans in the data-parallel shifts (all lanes active) ----
@@ -416,7 +415,7 @@ __device__ inline std::uint64_t row_hash_row(const WaveRow& r) {
 // the grammar declares; the node-by-node lowering then decides.
 // kJumps: all kinds; otherwise constants, inputs and operations only.
 // A statement row has been checked for definite assignment. `store`: this
-// wavefront's LDS, which keeps the code and the pool's payloads (kJumps).
+// wavefront's LDS, which alone has the code with kJumps.
 // Node by node a child took 1.2 us a node, and 75-100 us with traversals; a
 // row takes 3 us here, 6 with jumps. The program stays in LDS for the decoding,
 // which read its neighbours' words from global memory in 20 us and takes half.
@@ -652,7 +651,6 @@ __device__ inline bool lower_row(const WaveGrammar& w, const WaveRow& r, GAS con
     else *(GAS std::uint64_t*)(code + to) = word;
   };
   const auto put_value = [&](int to, std::uint64_t v, unsigned tag, unsigned flag) {
-    if constexpr (kJumps) store->values[to] = std::int64_t(tag == unsigned(TAG_BOOL) ? flag : v);
     pool[to].i = std::int64_t(v);
     *(GAS std::uint64_t*)(&pool[to].b) = std::uint64_t(flag) | std::uint64_t(tag) << 8;
   };
@@ -804,10 +802,7 @@ __device__ inline bool lower_row(const WaveGrammar& w, const WaveRow& r, GAS con
     }
   }
   if (!statement && lane == 0) put(words - 1, OP_RETURN, 0, 1, 1, 0);
-  if constexpr (kJumps) {
-    lanes_meet();
-    for (int k = lane; k < words; k += 64) *(GAS std::uint64_t*)(code + k) = *(LAS std::uint64_t*)(store->code + k);
-  }
+  lanes_meet();
   const bool straight = __ballot(live && (!fast || branch || logic || walk || bind || let)) == 0 && !statement;
   const bool few = local_count <= kFastInputs;
   const int value = statement ? returned : root;

@@ -601,6 +601,12 @@ struct StepProgram {
   unsigned w0[4], w1[4], c0[4], c1[4];
   int n;
 };
+__device__ inline void steps_hold(StepProgram& f, int g, const Step& s) {
+  f.w0[g] = s.w0;
+  f.w1[g] = s.w1;
+  f.c0[g] = unsigned(std::uint64_t(s.c));
+  f.c1[g] = unsigned(std::uint64_t(s.c) >> 32);
+}
 __device__ inline StepProgram steps_load(GAS const Step* steps, int n, int lane) {
   StepProgram f;
   f.n = n;
@@ -613,10 +619,26 @@ __device__ inline StepProgram steps_load(GAS const Step* steps, int n, int lane)
       s.w1 = steps[j].w1;
       s.c = steps[j].c;
     }
-    f.w0[g] = s.w0;
-    f.w1[g] = s.w1;
-    f.c0[g] = unsigned(std::uint64_t(s.c));
-    f.c1[g] = unsigned(std::uint64_t(s.c) >> 32);
+    steps_hold(f, g, s);
+  }
+  return f;
+}
+// Packed steps and the constants they index: two round trips instead of one,
+// once per item of 64 cases.
+__device__ inline StepProgram steps_load(GAS const std::uint64_t* words, GAS const Val* pool, int n, int lane) {
+  StepProgram f;
+  f.n = n;
+  std::uint64_t word[4];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) word[g] = g * 64 + lane < n ? words[g * 64 + lane] : 0;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    Step s = unpack_step(word[g]);
+    if (step_indexes(s)) {  // never of an absent step: its word names no constant
+      GAS const Val* const v = pool + s.c;
+      s.c = v->tag == TAG_BOOL ? std::int64_t(v->b != 0) : v->i;
+    }
+    steps_hold(f, g, s);
   }
   return f;
 }

@@ -2,8 +2,8 @@
 // on one lane (tests/one_lane), with cases that leave inputs unset.
 //
 //   looping_vm TASK.json N
-//     lowers and decodes N seeded random programs of the task's grammar, runs
-//     every train case with every subset of the inputs unset, at the task's
+//     lowers and decodes N seeded random programs of the task's grammar, packs
+//     and unpacks their steps, runs every train case with every subset of the inputs unset, at the task's
 //     fuel and on a few cases at every small fuel, and compares value, error
 //     and charged fuel with the C oracle VM on the bytecode.
 //   looping_vm division
@@ -100,7 +100,7 @@ int main(int argc, char** argv) {
   std::vector<Val> pool(std::size_t(8 * R + 16));
   std::vector<std::int64_t> slots(std::size_t(64 * step_slots(K)));
   long long compared = 0, mismatches = 0, errors[5] = {0, 0, 0, 0, 0};
-  int programs = 0;
+  int programs = 0, repacked = 0;
   for (int i = 0; i < n; ++i) {
     GenResult gen{ST_INVALID, 0, 0, 0};
     for (int attempt = 0; gen.status != ST_OK && attempt < 64; ++attempt) {
@@ -124,7 +124,15 @@ int main(int argc, char** argv) {
       fuel.push_back(x.fuel);
     }
     const OProg p{oc.data(), std::int32_t(oc.size()), fuel.data(), pool.data(), lr.constants, lr.locals};
-    program_of_lane.n = decode_steps(code.data(), lr.code, pool.data(), K, true, steps_of_lane);
+    // The steps as a search keeps them: packed, the constants by pool index.
+    program_of_lane.n = decode_steps(code.data(), lr.code, nullptr, K, true, steps_of_lane);
+    for (int k = 0; k < program_of_lane.n; ++k) {
+      Step& s = steps_of_lane[k];
+      const Step again = unpack_step(pack_step(s));
+      repacked += again.w0 != s.w0 || again.w1 != s.w1 || again.c != s.c;
+      s = again;
+      if (step_indexes(s)) s.c = pool_payload(pool[std::size_t(s.c)]);
+    }
     for (int c = 0; c < cases.n; ++c)
       for (unsigned bound = 0; bound < 1u << K; ++bound) {
         std::uint8_t set[kFastInputs] = {};
@@ -151,7 +159,7 @@ int main(int argc, char** argv) {
         }
       }
   }
-  std::printf("{\"compared\":%lld,\"mismatches\":%lld,\"programs\":%d,\"errors\":[%lld,%lld,%lld,%lld,%lld]}\n", compared, mismatches, programs,
-              errors[0], errors[1], errors[2], errors[3], errors[4]);
+  std::printf("{\"compared\":%lld,\"mismatches\":%lld,\"programs\":%d,\"repacked\":%d,\"errors\":[%lld,%lld,%lld,%lld,%lld]}\n", compared, mismatches, programs,
+              repacked, errors[0], errors[1], errors[2], errors[3], errors[4]);
   return 0;
 }

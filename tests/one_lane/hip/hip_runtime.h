@@ -25,3 +25,5 @@ static double reciprocal_error = 0;
 #define __builtin_amdgcn_readlane(x, lane) ((void)(lane), (x))
 #define __builtin_amdgcn_readfirstlane(x) (x)
 #define __builtin_amdgcn_update_dpp(old, x, control, rows, banks, bound) ((void)(x), (old))  // no lane beside this one
+#define __builtin_amdgcn_fence(order, scope) ((void)0)
+#define __builtin_amdgcn_wave_barrier() ((void)0)

@@ -1,6 +1,7 @@
 """The looping path's VM on the host (CPU): tests/looping_vm.cpp compiles
 vm_steps itself for one lane and compares value, error and charged fuel with
-the C oracle VM on the bytecode, for seeded random programs, with every subset
+the C oracle VM on the bytecode, for seeded random programs whose steps
+were packed and unpacked, with every subset
 of the inputs unset, at the task's fuel and at small ones; and its division
 with the host's at the edges of the 32-bit path, with the reciprocal off by
 2^-23 either way. Integers and error codes: equality."""
@@ -35,7 +36,7 @@ def test_unset_inputs_match_the_bytecode(driver, task, n):
     r = json.loads(out.stdout)
     assert r["programs"] >= 50 and r["compared"] > 10000
     assert r["errors"][0] > 1000  # cases that read an unset input
-    assert r["mismatches"] == 0
+    assert r["mismatches"] == 0 and r["repacked"] == 0
 
 
 def test_division_at_its_edges(driver):
