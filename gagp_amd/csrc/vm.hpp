@@ -588,12 +588,17 @@ __device__ inline LaneResult vm_fast(const FastProgram& f, const FastInputs& in,
 // j / 64 and is read with readlane, so a fetch costs no memory round trip.
 //
 // Lanes follow their own branches. The lanes at the smallest step index run
-// together as a group under the execution mask: inside a run the step index,
-// the decoded fields and the fuel charged are scalar, no operation is
-// predicated, and fuel is checked against the group's smallest balance by one
-// scalar compare. A run ends where the group's lanes part, a lane finishes,
-// or the group reaches the step at which other lanes wait; only there are the
-// per-lane indexes and balances written and the next group chosen.
+// together as a group: inside a run the step index, the decoded fields and the
+// fuel charged are scalar, and fuel is checked against the group's smallest
+// balance by one scalar compare. A run ends where the group's lanes part, a
+// lane finishes, or the group reaches the step at which other lanes wait; only
+// there are the per-lane indexes and balances written and the next group
+// chosen. Every lane computes; what it keeps (the top, slots, a list element)
+// is selected by the group's mask. Under the mask as execution mask the steps
+// would be read from registers whose other lanes the compiler may drop in any
+// copy or spill it makes there; so it was, with none made by chance. The
+// selects cost k_eval_loop 3% on 4096 list programs x 200 cases (453 to 468 us)
+// and 7% on 1500 statement programs x 130 (475 to 511).
 // Interpreting the bytecode itself, predicated and one instruction (or fixed
 // sequence) at a time, issued about 31 vector and 40 scalar instructions per
 // step and three times the steps; k_eval_loop has the measured times.
@@ -673,8 +678,8 @@ __device__ inline int wave_min_all(int x) {
 // `slots`: this wave's LDS area of step_slots(n_inputs) slots (slot k of lane
 // j at k * 64 + j). kGroups: register groups that hold the program's steps.
 // The run loop is one nest of two-way uniform branches with a single exit (no
-// switch, break or continue) and no divergent branch: what a lane records when
-// it ends is written after the loop, from the event that ended it. In this
+// switch, break or continue) and no divergent branch but a lane's stores: what a
+// lane records when it ends is written after the loop, from the event that ended it. In this
 // form the compiler keeps the step index, the fields, the balances and the
 // event in scalar registers and only the stack's top in vector ones; any
 // per-lane record merged inside the loop would be copied on every path of
@@ -723,6 +728,9 @@ __device__ inline LaneResult vm_steps(const StepProgram& f, const FastInputs& in
       continue;
     }
     const bool mine = !done && ip == at;
+    const auto store = [&](int slot, std::int64_t v) {
+      if (mine) sl[slot * 64] = v;
+    };
     int budget = low;
     if (low < kMost) {
       // Near exhaustion the group takes one step at a time. Lanes that cannot
@@ -758,158 +766,157 @@ __device__ inline LaneResult vm_steps(const StepProgram& f, const FastInputs& in
         budget = wave_min_all(mine ? fuel : kNone);
       }
     }
-    int charged = 0;
     budget = __builtin_amdgcn_readfirstlane(budget);
-    if (mine) {
-      // Here ip == at, and the compiler may take the lane's value for both.
-      at = __builtin_amdgcn_readfirstlane(at);
-      int spent = 0, event = EV_NONE, last = at;
-      unsigned long long mask = 0;  // the lanes an event names
-      unsigned sink_slot = kStepNoSlot;
-      do {
-        const unsigned w0 = step_word<kGroups>(f.w0, at), w1 = step_word<kGroups>(f.w1, at);
-        const int op = int(w0 & 63u), cost = int(w0 >> 24);
-        budget -= cost;
-        spent += cost;
-        const int a = int(w1 & 31u), b = int((w1 >> 5) & 31u), p = int((w1 >> 10) & 31u), target = int(w1 >> 16);
-        int next = at + 1;
-        if (op < kStepControl) {
-          std::int64_t x = top, y = top;
-          if (w0 & kStepPush) sl[p * 64] = top;
-          if (w0 & kStepX) x = sl[a * 64];
-          const unsigned yk = (w0 >> 8) & 3u, sink = (w0 >> 10) & 7u;
-          if (yk == 2) y = std::int64_t(std::uint64_t(step_word<kGroups>(f.c1, at)) << 32 | step_word<kGroups>(f.c0, at));
-          else if (yk == 1) y = sl[b * 64];
-          unsigned long long holds = 0;
-          std::int64_t out = y;
-          if (op >= kStepBool) {
-            if (op < SO_GT) {
-              if (op < SO_LT) holds = op == SO_TEST ? __ballot(x != 0) : __ballot(x == 0);
-              else if (op == SO_LT) holds = __ballot(x < y);
-              else holds = __ballot(x <= y);
-            } else {
-              if (op < SO_EQ) {
-                if (op == SO_GT) holds = __ballot(x > y);
-                else holds = __ballot(x >= y);
-              } else {
-                if (op == SO_EQ) holds = __ballot(x == y);
-                else holds = __ballot(x != y);
-              }
-            }
-            out = std::int64_t((holds >> lane) & 1u);
-          } else if (op < SO_MIN) {
-            if (op < SO_SUB) {
-              if (op == SO_ADD) out = wrap_add(x, y);
-            } else {
-              if (op == SO_SUB) out = wrap_sub(x, y);
-              else out = wrap_mul(x, y);
-            }
-          } else if (op < SO_INDEX) {
-            if (op < SO_MOD) {
-              if (op == SO_MIN) out = x < y ? x : y;
-              else out = x > y ? x : y;
-            } else {
-              out = step_divide(op, x, y);
-              mask = op == SO_MOD ? __ballot(y == 0) : 0;
-              event = mask != 0 ? EV_ZERO_DIV : EV_NONE;
-            }
-          } else if (op < SO_NEG) {
-            // List indexing, as in vm_run. Only a valid index is read; the
-            // rest read the arena's first element (it is never empty).
-            const std::int64_t n = std::int64_t(std::uint64_t(x) & 0xffff);
-            const bool clamped = op == SO_INDEX_CLAMPED;  // an empty list reads as 0
-            const bool negative = op == SO_INDEX_NONNEG && y < 0;
-            const std::int64_t inside = y < 0 ? 0 : y >= n ? n - 1 : y, wrapped = y < 0 ? y + n : y;
-            const std::int64_t k = clamped ? inside : wrapped;
-            const bool ok = !negative && k >= 0 && k < n;
-            const std::int64_t v = arena[ok ? (std::uint64_t(x) >> 16) + std::uint64_t(k) : 0];
-            out = ok ? v : 0;
-            mask = clamped ? 0 : __ballot(!ok);
-            event = mask != 0 ? EV_VALUE : EV_NONE;
-          } else if (op < SO_LEN) {
-            out = op == SO_NEG || x < 0 ? wrap_neg(x) : x;  // NEG, ABS
-          } else if (op < SO_CLIP) {
-            out = op == SO_LEN ? std::int64_t(std::uint64_t(x) & 0xffff) : 1;
+    const unsigned long long group = __ballot(mine);
+    int spent = 0, event = EV_NONE, last = at;
+    unsigned long long mask = 0;  // the lanes an event names
+    unsigned sink_slot = kStepNoSlot;
+    do {
+      const unsigned w0 = step_word<kGroups>(f.w0, at), w1 = step_word<kGroups>(f.w1, at);
+      const int op = int(w0 & 63u), cost = int(w0 >> 24);
+      budget -= cost;
+      spent += cost;
+      const int a = int(w1 & 31u), b = int((w1 >> 5) & 31u), p = int((w1 >> 10) & 31u), target = int(w1 >> 16);
+      int next = at + 1;
+      if (op < kStepControl) {
+        std::int64_t x = top, y = top;
+        if (w0 & kStepPush) store(p, top);
+        if (w0 & kStepX) x = sl[a * 64];
+        const unsigned yk = (w0 >> 8) & 3u, sink = (w0 >> 10) & 7u;
+        if (yk == 2) y = std::int64_t(std::uint64_t(step_word<kGroups>(f.c1, at)) << 32 | step_word<kGroups>(f.c0, at));
+        else if (yk == 1) y = sl[b * 64];
+        unsigned long long holds = 0;
+        std::int64_t out = y;
+        if (op >= kStepBool) {
+          if (op < SO_GT) {
+            if (op < SO_LT) holds = op == SO_TEST ? __ballot(x != 0) : __ballot(x == 0);
+            else if (op == SO_LT) holds = __ballot(x < y);
+            else holds = __ballot(x <= y);
           } else {
-            const std::int64_t m = x > y ? x : y;
-            out = m < top ? m : top;
-          }
-          if (sink < SK_IF_FALSE) {
-            top = out;
-            next = sink == SK_TOP_JUMP ? target : next;
-          } else {
-            if (sink == SK_STORE) {
-              sl[target * 64] = out;
-              sink_slot = unsigned(target);
+            if (op < SO_EQ) {
+              if (op == SO_GT) holds = __ballot(x > y);
+              else holds = __ballot(x >= y);
             } else {
-              const unsigned long long group = __ballot(true), jumps = sink == SK_IF_TRUE ? holds : group & ~holds;
-              mask = jumps;
-              event = jumps != 0 && jumps != group ? EV_BRANCH : EV_NONE;
-              next = jumps == group ? target : next;
+              if (op == SO_EQ) holds = __ballot(x == y);
+              else holds = __ballot(x != y);
             }
-            if (w0 & kStepPop) top = sl[p * 64];
           }
-        } else if (op < SO_WALK_TEST) {
-          event = op == SO_JUMP ? EV_NONE : EV_RETURN;
-          next = target;
-        } else if (op < SO_RANGE_TEST) {
-          if (op == SO_WALK_NEXT) {
-            sl[a * 64] = top;
-            if (w0 & kStepPop) top = sl[p * 64];
-            const std::int64_t counter = sl[b * 64];
-            sl[b * 64] = wrap_add(counter, step_word<kGroups>(f.c0, at) ? -1 : 1);
-            next = target;
+          out = std::int64_t((holds >> lane) & 1u);
+        } else if (op < SO_MIN) {
+          if (op < SO_SUB) {
+            if (op == SO_ADD) out = wrap_add(x, y);
           } else {
-            // A loop's test: leaving it charges four units. Leaving lanes
-            // bind the arena's first element, which nothing reads.
-            const unsigned c0 = step_word<kGroups>(f.c0, at);
-            const std::int64_t counter = sl[a * 64], limit = sl[b * 64], xs = sl[p * 64], start = sl[((c0 >> 8) & 31u) * 64];
-            const bool more = (c0 >> 24) != 0 ? counter >= limit : counter < limit;
-            const unsigned long long stay = __ballot(more), group = __ballot(true);
-            // The counter of a staying lane lies in [0, length).
-            sl[(c0 & 31u) * 64] = arena[more ? (std::uint64_t(xs) >> 16) + std::uint64_t(counter) : 0];
-            sl[((c0 >> 16) & 31u) * 64] = wrap_add(start, counter);
-            mask = stay;
-            event = stay != 0 && stay != group ? EV_TEST : EV_NONE;
-            next = stay == 0 ? target : next;
-            const int refund = stay == 0 ? cost - 4 : 0;
-            budget += refund;
-            spent -= refund;
+            if (op == SO_SUB) out = wrap_sub(x, y);
+            else out = wrap_mul(x, y);
           }
-        } else if (op < SO_FAIL_TYPE) {
-          const std::int64_t counter = sl[a * 64];
-          if (op == SO_RANGE_NEXT) {
-            sl[a * 64] = wrap_add(counter, 1);
-            next = target;
+        } else if (op < SO_INDEX) {
+          if (op < SO_MOD) {
+            if (op == SO_MIN) out = x < y ? x : y;
+            else out = x > y ? x : y;
           } else {
-            // Leaving lanes keep the variable, and an unset input unset.
-            const std::int64_t limit = sl[b * 64], old = sl[p * 64];
-            const bool more = counter < limit;
-            const unsigned long long stay = __ballot(more), group = __ballot(true);
-            sl[p * 64] = more ? counter : old;
-            sink_slot = stay != 0 ? unsigned(p) : kStepNoSlot;
-            mask = stay;
-            event = stay != 0 && stay != group ? EV_TEST : EV_NONE;
-            next = stay == 0 ? target : next;
-            const int refund = stay == 0 ? cost - 4 : 0;
-            budget += refund;
-            spent -= refund;
+            out = step_divide(op, mine ? x : 0, mine ? y : 1);
+            mask = op == SO_MOD ? __ballot(y == 0) & group : 0;
+            event = mask != 0 ? EV_ZERO_DIV : EV_NONE;
           }
+        } else if (op < SO_NEG) {
+          // List indexing, as in vm_run. Only a valid index is read; the
+          // rest read the arena's first element (it is never empty).
+          const std::int64_t n = std::int64_t(std::uint64_t(x) & 0xffff);
+          const bool clamped = op == SO_INDEX_CLAMPED;  // an empty list reads as 0
+          const bool negative = op == SO_INDEX_NONNEG && y < 0;
+          const std::int64_t inside = y < 0 ? 0 : y >= n ? n - 1 : y, wrapped = y < 0 ? y + n : y;
+          const std::int64_t k = clamped ? inside : wrapped;
+          const bool ok = mine && !negative && k >= 0 && k < n;
+          const std::int64_t v = arena[ok ? (std::uint64_t(x) >> 16) + std::uint64_t(k) : 0];
+          out = ok ? v : 0;
+          mask = clamped ? 0 : group & ~__ballot(ok);
+          event = mask != 0 ? EV_VALUE : EV_NONE;
+        } else if (op < SO_LEN) {
+          out = op == SO_NEG || x < 0 ? wrap_neg(x) : x;  // NEG, ABS
+        } else if (op < SO_CLIP) {
+          out = op == SO_LEN ? std::int64_t(std::uint64_t(x) & 0xffff) : 1;
         } else {
-          event = op == SO_FAIL_TYPE ? EV_FAIL_TYPE : EV_FAIL_VALUE;
+          const std::int64_t m = x > y ? x : y;
+          out = m < top ? m : top;
         }
-        last = at;
-        at = next;
-      } while (event == EV_NONE && at < stop && budget >= kMost);
-      // What ended the run.
-      const bool named = (mask >> lane) & 1u;
+        if (sink < SK_IF_FALSE) {
+          top = mine ? out : top;
+          next = sink == SK_TOP_JUMP ? target : next;
+        } else {
+          if (sink == SK_STORE) {
+            store(target, out);
+            sink_slot = unsigned(target);
+          } else {
+            const unsigned long long jumps = sink == SK_IF_TRUE ? holds & group : group & ~holds;
+            mask = jumps;
+            event = jumps != 0 && jumps != group ? EV_BRANCH : EV_NONE;
+            next = jumps == group ? target : next;
+          }
+          if (w0 & kStepPop) top = mine ? sl[p * 64] : top;
+        }
+      } else if (op < SO_WALK_TEST) {
+        event = op == SO_JUMP ? EV_NONE : EV_RETURN;
+        next = target;
+      } else if (op < SO_RANGE_TEST) {
+        if (op == SO_WALK_NEXT) {
+          store(a, top);
+          if (w0 & kStepPop) top = mine ? sl[p * 64] : top;
+          const std::int64_t counter = sl[b * 64];
+          store(b, wrap_add(counter, step_word<kGroups>(f.c0, at) ? -1 : 1));
+          next = target;
+        } else {
+          // A loop's test: leaving it charges four units. Leaving lanes
+          // bind the arena's first element, which nothing reads.
+          const unsigned c0 = step_word<kGroups>(f.c0, at);
+          const std::int64_t counter = sl[a * 64], limit = sl[b * 64], xs = sl[p * 64], start = sl[((c0 >> 8) & 31u) * 64];
+          const bool more = mine && ((c0 >> 24) != 0 ? counter >= limit : counter < limit);
+          const unsigned long long stay = __ballot(more);
+          // The counter of a staying lane lies in [0, length).
+          store(int(c0 & 31u), arena[more ? (std::uint64_t(xs) >> 16) + std::uint64_t(counter) : 0]);
+          store(int((c0 >> 16) & 31u), wrap_add(start, counter));
+          mask = stay;
+          event = stay != 0 && stay != group ? EV_TEST : EV_NONE;
+          next = stay == 0 ? target : next;
+          const int refund = stay == 0 ? cost - 4 : 0;
+          budget += refund;
+          spent -= refund;
+        }
+      } else if (op < SO_FAIL_TYPE) {
+        const std::int64_t counter = sl[a * 64];
+        if (op == SO_RANGE_NEXT) {
+          store(a, wrap_add(counter, 1));
+          next = target;
+        } else {
+          // Leaving lanes keep the variable, and an unset input unset.
+          const std::int64_t limit = sl[b * 64], old = sl[p * 64];
+          const bool more = mine && counter < limit;
+          const unsigned long long stay = __ballot(more);
+          store(p, more ? counter : old);
+          sink_slot = stay != 0 ? unsigned(p) : kStepNoSlot;
+          mask = stay;
+          event = stay != 0 && stay != group ? EV_TEST : EV_NONE;
+          next = stay == 0 ? target : next;
+          const int refund = stay == 0 ? cost - 4 : 0;
+          budget += refund;
+          spent -= refund;
+        }
+      } else {
+        event = op == SO_FAIL_TYPE ? EV_FAIL_TYPE : EV_FAIL_VALUE;
+      }
+      last = at;
+      at = next;
+    } while (event == EV_NONE && at < stop && budget >= kMost);
+    // What ended the run.
+    const bool named = (mask >> lane) & 1u;
+    const unsigned w0 = step_word<kGroups>(f.w0, last), w1 = step_word<kGroups>(f.w1, last);
+    const int target = int(w1 >> 16), refund = int(w0 >> 24) - 4;
+    if (mine) {
       ip = at;
       if (event == EV_BRANCH) {
-        ip = named ? int(step_word<kGroups>(f.w1, last) >> 16) : at;
+        ip = named ? target : at;
       } else if (event == EV_TEST) {
-        const unsigned w0 = step_word<kGroups>(f.w0, last);
-        ip = named ? at : int(step_word<kGroups>(f.w1, last) >> 16);
-        fuel += named ? 0 : int(w0 >> 24) - 4;
+        ip = named ? at : target;
+        fuel += named ? 0 : refund;
       } else if (event != EV_NONE) {
         const bool all = event >= EV_RETURN;
         if (all || named) {
@@ -926,10 +933,9 @@ __device__ inline LaneResult vm_steps(const StepProgram& f, const FastInputs& in
       }
       if (unbound && sink_slot < unsigned(n_inputs)) bound |= named || event != EV_TEST ? 1u << sink_slot : 0u;
       fuel -= spent;
-      charged = spent;
     }
     // No lane was charged more than the group.
-    low -= unbound ? 0 : __builtin_amdgcn_readlane(charged, __ffsll((long long)__ballot(mine)) - 1);
+    low -= unbound ? 0 : spent;
   }
   return r;
 }
