@@ -371,10 +371,14 @@ __device__ inline void pend_child(const DSearch& d, int c, int flags) {
 // the small lowering here covers). The node-by-node lowering of a traversal is
 // 75-100 us of dependent steps, and its registers in this kernel cost one more
 // wavefront per SIMD: 8192 children of a list grammar took 352 us with it, and
-// take 158 plus 8 for the launch that finds nothing to lower. At most 80 vector
-// registers, so six wavefronts per SIMD and not five.
+// take 150 plus 8 for the launch that finds nothing to lower. With kDefer at
+// most 80 vector registers and not 89, so six wavefronts per SIMD and not five,
+// for 8 or 9 values spilled to scratch: 150 us for 153 on those children, 154 for
+// 159 on 8192 of a statement grammar. Without, six took 93 us for 91 on 8192
+// children of the quintic grammar (9 and, for rows in memory, 28 values spilled),
+// so those keep their five.
 template <bool kStaged, bool kDefer>
-__global__ __launch_bounds__(64 * kVaryWaves) __attribute__((amdgpu_waves_per_eu(6))) void k_vary(DSearch* all, const BlockMap* map) {
+__global__ __launch_bounds__(64 * kVaryWaves) __attribute__((amdgpu_waves_per_eu(kDefer ? 6 : 5))) void k_vary(DSearch* all, const BlockMap* map) {
   const BlockMap bm = map[blockIdx.x];
   const DSearch& d = all[bm.search];
   if (!search_live(d) || (d.stage_tables != 0) != kStaged || (d.defer != 0) != kDefer) return;  // uniform per block
