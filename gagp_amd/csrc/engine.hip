@@ -1782,6 +1782,12 @@ __global__ __launch_bounds__(kEvalThreads) void k_eval_cases(DProg p, CaseData c
   }
 }
 
+// Lets a kernel take `bytes` of dynamic LDS. Without it a block has 64 KB in
+// all, of which no kernel here declares more than 30 KB beside them.
+void allow_lds(const void* kernel, std::size_t bytes) {
+  if (bytes > 32 * 1024) HIP_OK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)));
+}
+
 // ---- device buffers ----
 // Bump allocator over device chunks that double in size (1 MiB up to
 // 256 MiB): a search's arrays take a handful of hipMalloc calls in all.
@@ -2378,21 +2384,18 @@ struct Batch::Impl {
       max_slots = std::max(max_slots, x.d.stack_slots);
       max_table = std::max(max_table, x.d.table_mask + 1);
     }
-    const auto attr = [](const void* k, std::size_t bytes) {
-      if (bytes > 48 * 1024) HIP_OK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)));
-    };
-    attr(reinterpret_cast<const void*>(&k_init_pop<true>), vary_lds_bytes);
-    attr(reinterpret_cast<const void*>(&k_vary<true, false>), vary_lds_bytes);
-    attr(reinterpret_cast<const void*>(&k_vary<true, true>), vary_lds_bytes);
-    attr(reinterpret_cast<const void*>(&k_lower<false>), vary_lds_bytes);
-    attr(reinterpret_cast<const void*>(&k_lower<true>), vary_lds_bytes);
-    attr(reinterpret_cast<const void*>(&k_eval<0>), eval_general_lds);
-    attr(reinterpret_cast<const void*>(&k_eval<1>), eval_fast_lds);
-    attr(reinterpret_cast<const void*>(&k_eval_tiles), eval_tiles_lds);
-    attr(reinterpret_cast<const void*>(&k_eval_loop<false>), eval_loop_lds);
-    attr(reinterpret_cast<const void*>(&k_eval_loop<true>), eval_loop_lds);
-    attr(reinterpret_cast<const void*>(&k_place<true>), place_lds_bytes);
-    attr(reinterpret_cast<const void*>(&k_place<false>), place_hbm_bytes);
+    allow_lds(reinterpret_cast<const void*>(&k_init_pop<true>), vary_lds_bytes);
+    allow_lds(reinterpret_cast<const void*>(&k_vary<true, false>), vary_lds_bytes);
+    allow_lds(reinterpret_cast<const void*>(&k_vary<true, true>), vary_lds_bytes);
+    allow_lds(reinterpret_cast<const void*>(&k_lower<false>), vary_lds_bytes);
+    allow_lds(reinterpret_cast<const void*>(&k_lower<true>), vary_lds_bytes);
+    allow_lds(reinterpret_cast<const void*>(&k_eval<0>), eval_general_lds);
+    allow_lds(reinterpret_cast<const void*>(&k_eval<1>), eval_fast_lds);
+    allow_lds(reinterpret_cast<const void*>(&k_eval_tiles), eval_tiles_lds);
+    allow_lds(reinterpret_cast<const void*>(&k_eval_loop<false>), eval_loop_lds);
+    allow_lds(reinterpret_cast<const void*>(&k_eval_loop<true>), eval_loop_lds);
+    allow_lds(reinterpret_cast<const void*>(&k_place<true>), place_lds_bytes);
+    allow_lds(reinterpret_cast<const void*>(&k_place<false>), place_hbm_bytes);
   }
   // Builds and scores the initial populations of `ids` (not yet in the
   // round table) on the stream, through a table of their own.
@@ -3828,20 +3831,14 @@ void Session::Impl::launch(const PackedPrograms& k, const DProg* progs, const St
   const EvalParams e{I.cases.cd, I.fuel, I.lanes, I.penalty, I.policy};
   const std::size_t lds = std::size_t(kWavesPerBlock) * (k.slots + k.temps) * 64 * 10;
   const std::size_t fast_lds = std::size_t(kWavesPerBlock) * 8 * std::size_t(I.cases.cd.C);
-  if (k.any_general && lds > 65536)
-    HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_eval_programs<false>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                               int(lds)));
-  if (k.any_fast && fast_lds > 65536)
-    HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_eval_programs<true>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                               int(fast_lds)));
+  if (k.any_general) allow_lds(reinterpret_cast<const void*>(&k_eval_programs<false>), lds);
+  if (k.any_fast) allow_lds(reinterpret_cast<const void*>(&k_eval_programs<true>), fast_lds);
   const int blocks = std::min(4096, (n + kWavesPerBlock - 1) / kWavesPerBlock);
   if (const int loops = int(k.step_n.size())) {
     const int waves = std::min(kWavesPerBlock, (I.cases.cd.C + 63) / 64);
     const std::size_t step_lds =
         std::size_t(waves) * step_slots(I.cases.cd.n_inputs) * 64 * 8 + 8 * std::size_t(I.cases.cd.C);
-    if (step_lds > 65536)
-      HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_eval_steps), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                 int(step_lds)));
+    allow_lds(reinterpret_cast<const void*>(&k_eval_steps), step_lds);
     hipLaunchKernelGGL(k_eval_steps, dim3(std::min(16384, loops)), dim3(64 * waves), step_lds, nullptr, step_progs, loops, e, fit,
                        wrong, counts);
   }
@@ -4010,9 +4007,7 @@ void Session::eval_cases(const ProgramIn& program, std::vector<Val>& values, std
                        dv, de);
   } else {
     const std::size_t lds = std::size_t(kWavesPerBlock) * (slots + temps) * 64 * 10;
-    if (lds > 65536)
-      HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_eval_cases<false>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                 int(lds)));
+    allow_lds(reinterpret_cast<const void*>(&k_eval_cases<false>), lds);
     hipLaunchKernelGGL(k_eval_cases<false>, dim3(blocks), dim3(kEvalThreads), lds, nullptr, p, I.cases.cd, I.fuel, slots, temps, shadow,
                        dv, de);
   }
