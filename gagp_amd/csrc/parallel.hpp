@@ -3,7 +3,6 @@
 #include <algorithm>
 #include <cstddef>
 #include <exception>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -32,7 +31,7 @@ void parallel_ranges(std::size_t n, std::size_t grain, F f) {
   for (std::size_t k = 1; k < parts; ++k) {
     try {
       threads.emplace_back(run, k);
-    } catch (const std::system_error&) {
+    } catch (...) {  // no thread, or no memory for one; what is started has to be joined
       inline_from = k;
       break;
     }
