@@ -803,8 +803,8 @@ __host__ __device__ inline int loop_blocks(int C, int n, int group = 1) {
 // Four-wavefront blocks of one program held their slots until the longest of
 // its tiles ended, and every item paid two device-wide fences and thirteen
 // atomics. Measured together with the decoded steps, per launch: population
-// 8192 x 200 list cases 3.18 -> 0.65 ms, 64 mixed searches 5.59 -> 1.52 ms,
-// population 1500 x 130 cases of statement programs 0.85 -> 0.32 ms.
+// 8192 x 200 list cases 3.18 -> 0.68 ms, 64 mixed searches 5.56 -> 1.62 ms,
+// population 1500 x 130 cases of statement programs 0.85 -> 0.33 ms.
 template <bool kGrouped>
 __global__ __launch_bounds__(64) void k_eval_loop(DSearch* all, const BlockMap* map, int mode, int group_arg) {
   const int group = kGrouped ? group_arg : 1;

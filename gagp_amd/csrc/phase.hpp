@@ -427,7 +427,9 @@ constexpr int kWalkTest = 0x80, kWalkNext = 0x90;
 // its 5-instruction advance (LOAD counter, PUSH 1, ADD, STORE counter, JMP head).
 constexpr int kRangeTest = 0xA0, kRangeNext = 0xB0;
 // A LOAD or PUSH_CONST whose next instruction is a binary operation taking it
-// as its second operand, entered by no jump: the pair runs as one step.
+// as its second operand, entered by no jump. The decoder (steps.hpp) finds such
+// pairs by itself; the node-by-node lowering marks them all the same, and the
+// tests of it on the host hold it to that.
 constexpr int kFuse = 0xC0;
 GHD inline bool fusable_binary(int op) {
   return op == OP_ADD || op == OP_SUB || op == OP_MUL || op == OP_MOD || (op >= OP_LT && op <= OP_NE);

@@ -60,8 +60,8 @@ constexpr int kStepMax = kLoopCode;  // steps of a program: at most one per inst
 // a step leaves free; a WALK_TEST's three further slots and direction in w0
 // [21:6]. Kept beside the code at 16 bytes each, a search of 8192 list programs
 // asked for 164 MB instead of 144, and a server refused some it had admitted.
-// Reading them takes a second round trip, for the constants: k_eval_loop on
-// 4096 list programs x 200 cases 440 and 453 us.
+// Reading them takes a second round trip, for the constants: 13 of 450 us of
+// k_eval_loop on 4096 list programs x 200 cases.
 static_assert(sizeof(Ins) == sizeof(std::uint64_t) && kLoopPool <= 256, "a packed step replaces an instruction");
 STEP_FN std::uint64_t pack_step(const Step& s) {
   const unsigned c = unsigned(std::uint64_t(s.c));
@@ -80,10 +80,10 @@ STEP_FN Step unpack_step(std::uint64_t word) {
 STEP_FN bool step_indexes(const Step& s) { return (s.w0 & 63u) < unsigned(kStepControl) && (s.w0 >> 8 & 3u) == 2; }
 STEP_FN std::int64_t pool_payload(const Val& v) { return v.tag == TAG_BOOL ? std::int64_t(v.b != 0) : v.i; }
 
-// Slots of a lane: the evaluator inputs, the hidden locals, then the operand
-// stack's elements below the register top.
+// Slots of a lane: the evaluator inputs, the hidden locals, the operand stack's
+// elements below the register top, and a spare one for what a lane must not keep.
 constexpr int kStepStack = kLoopStack - 1;
-STEP_FN int step_slots(int n_inputs) { return n_inputs + kLoopLocals + kStepStack; }
+STEP_FN int step_slots(int n_inputs) { return n_inputs + kLoopLocals + kStepStack + 1; }
 
 // 256 flags, one per instruction.
 struct CodeBits {

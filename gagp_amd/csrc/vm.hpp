@@ -55,16 +55,6 @@ struct WaveStack {
   int shadow;
 };
 
-#if defined(__HIPCC__)
-__device__ inline int wave_min(int x) {
-  for (int off = 32; off > 0; off >>= 1) {
-    const int y = __shfl_xor(x, off, 64);
-    x = y < x ? y : x;
-  }
-  return x;
-}
-#endif
-
 // Smallest value of x over the wave for 0 <= x < 2^kBits, by a bitwise
 // search with ballots (scalar compares, no LDS round trips): bit b of the
 // minimum is 0 iff some lane lies in [m, m + 2^b - 1] for the bits m above it.
@@ -439,14 +429,6 @@ struct FastInputs {
   std::int64_t v0, v1, v2, v3;
   unsigned bound;
   __device__ std::int64_t pick(int k) const { return k == 0 ? v0 : k == 1 ? v1 : k == 2 ? v2 : v3; }
-  // A store into input k (uniform): later loads read it, and it is bound.
-  __device__ void set(int k, std::int64_t v) {
-    if (k == 0) v0 = v;
-    else if (k == 1) v1 = v;
-    else if (k == 2) v2 = v;
-    else v3 = v;
-    bound |= 1u << (k & 31);
-  }
 };
 __device__ inline FastInputs fast_inputs(const CaseData& cd, int n_inputs, int c, bool active) {
   FastInputs in{0, 0, 0, 0, 0};
@@ -593,12 +575,13 @@ __device__ inline LaneResult vm_fast(const FastProgram& f, const FastInputs& in,
 // balance by one scalar compare. A run ends where the group's lanes part, a
 // lane finishes, or the group reaches the step at which other lanes wait; only
 // there are the per-lane indexes and balances written and the next group
-// chosen. Every lane computes; what it keeps (the top, slots, a list element)
-// is selected by the group's mask. Under the mask as execution mask the steps
-// would be read from registers whose other lanes the compiler may drop in any
-// copy or spill it makes there; so it was, with none made by chance. The
-// selects cost k_eval_loop 3% on 4096 list programs x 200 cases (453 to 468 us)
-// and 7% on 1500 statement programs x 130 (475 to 511).
+// chosen. Every lane computes; the group's mask selects what it keeps (the top,
+// a list element) and where it stores (its slot, else a spare one). Under the
+// mask as execution mask the steps would be read from registers whose other
+// lanes the compiler may drop in any copy or spill it makes there, which only
+// chance kept it from. Stores under the mask cost k_eval_loop more branches: 468
+// and 436 us on 4096 list programs x 200 cases, 511 and 479 on 1500 statement
+// programs x 130.
 // Interpreting the bytecode itself, predicated and one instruction (or fixed
 // sequence) at a time, issued about 31 vector and 40 scalar instructions per
 // step and three times the steps; k_eval_loop has the measured times.
@@ -678,8 +661,8 @@ __device__ inline int wave_min_all(int x) {
 // `slots`: this wave's LDS area of step_slots(n_inputs) slots (slot k of lane
 // j at k * 64 + j). kGroups: register groups that hold the program's steps.
 // The run loop is one nest of two-way uniform branches with a single exit (no
-// switch, break or continue) and no divergent branch but a lane's stores: what a
-// lane records when it ends is written after the loop, from the event that ended it. In this
+// switch, break or continue) and no divergent branch: what a lane records when
+// it ends is written after the loop, from the event that ended it. In this
 // form the compiler keeps the step index, the fields, the balances and the
 // event in scalar registers and only the stack's top in vector ones; any
 // per-lane record merged inside the loop would be copied on every path of
@@ -693,6 +676,7 @@ __device__ inline LaneResult vm_steps(const StepProgram& f, const FastInputs& in
   LaneResult r{0, TAG_INVALID, 0, active ? ERR_NONE : ERR_VALUE, 0};
   LAS std::int64_t* const sl = slots + lane;
   for (int k = 0; k < n_inputs; ++k) sl[k * 64] = in.pick(k);
+  const int spare = step_slots(n_inputs) - 1;
   bool done = !active;
   std::int64_t top = 0;
   int ip = 0, fuel = fuel0;
@@ -728,9 +712,7 @@ __device__ inline LaneResult vm_steps(const StepProgram& f, const FastInputs& in
       continue;
     }
     const bool mine = !done && ip == at;
-    const auto store = [&](int slot, std::int64_t v) {
-      if (mine) sl[slot * 64] = v;
-    };
+    const auto store = [&](int slot, std::int64_t v) { sl[(mine ? slot : spare) * 64] = v; };
     int budget = low;
     if (low < kMost) {
       // Near exhaustion the group takes one step at a time. Lanes that cannot
