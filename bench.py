@@ -16,6 +16,8 @@ bytes, and the reference CPU engine's rate on the same search timed on this
 host's cores (one thread).
 """
 import argparse
+import glob
+import hashlib
 import json
 import os
 import re
@@ -87,16 +89,35 @@ PROFILED_NAME = {"k_vary": "k_vary<true, false>", "k_vary_global": "k_vary<false
                  "k_vary_deferred": "k_vary<true, true>", "k_vary_global_deferred": "k_vary<false, true>",
                  "k_lower": "k_lower<false>", "k_lower_walks": "k_lower<true>",
                  "k_eval": "k_eval<1>", "k_eval_general": "k_eval<0>", "k_place": "k_place<true>",
+                 "k_eval_loop": "k_eval_loop<false>",
                  "k_place_hbm": "k_place<false>"}
+
+
+def kernel_sources():
+    """Digest of the device sources' code, comments and spacing aside: what a
+    counter summary was measured on."""
+    digest = hashlib.sha256()
+    for path in sorted(glob.glob(os.path.join(ROOT, "gagp_amd", "csrc", "*.h*"))):
+        code = re.sub(r"//[^\n]*", "", open(path).read())
+        digest.update(os.path.basename(path).encode() + b"\0" + "".join(code.split()).encode())
+    return digest.hexdigest()[:16]
+
+
+def summary_lines(path):
+    """The lines of a committed counter summary, or none where it is absent or
+    was measured on other kernels than these (its counts divided by today's
+    launch times would be rates of nothing)."""
+    if not os.path.exists(path):
+        return []
+    lines = open(path).read().splitlines()
+    return lines if "Kernel sources: `%s`" % kernel_sources() in lines else []
 
 
 def measured_traffic(kernel):
     """HBM bytes per launch of `kernel` from the committed rocprofv3 FETCH_SIZE
     and WRITE_SIZE summary of this workload (None when absent)."""
-    if not os.path.exists(TRAFFIC):
-        return None
     name = PROFILED_NAME.get(kernel, kernel)
-    for line in open(TRAFFIC):
+    for line in summary_lines(TRAFFIC):
         m = re.match(r"\|\s*%s\s*\|\s*([0-9.]+)\s*\|" % re.escape(name), line)
         if m:
             return float(m.group(1))
@@ -110,11 +131,9 @@ def profiled_valu(kernel):
     """Per-launch VALU wave-instructions, lane utilization and LDS conflicts
     of `kernel` in the quintic section of the committed counter profile
     (None when absent)."""
-    if not os.path.exists(VALU_PROFILE):
-        return None
     name = PROFILED_NAME.get(kernel, kernel)
     section = None
-    for line in open(VALU_PROFILE):
+    for line in summary_lines(VALU_PROFILE):
         if line.startswith("## "):
             section = line
         if not section or "Quintic" not in section:
