@@ -13,10 +13,10 @@
 // What bounds it: the row-by-row form spent 57% of its cycles waiting for
 // about 78 global and 85 LDS loads a child, each a dependent round trip. Here
 // a child reads its tournament keys, its two rows at once, and its member
-// probe; what is left is the chain of the derivation and of the draws. A round
-// of 4096 children of the quintic grammar takes 59 us where it took 139, 1024
-// of a polynomial 39 for 78, 8192 of a list grammar 166 for 300, 1500 of a
-// statement grammar 105 for 183.
+// probe; what is left is the chain of the derivation and of the draws. With the
+// derivation over lane registers (derive_w), a round of 4096 children of the
+// quintic grammar takes 58 us where it took 154, 1024 of a polynomial 41 for 84,
+// 8192 of a list grammar 159 for 282, 1500 of a statement grammar 99 for 189.
 #pragma once
 #include "phase_wave.hpp"
 
