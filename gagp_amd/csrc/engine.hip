@@ -37,10 +37,15 @@
 
 namespace gagp_amd {
 
+// The runtime keeps a failed call's error until it is asked for: taken here, it
+// is not met again by the check after a later launch.
 #define HIP_OK(expr)                                                                                 \
   do {                                                                                               \
     const hipError_t e_ = (expr);                                                                    \
-    if (e_ != hipSuccess) throw std::runtime_error(std::string("HIP error: ") + hipGetErrorString(e_) + " at " #expr); \
+    if (e_ != hipSuccess) {                                                                          \
+      (void)hipGetLastError();                                                                       \
+      throw std::runtime_error(std::string("HIP error: ") + hipGetErrorString(e_) + " at " #expr);   \
+    }                                                                                                \
   } while (0)
 
 namespace {
