@@ -51,6 +51,7 @@ namespace gagp_amd {
 namespace {
 
 constexpr int kWavesPerBlock = 4;
+constexpr std::size_t kLdsLimit = 160 * 1024;  // of a block
 constexpr int kScoreCases = 4096;  // largest case count with an LDS score buffer per wavefront
 constexpr int kEvalThreads = 64 * kWavesPerBlock;
 
@@ -1669,18 +1670,19 @@ __device__ inline ProgView view_of(const DProg& p) {
 }
 // kFast: scores the programs certified for vm_fast (LDS: a score buffer of C
 // doubles per wavefront); otherwise the rest (LDS: the general stacks).
+// Scores a launch's typed straight-line (kFast) or general programs, one
+// wavefront each, as block `block` of `blocks`.
 template <bool kFast>
-__global__ __launch_bounds__(kEvalThreads) void k_eval_programs(const DProg* progs, int n, EvalParams e, int slots, int temps,
-                                                                 int shadow, double* fitness, unsigned* wrong, unsigned* counts) {
-  extern __shared__ unsigned char smem[];
-  __shared__ double replay[kFast ? kWavesPerBlock : 1][kFast ? kReplayWords : 1];
+__device__ __attribute__((always_inline)) inline void score_programs(int block, int blocks, const DProg* progs, int n, const EvalParams& e,
+                                                                     int slots, int temps, int shadow, unsigned char* smem, double* replay,
+                                                                     double* fitness, unsigned* wrong, unsigned* counts) {
   const int wave = wave_index(), lane = threadIdx.x % 64;
   WaveStack st = stack_of(smem, kFast ? 0 : slots, kFast ? 0 : temps, wave, kFast ? 0 : shadow);
   double* scores = kFast ? reinterpret_cast<double*>(smem) + std::size_t(wave) * e.cd.C : nullptr;
-  for (int i = blockIdx.x * kWavesPerBlock + wave; i < n; i += gridDim.x * kWavesPerBlock) {
+  for (int i = block * kWavesPerBlock + wave; i < n; i += blocks * kWavesPerBlock) {
     const DProg p = progs[i];
-    if (p.fast != int(kFast)) continue;  // 2: k_eval_steps scores it
-    const EvalOut r = eval_program<kFast ? 1 : 0>(e, view_of(p), st, scores, lane, replay[kFast ? wave : 0]);
+    if (p.fast != int(kFast)) continue;  // 2: score_steps has it
+    const EvalOut r = eval_program<kFast ? 1 : 0>(e, view_of(p), st, scores, lane, replay);
     if (lane == 0) {
       fitness[i] = r.fitness;
       wrong[i] = e.policy.metric == METRIC_LEGACY ? 0 : r.wrong;
@@ -1690,6 +1692,14 @@ __global__ __launch_bounds__(kEvalThreads) void k_eval_programs(const DProg* pro
     }
   }
 }
+template <bool kFast>
+__global__ __launch_bounds__(kEvalThreads) void k_eval_programs(const DProg* progs, int n, EvalParams e, int slots, int temps,
+                                                                 int shadow, double* fitness, unsigned* wrong, unsigned* counts) {
+  extern __shared__ unsigned char smem[];
+  __shared__ double replay[kFast ? kWavesPerBlock : 1][kFast ? kReplayWords : 1];
+  score_programs<kFast>(int(blockIdx.x), int(gridDim.x), progs, n, e, slots, temps, shadow, smem, replay[kFast ? wave_index() : 0],
+                        fitness, wrong, counts);
+}
 // A caller's looping programs on the decoded steps (certify_loop): one block
 // per program, whose wavefronts take its 64-case tiles in turn in the visiting
 // order (longest lists first). Totals are combined in LDS as in k_eval_tiles.
@@ -1698,16 +1708,18 @@ __global__ __launch_bounds__(kEvalThreads) void k_eval_programs(const DProg* pro
 // 6.17 ms on the general VM (tagged values, a few cases' branches predicated
 // per instruction) and take 0.45 ms here.
 struct StepProg { GAS const Step* steps; int n_steps, index, result_tag; };
-__global__ __launch_bounds__(kEvalThreads) void k_eval_steps(const StepProg* progs, int n, EvalParams e, double* fitness,
-                                                              unsigned* wrong, unsigned* counts) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  __shared__ double part_sum[kWavesPerBlock], replay[kReplayWords];
-  __shared__ unsigned part_count[kWavesPerBlock][4];  // wrong, errors, timeouts, integral
+struct StepTotals {
+  double sum[kWavesPerBlock], replay[kReplayWords];
+  unsigned count[kWavesPerBlock][4];  // wrong, errors, timeouts, integral
+};
+__device__ __attribute__((always_inline)) inline void score_steps(int block, int blocks, const StepProg* progs, int n, const EvalParams& e,
+                                                                  unsigned char* smem, StepTotals& part, double* fitness,
+                                                                  unsigned* wrong, unsigned* counts) {
   const int waves = int(blockDim.x) / 64, wave = wave_index(), lane = threadIdx.x % 64;
   const int C = e.cd.C, n_in = e.cd.n_inputs, slots = step_slots(n_in);
   LAS std::int64_t* const sl = (LAS std::int64_t*)smem + std::size_t(wave) * slots * 64;
   double* const scores = reinterpret_cast<double*>(smem + std::size_t(waves) * slots * 64 * 8);
-  for (int i = blockIdx.x; i < n; i += gridDim.x) {  // one program per block, uniform
+  for (int i = block; i < n; i += blocks) {  // one program per block, uniform
     const StepProg p = progs[i];
     const StepProgram sp = steps_load(p.steps, p.n_steps, lane);
     double isum = 0;
@@ -1734,11 +1746,11 @@ __global__ __launch_bounds__(kEvalThreads) void k_eval_steps(const StepProg* pro
     const unsigned ww = wave_sum_u(w), we = wave_sum_u(errs), wt = wave_sum_u(touts);
     const bool wint = __ballot(!integral) == 0;
     if (lane == 0) {
-      part_sum[wave] = ws;
-      part_count[wave][0] = ww;
-      part_count[wave][1] = we;
-      part_count[wave][2] = wt;
-      part_count[wave][3] = wint;
+      part.sum[wave] = ws;
+      part.count[wave][0] = ww;
+      part.count[wave][1] = we;
+      part.count[wave][2] = wt;
+      part.count[wave][3] = wint;
     }
     __syncthreads();  // every wavefront's scores and totals
     if (wave == 0) {
@@ -1746,13 +1758,13 @@ __global__ __launch_bounds__(kEvalThreads) void k_eval_steps(const StepProg* pro
       unsigned tw = 0, te = 0, tt = 0;
       bool all_integral = true;
       for (int k = 0; k < waves; ++k) {
-        total += part_sum[k];
-        tw += part_count[k][0];
-        te += part_count[k][1];
-        tt += part_count[k][2];
-        all_integral = all_integral && part_count[k][3] != 0;
+        total += part.sum[k];
+        tw += part.count[k][0];
+        te += part.count[k][1];
+        tt += part.count[k][2];
+        all_integral = all_integral && part.count[k][3] != 0;
       }
-      const double f = all_integral ? total : canonical_from_scores(e, C, scores, lane, replay);
+      const double f = all_integral ? total : canonical_from_scores(e, C, scores, lane, part.replay);
       if (lane == 0) {
         fitness[p.index] = f;
         wrong[p.index] = e.policy.metric == METRIC_LEGACY ? 0 : tw;
@@ -1763,6 +1775,26 @@ __global__ __launch_bounds__(kEvalThreads) void k_eval_steps(const StepProg* pro
     }
     __syncthreads();  // before the next program reuses the scores
   }
+}
+__global__ __launch_bounds__(kEvalThreads) void k_eval_steps(const StepProg* progs, int n, EvalParams e, double* fitness,
+                                                              unsigned* wrong, unsigned* counts) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  __shared__ StepTotals part;
+  score_steps(int(blockIdx.x), int(gridDim.x), progs, n, e, smem, part, fitness, wrong, counts);
+}
+// A launch with both kinds of looping program: the first `general` blocks score
+// the general VM's, each a chain of its own, and the others run the rest beside
+// them. 511 programs on the steps and one whose stack is past the path took
+// 6.41 ms one after the other and take 5.92 so; all of them on the general VM
+// had taken 6.29.
+__global__ __launch_bounds__(kEvalThreads) void k_eval_both(const DProg* progs, int n, int general, const StepProg* step_progs, int loops,
+                                                             EvalParams e, int slots, int temps, int shadow, double* fitness,
+                                                             unsigned* wrong, unsigned* counts) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  __shared__ StepTotals part;
+  const int block = int(blockIdx.x);
+  if (block < general) score_programs<false>(block, general, progs, n, e, slots, temps, shadow, smem, nullptr, fitness, wrong, counts);
+  else score_steps(block - general, int(gridDim.x) - general, step_progs, loops, e, smem, part, fitness, wrong, counts);
 }
 template <bool kFast>
 __global__ __launch_bounds__(kEvalThreads) void k_eval_cases(DProg p, CaseData cd, int fuel, int slots, int temps, int shadow,
@@ -2349,7 +2381,7 @@ struct Batch::Impl {
 
   // Allocates one search and fixes its kernel variants and LDS needs.
   void configure(SearchState& s) {
-    constexpr std::size_t kLdsLimit = 160 * 1024, kStageLimit = 64 * 1024;
+    constexpr std::size_t kStageLimit = 64 * 1024;
     s.configured = true;
     s.allocate();
     s.d.profile = timer.on ? 1 : 0;
@@ -3836,23 +3868,34 @@ void Session::Impl::launch(const PackedPrograms& k, const DProg* progs, const St
   const EvalParams e{I.cases.cd, I.fuel, I.lanes, I.penalty, I.policy};
   const std::size_t lds = std::size_t(kWavesPerBlock) * (k.slots + k.temps) * 64 * 10;
   const std::size_t fast_lds = std::size_t(kWavesPerBlock) * 8 * std::size_t(I.cases.cd.C);
-  if (k.any_general) allow_lds(reinterpret_cast<const void*>(&k_eval_programs<false>), lds);
-  if (k.any_fast) allow_lds(reinterpret_cast<const void*>(&k_eval_programs<true>), fast_lds);
-  const int blocks = std::min(4096, (n + kWavesPerBlock - 1) / kWavesPerBlock);
-  if (const int loops = int(k.step_n.size())) {
-    const int waves = std::min(kWavesPerBlock, (I.cases.cd.C + 63) / 64);
-    const std::size_t step_lds =
-        std::size_t(waves) * step_slots(I.cases.cd.n_inputs) * 64 * 8 + 8 * std::size_t(I.cases.cd.C);
-    allow_lds(reinterpret_cast<const void*>(&k_eval_steps), step_lds);
-    hipLaunchKernelGGL(k_eval_steps, dim3(std::min(16384, loops)), dim3(64 * waves), step_lds, nullptr, step_progs, loops, e, fit,
+  const int blocks = std::min(4096, (n + kWavesPerBlock - 1) / kWavesPerBlock), loops = int(k.step_n.size());
+  const auto step_lds = [&](int waves) {
+    return std::size_t(waves) * step_slots(I.cases.cd.n_inputs) * 64 * 8 + 8 * std::size_t(I.cases.cd.C);
+  };
+  const int step_blocks = std::min(16384, loops), step_waves = std::min(kWavesPerBlock, (I.cases.cd.C + 63) / 64);
+  // Both kinds of looping program go in one launch of whole blocks where the
+  // general VM's deepest stack leaves LDS for the steps' totals.
+  const std::size_t both_lds = std::max(lds, step_lds(kWavesPerBlock));
+  const bool both = loops && k.any_general && both_lds + sizeof(StepTotals) <= kLdsLimit;
+  if (both) {
+    allow_lds(reinterpret_cast<const void*>(&k_eval_both), both_lds);
+    hipLaunchKernelGGL(k_eval_both, dim3(blocks + step_blocks), dim3(kEvalThreads), both_lds, nullptr, progs, n, blocks, step_progs, loops, e,
+                       k.slots, k.temps, k.shadow, fit, wrong, counts);
+  } else if (loops) {
+    allow_lds(reinterpret_cast<const void*>(&k_eval_steps), step_lds(step_waves));
+    hipLaunchKernelGGL(k_eval_steps, dim3(step_blocks), dim3(64 * step_waves), step_lds(step_waves), nullptr, step_progs, loops, e, fit,
                        wrong, counts);
   }
-  if (k.any_fast)
+  if (k.any_fast) {
+    allow_lds(reinterpret_cast<const void*>(&k_eval_programs<true>), fast_lds);
     hipLaunchKernelGGL(k_eval_programs<true>, dim3(blocks), dim3(kEvalThreads), fast_lds, nullptr, progs, n, e, k.slots, k.temps,
                        k.shadow, fit, wrong, counts);
-  if (k.any_general)
+  }
+  if (k.any_general && !both) {
+    allow_lds(reinterpret_cast<const void*>(&k_eval_programs<false>), lds);
     hipLaunchKernelGGL(k_eval_programs<false>, dim3(blocks), dim3(kEvalThreads), lds, nullptr, progs, n, e, k.slots, k.temps,
                        k.shadow, fit, wrong, counts);
+  }
   HIP_OK(hipGetLastError());
 }
 
